@@ -15,12 +15,13 @@
 //     the state leaving the chunk, in registers (one workgroup per (sequence, value head,
 //     64 columns of dv), 16 columns per wavefront):
 //         dV_new = P^T dO + diag(e^{G_last - G}) K dS
-//         dS    <- e^{G_last} dS + scale Q^T diag(e^G) dO - K^T diag(e^G) diag(beta) X^T dV_new
-//     and stores dS per chunk and dV_new.
+//         dR     = X^T dV_new
+//         dS    <- e^{G_last} dS + scale Q^T diag(e^G) dO - K^T diag(e^G) diag(beta) dR
+//     and stores dS per chunk and dR.
 //  2. cgrad_kernel forms, for every (chunk, value head) at once, the chunk-local
-//     gradients of q, k (per value head), v, g and beta from S, dS, V_new, dV_new and
-//     the chunk's matrices, differentiating :100-142 step by step (the derivation is the
-//     one of the fp64 test oracle, oracle/gdn_vjp.py).
+//     gradients of q, k (per value head), v, g and beta from S, dS, V_new, dR and the
+//     chunk's matrices (the test oracle, oracle/gdn_vjp.py, differentiates :100-142 step
+//     by step; the products by X it takes drop out, see there).
 //  3. qk_final_kernel sums the per-value-head q/k gradients over each key head's value
 //     heads (the adjoint of the repeat-interleave, :272-280) and applies the L2-norm
 //     backward (:30-32), writing dq, dk at the input precision.
@@ -99,8 +100,7 @@ __device__ __forceinline__ void frag_col(const T* m, int ld, int col, int k0, fl
 
 // K / Q operand fragments from the staged rows: bf16 rows are exact bf16 (one vector or
 // two transposed LDS reads, no lo part); fp32 rows are read element-wise and split.
-// kq_row: row row0 + lane%16, slots over columns from k0; kq_col: column col0 + lane%16,
-// slots over rows from k0.
+// kq_row: row row0 + lane%16, slots over columns from k0.
 template <bool PAIR>
 __device__ __forceinline__ Op kq_row(const float* m, int ld, int row0, int k0) {
   float x[8];
@@ -121,51 +121,23 @@ __device__ __forceinline__ Op kq_row(const bf16_t* m, int ld, int row0, int k0) 
   o.l = o.h;
   return o;
 }
-template <bool PAIR>
-__device__ __forceinline__ Op kq_col(const float* m, int ld, int col0, int k0) {
+// kq_st: column (row lane%16 of state tile t in the scans' order), slots over rows from k0
+// in the block-pair order.
+__device__ __forceinline__ Op kq_st(const float* m, int ld, int t, int k0) {
+  const int r = lane_id() & 15;
   float x[8];
-  frag_col<PAIR>(m, ld, col0 + (lane_id() & 15), k0, x);
+  frag_col<true>(m, ld, 32 * (t >> 1) + 4 * (t & 1) + 8 * (r >> 2) + (r & 3), k0, x);
   return split8(x);
 }
-template <bool PAIR>
-__device__ __forceinline__ Op kq_col(const bf16_t* m, int ld, int col0, int k0) {
+__device__ __forceinline__ Op kq_st(const bf16_t* m, int ld, int t, int k0) {
+  const int l = lane_id(), q = l >> 4, s = l & 15;
+  // source lane s of a 16-lane group points at row s / 4 and the 4 columns of row group s % 4
+  const bf16_t* pr = m + (k0 + 4 * q + (s >> 2)) * ld + 32 * (t >> 1) + 4 * (t & 1) + 8 * (s & 3);
+  const u32x2 a = ds_read_tr(pr), b = ds_read_tr(pr + 16 * ld);
   Op o;
-  if constexpr (PAIR) {
-    const u32x2 a = rows4_tr(m, ld, k0, col0), b = rows4_tr(m, ld, k0 + 16, col0);
-    o.h = u32x4{a[0], a[1], b[0], b[1]};
-  } else {
-    o.h = frag_tr(m, ld, k0, col0);
-  }
+  o.h = u32x4{a[0], a[1], b[0], b[1]};
   o.l = o.h;
   return o;
-}
-
-// global: 8 consecutive values of row `row` from column k0 + 8q (zero when row >= nvalid)
-template <class T>
-__device__ __forceinline__ void gfrag_row(const T* base, long long ld, int row, int nvalid, int k0,
-                                          float* x) {
-  const int q = lane_id() >> 4;
-  if (row < nvalid) {
-    const T* pr = base + (long long)row * ld + k0 + 8 * q;
-    if constexpr (std::is_same<T, float>::value) {
-      const float4 a = ((const float4*)pr)[0], b = ((const float4*)pr)[1];
-      x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
-      x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-    } else {
-      const u32x4 w = *(const u32x4*)pr;
-      unpack8<false>(&w, x);
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = 0.f;
-  }
-}
-// global: column `col`, rows k0 + 8q + e of a row-major fp32 array (stride ld)
-__device__ __forceinline__ void gfrag_col(const float* base, long long ld, int col, int k0,
-                                          float* x) {
-  const int q = lane_id() >> 4;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = base[(long long)(k0 + 8 * q + e) * ld + col];
 }
 
 // Loads whose rows may lie past a sequence's end go through a buffer resource whose range
@@ -173,23 +145,14 @@ __device__ __forceinline__ void gfrag_col(const float* base, long long ld, int c
 // a branch, which would leave the count of outstanding memory operations unknown and turn
 // every later wait for one of them into a wait for all (the previous chunk's stores too).
 // Byte offsets are 32-bit.
-__device__ __forceinline__ float4 bload4(__amdgpu_buffer_rsrc_t r, unsigned off, const float*) {
-  const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+__device__ __forceinline__ float4 bload4(__amdgpu_buffer_rsrc_t r, unsigned off, const float*, int soff = 0) {
+  const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0);
   return float4{__uint_as_float(w[0]), __uint_as_float(w[1]), __uint_as_float(w[2]),
                 __uint_as_float(w[3])};
 }
-__device__ __forceinline__ u32x2 bload4(__amdgpu_buffer_rsrc_t r, unsigned off, const bf16_t*) {
-  return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+__device__ __forceinline__ u32x2 bload4(__amdgpu_buffer_rsrc_t r, unsigned off, const bf16_t*, int soff = 0) {
+  return __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0);
 }
-// gfrag_col over a buffer resource of fp32 rows (zeros past its range)
-__device__ __forceinline__ void gfrag_col_b(__amdgpu_buffer_rsrc_t r, unsigned ld, unsigned col,
-                                            unsigned k0, float* x) {
-  const unsigned q = (unsigned)lane_id() >> 4;
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    x[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, 4u * ((k0 + 8u * q + e) * ld + col), 0, 0));
-}
-
 // 4 elements in registers (4 bf16 in two words, or 4 floats)
 template <class T> struct Vec4;
 template <> struct Vec4<float> { typedef float4 type; };
@@ -217,12 +180,28 @@ __device__ __forceinline__ void load8v(const float* p, float* x) {
   x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
 }
 
+// N consecutive values of one row at a buffer offset (bytes), at the precision T
+template <class T, int N>
+__device__ __forceinline__ void store_row(__amdgpu_buffer_rsrc_t r, unsigned off, const float* x) {
+  if constexpr (std::is_same<T, float>::value) {
+#pragma unroll
+    for (int e = 0; e < N; e += 4)
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(x[e]), __float_as_uint(x[e + 1]),
+                                                   __float_as_uint(x[e + 2]), __float_as_uint(x[e + 3])},
+                                             r, off + 4u * e, 0, 0);
+  } else if constexpr (N == 8) {
+    __builtin_amdgcn_raw_buffer_store_b128(pack8(x), r, off, 0, 0);
+  } else {
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3])}, r, off, 0, 0);
+  }
+}
+
 // Row sums of a C-layout tile (lane (q, r) holds rows 16 bi + 4q + v, v = 0..3, of
-// column r) added into arr[row], without LDS traffic: a reduce-scatter over the 16 lanes of
+// column r) into arr[row], without LDS traffic: a reduce-scatter over the 16 lanes of
 // each row group with DPP moves.  Lanes r and r ^ 8 split the four rows between them
 // (row_ror:8), lanes r and its mirror in the 8-lane half split the pair (row_half_mirror),
 // then each quad sums (quad_perm); lane r with r % 4 == 0 ends with row 16 bi + 4q + r / 4.
-__device__ __forceinline__ void add_rows(float* arr, int bi, f32x4 x) {
+__device__ __forceinline__ void set_rows(float* arr, int bi, f32x4 x) {
   const int l = lane_id(), r = l & 15;
   const bool up8 = (r & 8) != 0, up4 = (r & 4) != 0;
   const float k0 = up8 ? x[2] : x[0], k1 = up8 ? x[3] : x[1];
@@ -232,19 +211,19 @@ __device__ __forceinline__ void add_rows(float* arr, int bi, f32x4 x) {
   float s = kb + dpp_f<0x141>(gb);
   s += dpp_f<0x4E>(s);
   s += dpp_f<0xB1>(s);
-  if ((r & 3) == 0) arr[16 * bi + 4 * (l >> 4) + (r >> 2)] += s;
+  if ((r & 3) == 0) arr[16 * bi + 4 * (l >> 4) + (r >> 2)] = s;
 }
-// Column sums of a C-layout tile (column 16 bj + r, summed over its 16 rows) added into
+// Column sums of a C-layout tile (column 16 bj + r, summed over its 16 rows) into
 // arr[col]: the lane's four rows, then across the four row groups with the 16- and 32-lane
 // swaps (lanes of row group 0 write).
-__device__ __forceinline__ void add_cols(float* arr, int bj, f32x4 x) {
+__device__ __forceinline__ void set_cols(float* arr, int bj, f32x4 x) {
   const int l = lane_id();
   float s = x[0] + x[1] + x[2] + x[3];
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false);
   s = __uint_as_float(a[0]) + __uint_as_float(a[1]);
   const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false);
   s = __uint_as_float(b[0]) + __uint_as_float(b[1]);
-  if ((l >> 4) == 0) arr[16 * bj + (l & 15)] += s;
+  if ((l >> 4) == 0) arr[16 * bj + (l & 15)] = s;
 }
 
 // Sum over the 64 lanes, left in every lane (DPP within each row, then the row swaps).
@@ -389,15 +368,21 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
   const size_t rec_stride = (size_t)rec_bytes(rec_mode(F32), true);
   const long long rs = (long long)p.Hv * DV;  // row stride of dO / dV_new
 
-  // dS[t][v] = dS[16t + 4lq + v][col0 + c + lr]: gradient of the state leaving the chunk
+  // dS[t][v] = dS[st_row(t, v)][col0 + c + lr]: gradient of the state leaving the chunk, its
+  // rows in the forward scan's order (two tiles side by side are the B operand over 32
+  // consecutive dk, so K's operands are plain rows); dsb: its split operands
+  auto st_row = [&](int t, int v) { return 32 * (t >> 1) + 8 * lq + 4 * (t & 1) + v; };
   f32x4 dS[DK / 16];
+  Op dsb[DK / 32];
   const size_t st_off = ((size_t)n * p.Hv + h) * DK * DV + col0 + c + lr;
   auto init_dS = [&]() {
 #pragma unroll
     for (int t = 0; t < DK / 16; ++t)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        dS[t][v] = p.dht ? p.dht[st_off + (size_t)(16 * t + 4 * lq + v) * DV] : 0.f;
+        dS[t][v] = p.dht ? p.dht[st_off + (size_t)st_row(t, v) * DV] : 0.f;
+#pragma unroll
+    for (int s = 0; s < DK / 32; ++s) dsb[s] = join_op(dS[2 * s], dS[2 * s + 1]);
   };
   // gradient of the initial state
   auto write_dh0 = [&]() {
@@ -405,7 +390,7 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
 #pragma unroll
       for (int t = 0; t < DK / 16; ++t)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) p.dh0[st_off + (size_t)(16 * t + 4 * lq + v) * DV] = dS[t][v];
+        for (int v = 0; v < 4; ++v) p.dh0[st_off + (size_t)st_row(t, v) * DV] = dS[t][v];
     }
   };
 
@@ -516,6 +501,24 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
       sPT[t][l] = u32x4{hi[0], hi[1], lo[0], lo[1]};
     }
   };
+  // dR^T of the last computed chunk (tokens dr_t0 .. + dr_n - 1): a lane holds 4 consecutive
+  // columns of one token row, one 16-byte store per row block.  It is stored a step later,
+  // between the products of the next chunk: stored at once, it met the next chunk's dS stores
+  // and the loaders' loads (rscan 334 us; so 320 us; C1).  Rows past the chunk's end lie
+  // outside the buffer range and are dropped: no branch.
+  f32x4 dr[4];
+  long long dr_t0 = 0;
+  int dr_n = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) dr[i] = zero4();
+  auto put_dr = [&]() {
+    const auto vd = buf_rsrc(p.drows + dr_t0 * rs + (long long)h * DV + col0, 4u * (unsigned)dr_n * (unsigned)rs);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_buffer_store_b128(
+          u32x4{__float_as_uint(dr[i][0]), __float_as_uint(dr[i][1]), __float_as_uint(dr[i][2]), __float_as_uint(dr[i][3])},
+          vd, 4u * ((unsigned)(16 * i + lr) * (unsigned)rs + (unsigned)(c + 4 * lq)), 0, 0);
+  };
   // chunk j on the compute wavefronts, from the rows staged in bf
   auto compute = [&](const int j, const Buf& bf) {
     const long long t0 = s0 + (long long)j * C;
@@ -533,27 +536,36 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
     const float* sEL = sGate + kGateEL * C;  // e^{G_last - G}; e^{G_last} in the last slot
     const float* sB = sGate + kGateBeta * C;
 
-    // gradient of the state leaving chunk j, for the chunk-local gradients
-    {
-      // column-major per state ([dv][dk]): a lane's 4 rows of a tile are contiguous
-      float* dd = p.dstates + ((size_t)slot * p.Hv + h) * DK * DV + (size_t)(col0 + c + lr) * DK;
+    // dO of the wavefront's 16 columns over each half of the chunk, in the block-pair order
+    // of every product it enters, and scale e^G dO for the state's Q^T term: neither waits
+    // for dS, so both are formed beside K dS
+    Op dob[2], b1[2];
 #pragma unroll
-      for (int t = 0; t < DK / 16; ++t) *(f32x4*)(dd + 16 * t + 4 * lq) = dS[t];
-    }
-
+    for (int p2 = 0; p2 < 2; ++p2) dob[p2] = op_tr_pair(sDOh, sDOl, LDB, c, 32 * p2);
     // ---------------------------------------------------------------- K dS
-    Op dsb[DK / 32];
-#pragma unroll
-    for (int s = 0; s < DK / 32; ++s) dsb[s] = join_op(dS[2 * s], dS[2 * s + 1]);
     f32x4 kds[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f32x4 acc = zero4();
+    for (int i = 0; i < 4; ++i) kds[i] = zero4();
 #pragma unroll
-      for (int s = 0; s < DK / 32; ++s) {
-        acc = mm3<F32, true>(acc, kq_row<true>(sK, LDK, 16 * i, 32 * s), dsb[s]);
-      }
-      kds[i] = acc;
+    for (int s = 0; s < DK / 32; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) kds[i] = mm3<F32, true>(kds[i], kq_row<false>(sK, LDK, 16 * i, 32 * s), dsb[s]);
+#pragma unroll
+    for (int p2 = 0; p2 < 2; ++p2) {
+      float x[8];
+      op_values(dob[p2], x);
+      const float4 ga = *(const float4*)(sEGS + 32 * p2 + 4 * lq), gb = *(const float4*)(sEGS + 32 * p2 + 16 + 4 * lq);
+      const float g[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] *= g[e];
+      b1[p2] = split8(x);
+    }
+    // gradient of the state leaving chunk j, for the chunk-local gradients: column-major per
+    // state ([dv][dk]), a lane's 8 rows of a tile pair are contiguous
+    {
+      float* dd = p.dstates + ((size_t)slot * p.Hv + h) * DK * DV + (size_t)(col0 + c + lr) * DK;
+#pragma unroll
+      for (int t = 0; t < DK / 16; ++t) *(f32x4*)(dd + st_row(t, 0)) = dS[t];
     }
     // (LDR) the loaders' P tiles of this chunk are in sPT after this barrier
     if constexpr (LDR) lds_barrier();
@@ -564,84 +576,72 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
       f32x4 acc = zero4();
 #pragma unroll
       for (int p2 = i / 2; p2 < 2; ++p2) {  // P^T is upper triangular
+        Op pt;
         if constexpr (PREC) {
           // P^T rows 16i .. +15 over tokens 32 p2 .. +31 from the P tiles (2 p2, i) and
-          // (2 p2 + 1, i) side by side (block-pair order; (2 p2, i) is above the diagonal,
-          // zero, when 2 p2 < i), against dO read in the same order
+          // (2 p2 + 1, i) side by side ((2 p2, i) is above the diagonal, zero, when
+          // 2 p2 < i)
           const u32x4 tb = sPT[ptile_index(2 * p2 + 1, i)][l];
           const u32x4 ta = 2 * p2 >= i ? sPT[ptile_index(2 * p2, i)][l] : u32x4{0u, 0u, 0u, 0u};
-          Op pt;
           pt.h = u32x4{ta[0], ta[1], tb[0], tb[1]};
           pt.l = u32x4{ta[2], ta[3], tb[2], tb[3]};
-          acc = mm3<true, true>(acc, pt, op_tr_pair(sDOh, sDOl, LDB, c, 32 * p2));
         } else {
-          acc = mm3<true, true>(acc, op_tr(sPh, sPl, LDB, 16 * i, 32 * p2),
-                                op_tr(sDOh, sDOl, LDB, c, 32 * p2));
+          pt = op_tr_pair(sPh, sPl, LDB, 16 * i, 32 * p2);
         }
+        acc = mm3<true, true>(acc, pt, dob[p2]);
       }
+      const float4 el4 = *(const float4*)(sEL + 16 * i + 4 * lq);
+      const float el[4] = {el4.x, el4.y, el4.z, i == 3 && lq == 3 ? 1.f : el4.w};  // row C - 1: e^0
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * i + 4 * lq + v;
-        const float el = row == C - 1 ? 1.f : sEL[row];
-        dvn[i][v] = acc[v] + el * kds[i][v];
-      }
+      for (int v = 0; v < 4; ++v) dvn[i][v] = acc[v] + el[v] * kds[i][v];
     }
-    {
-      // rows at or past nvalid lie outside the buffer range and are dropped: no branch
-      const auto vd = buf_rsrc(p.dvnew + t0 * rs + (long long)h * DV + col0,
-                               4u * (unsigned)nvalid * (unsigned)rs);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          __builtin_amdgcn_raw_buffer_store_b32(
-              __float_as_uint(dvn[i][v]), vd,
-              4u * ((unsigned)(16 * i + 4 * lq + v) * (unsigned)rs + (unsigned)(c + lr)), 0, 0);
-    }
-    // ---------------------------------------------------------------- Y = diag(beta) X^T dV_new
+    __builtin_amdgcn_sched_barrier(0);
+    put_dr();
+    __builtin_amdgcn_sched_barrier(0);
     Op dvp[2];
 #pragma unroll
     for (int pp = 0; pp < 2; ++pp) dvp[pp] = join_op(dvn[2 * pp], dvn[2 * pp + 1]);
+    // ------------------------------------------------ dS <- e^{G_last} dS + scale Q^T diag(e^G) dO
+    // (its products fill the matrix cores while the chain's vector work, dV_new and Y, runs)
+    const float egl = sEL[C - 1];
+#pragma unroll
+    for (int t = 0; t < DK / 16; ++t) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) dS[t][v] *= egl;
+#pragma unroll
+      for (int p2 = 0; p2 < 2; ++p2) dS[t] = mm3<F32, true>(dS[t], kq_st(sQ, LDK, t, 32 * p2), b1[p2]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // ---------------------------------------------------------------- dR = X^T dV_new, Y = diag(beta) dR
+    // dR is also formed transposed (dR^T = dV_new^T X, the same operands exchanged), for its
+    // stores (put_dr)
     f32x4 y[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       f32x4 acc = zero4();
+      dr[i] = zero4();
 #pragma unroll
-      for (int p2 = i / 2; p2 < 2; ++p2)  // X^T is upper triangular; X^T rows (stored transposed)
-        acc = mm3<true, true>(acc, op_pair(sXh, sXl, LDB, 16 * i, 32 * p2), dvp[p2]);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) y[i][v] = sB[16 * i + 4 * lq + v] * acc[v];
-    }
-    // ---------------------------------------------------------------- dS update
-    Op b1[2], b2[2];
-#pragma unroll
-    for (int p2 = 0; p2 < 2; ++p2) {
-      float x[8];
-      op_values(op_tr(sDOh, sDOl, LDB, c, 32 * p2), x);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] *= sEGS[32 * p2 + 8 * lq + e];
-      b1[p2] = split8(x);
-      f32x4 ya, yb;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        ya[v] = -sEG[32 * p2 + 4 * lq + v] * y[2 * p2][v];
-        yb[v] = -sEG[32 * p2 + 16 + 4 * lq + v] * y[2 * p2 + 1][v];
+      for (int p2 = i / 2; p2 < 2; ++p2) {  // X^T is upper triangular; X^T rows (stored transposed)
+        const Op x = op_pair(sXh, sXl, LDB, 16 * i, 32 * p2);
+        acc = mm3<true, true>(acc, x, dvp[p2]);
+        dr[i] = mm3<true, true>(dr[i], dvp[p2], x);
       }
-      b2[p2] = join_op(ya, yb);
+      const float4 b4 = *(const float4*)(sB + 16 * i + 4 * lq), e4 = *(const float4*)(sEG + 16 * i + 4 * lq);
+      y[i] = f32x4{-e4.x * (b4.x * acc[0]), -e4.y * (b4.y * acc[1]), -e4.z * (b4.z * acc[2]), -e4.w * (b4.w * acc[3])};
     }
-    const float egl = sEL[C - 1];
+    __builtin_amdgcn_sched_barrier(0);
+    // ---------------------------------------------------------------- dS <- dS - K^T diag(e^G) Y
+    Op b2[2];
 #pragma unroll
-    for (int t = 0; t < DK / 16; ++t) {
-      f32x4 acc;
+    for (int p2 = 0; p2 < 2; ++p2) b2[p2] = join_op(y[2 * p2], y[2 * p2 + 1]);
+    dr_t0 = t0;
+    dr_n = nvalid;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) acc[v] = egl * dS[t][v];
+    for (int t = 0; t < DK / 16; ++t)
 #pragma unroll
-      for (int p2 = 0; p2 < 2; ++p2) {
-        acc = mm3<F32, true>(acc, kq_col<false>(sQ, LDK, 16 * t, 32 * p2), b1[p2]);
-        acc = mm3<F32, true>(acc, kq_col<true>(sK, LDK, 16 * t, 32 * p2), b2[p2]);
-      }
-      dS[t] = acc;
-    }
+      for (int p2 = 0; p2 < 2; ++p2) dS[t] = mm3<F32, true>(dS[t], kq_st(sK, LDK, t, 32 * p2), b2[p2]);
+#pragma unroll
+    for (int s = 0; s < DK / 32; ++s) dsb[s] = join_op(dS[2 * s], dS[2 * s + 1]);
   };
   // Barriers here order LDS accesses only (lds_barrier): the global stores go to later
   // kernels and the staged rows come from per-thread registers, so neither the loads nor
@@ -687,6 +687,7 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
         cstep(j - 1, B1);
       }
       if (j == 0) cstep(0, B0);
+      put_dr();
       write_dh0();
     }
   } else {
@@ -716,51 +717,75 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
       step(j - 1, pfb, j - 3);
     }
     if (j == 0) step(0, pfa, -2);
+    put_dr();
     write_dh0();
   }
 }
 
 // ============================================================================ chunk-local gradients
 
-// Eight wavefronts (two per SIMD: the LDS holds one workgroup per CU).  Wavefront w owns
-// dk column blocks w + 8m and dv column blocks w + 8m of the (chunk x head) gradients,
-// and of the 64x64 chunk matrices row block w % 4, column blocks 2 (w / 4) and
-// 2 (w / 4) + 1.
-constexpr int CW = 8, CNT = 64 * CW;
+// One workgroup of four wavefronts per (chunk, value head).  With dR = X^T dV_new (the
+// gradient of R = diag(beta) (V - diag(e^G) K S), V_new = X R; stored by the reverse scan)
+// the derivative of the solve needs no product with X: dX = dV_new R^T, so
+//     dL = -strict_lower(X^T dX X^T) = -strict_lower(dR V_new^T).
+// The chunk's gradients are then
+//     X1 = diag(e^G) dO S^T          -> dq, G          dP = lower(dO V_new^T)  -> P, G
+//     Z  = dR S^T                    -> dk, beta, G    dL                     -> L, beta, G
+//     Y  = diag(e^{G_last-G}) V_new dS^T -> dk, G      dv = diag(beta) dR
+//     dq = scale (X1 + dPg K),  dk = Y - diag(beta e^G) Z + (Qm + Qm^T) K + scale dPg^T Q,
+// dPg = dP * Gamma, Qm = diag(beta) (dL * Gamma).
+//
+// Bound by memory (328 KiB per workgroup at d = 128, two thirds of it fp32 states and row
+// gradients).  So the tile is chosen for loads in flight: 78 KB of LDS and at most 256
+// VGPRs leave two workgroups per CU, one of which loads while the other multiplies.  The
+// products over dv are formed transposed ([dk][token]: the state's fragments as A operand,
+// the rows as B), so a lane ends with consecutive dk of one token: the row sums are
+// in-lane, the K and Q rows are read and the gradients written by vectors, and every gate
+// is one value per lane.  Wavefront w owns dk rows [CB w, CB w + CB), CB = DK / 4 (16 at
+// dk = 32, on two wavefronts), and of the chunk matrices row block w of dP and 3 - w of dL
+// (five tiles in all: the lower triangles are dealt evenly).
+// C1 (B=4, T=4096, Hk=16, Hv=32, d=128): cgrad 933 -> 553 us, moving 2.9 GB at 5.3 TB/s (the
+// build with the products by X: 156 KB of LDS, one workgroup per CU, 336 KiB, 2.9 TB/s);
+// the core call 1984 -> 1650 us forward and backward.
+constexpr int CW = 4, CNT = 64 * CW;
 
 template <int DK, int DV, bool F32>
-__global__ __launch_bounds__(CNT) void cgrad_kernel(BwdParams p) {
+__global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) void cgrad_kernel(BwdParams p) {
   using KT = typename std::conditional<F32, float, bf16_t>::type;
   using In = KT;  // v has the input precision too
   constexpr int LDK = DK + (F32 ? 4 : 8);
   constexpr int LDB = C + 8;  // stride (bf16) of a split plane: 64 entries and a pad
-  constexpr int NCB = DK / 16, NKB = (NCB + CW - 1) / CW;  // dk column blocks; per wavefront
-  constexpr int NVB = DV / 16, NVW = (NVB + CW - 1) / CW;  // dv column blocks; per wavefront
+  constexpr int NKB = DK >= 128 ? 2 : 1;  // 16-row dk blocks per wavefront
+  constexpr int NACT = DK / 16 / NKB;     // wavefronts that own dk rows
+  static_assert(NACT <= CW && NACT * NKB * 16 == DK, "dk split");
   __shared__ __align__(16) KT sK[C * LDK];
   __shared__ __align__(16) KT sQ[C * LDK];
-  // split planes (hi, lo): dW column-major [dk][token], dPg column-major
-  __shared__ __align__(16) bf16_t sDW[2 * DK * LDB];
-  __shared__ __align__(16) bf16_t sDP[2 * C * LDB];
-  // X (row-major), dX and M1 / Qm (column-major), split; during the products over dv the
-  // region stages their operand rows
-  __shared__ __align__(16) bf16_t sR[3 * 2 * C * LDB];
-  bf16_t* const sXh = sR;
-  bf16_t* const sXl = sR + C * LDB;
-  bf16_t* const sDXh = sR + 2 * C * LDB;
-  bf16_t* const sDXl = sR + 3 * C * LDB;
-  bf16_t* const sMh = sR + 4 * C * LDB;
-  bf16_t* const sMl = sR + 5 * C * LDB;
-  bf16_t* const sDWh = sDW;
-  bf16_t* const sDWl = sDW + DK * LDB;
-  bf16_t* const sDPh = sDP;
-  bf16_t* const sDPl = sDP + C * LDB;
+  // during the products over dv: the staged 32-column slices of dO, dR and V_new; then the
+  // split planes of dPg and Qm, column-major (storage [col][row])
+  constexpr int LDR = 40;  // stride (bf16) of a staged 32-column slice plane
+  constexpr int SZR = 4 * C * LDB > 6 * C * LDR ? 4 * C * LDB : 6 * C * LDR;
+  __shared__ __align__(16) bf16_t sR[SZR];
+  bf16_t* const sDOh = sR;
+  bf16_t* const sDOl = sR + C * LDR;
+  bf16_t* const sDRh = sR + 2 * C * LDR;
+  bf16_t* const sDRl = sR + 3 * C * LDR;
+  bf16_t* const sVNh = sR + 4 * C * LDR;
+  bf16_t* const sVNl = sR + 5 * C * LDR;
+  bf16_t* const sDPh = sR;
+  bf16_t* const sDPl = sR + C * LDB;
+  bf16_t* const sQMh = sR + 2 * C * LDB;
+  bf16_t* const sQMl = sR + 3 * C * LDB;
   __shared__ float sG[C], sBt[C];
-  // per-wavefront partial row / column sums (deterministic: one writer per entry at a time)
-  __shared__ float sRowG[CW][C], sColG[CW][C], sRowB[CW][C], sRowT[CW][C], sRP[CW][C];
+  // partial sums per wavefront (deterministic: every entry has one writer)
+  __shared__ float sX1[CW][C], sZ[CW][C], sY[CW][C];  // rows over the wavefront's dk
+  __shared__ float sCol[CW][C];                       // columns of its tiles of P dP and L dL
+  __shared__ float sRowP[C], sRowL[C], sRowB[C];      // rows of P dP, of L dL, of Lg dL
+  __shared__ float sRV[C];                            // dR . v
   __shared__ float sRed[CW];
 
   const int tid = threadIdx.x, l = tid & 63, lq = l >> 4, lr = l & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool active = NACT == CW || wave < NACT;
   const int Hv = p.Hv, h = blockIdx.x % Hv, ci = blockIdx.x / Hv;
   int n, cc;
   if (p.chunk_off) {
@@ -785,121 +810,35 @@ __global__ __launch_bounds__(CNT) void cgrad_kernel(BwdParams p) {
   const int gqa = Hv / p.Hk, hk = h / gqa;
   const size_t rec_stride = (size_t)rec_bytes(rec_mode(F32), true);
   const float* xb = p.xlpg + ((size_t)ci * Hv + h) * kXlpgFloats;
-  const float* Sg = p.states + ((size_t)ci * Hv + h) * DK * DV;
-  const float* dSg = p.dstates + ((size_t)ci * Hv + h) * DK * DV;
-  const long long rs = (long long)Hv * DV;  // row stride of dO, V_new, dV_new, v
-  const float* dOb = p.dO + t0 * rs + (long long)h * DV;
-  const float* Vnb = p.vnew + t0 * rs + (long long)h * DV;
-  const float* dVnb = p.dvnew + t0 * rs + (long long)h * DV;
-  const In* vb = (const In*)p.v + t0 * rs + (long long)h * DV;
+  const long long rs = (long long)Hv * DV;  // row stride of dO, V_new, dR, v
   const float scale = p.scale;
 
-  // (the gates and the K, Q rows are staged just before the products over dv, together
-  // with the first step's loads)
-  auto eg = [&](int row) { return __expf(sG[row]); };
-  auto el = [&](int row) { return row == C - 1 ? 1.f : __expf(sG[C - 1] - sG[row]); };
-  auto gam = [&](int row, int col) {
-    return row >= col ? __expf(fminf(sG[row] - sG[col], 0.f)) : 0.f;
-  };
-  float* rowG = sRowG[wave];
-  float* colG = sColG[wave];
-  float* rowB = sRowB[wave];
-  float* rowT = sRowT[wave];
-  float* rP = sRP[wave];
+  // dk index of row r of the wavefront's tile t, and of the first of the four consecutive
+  // dk a lane holds of that tile: with two tiles, lane group q holds dk 8q .. 8q + 7
+  const int dk0 = 16 * NKB * (active ? wave : 0);
+  auto dk_row = [&](int t, int r) { return dk0 + (NKB == 2 ? 8 * (r >> 2) + 4 * t + (r & 3) : r); };
+  auto dk_own = [&](int t) { return dk0 + (NKB == 2 ? 8 * lq + 4 * t : 4 * lq); };
 
-  // dq, dk accumulators of the wavefront's dk column blocks cb = wave + 4 kb
-  f32x4 dq[NKB][4], dk[NKB][4];
-
-  // ---------------------------------------------------------------- products over dv
-  // One pass over dv in 32-column steps:
-  //   X1 = diag(e^G) dO S^T, dW = -dV_new S^T, dkdec = V_new dS^T (the wavefront's dk
-  //   column blocks), dP = (dO V_new^T) * tril and dXa = dV_new v^T (its row block bi,
-  //   column blocks 2 half, 2 half + 1).
-  // The step's dO, dV_new, V_new and v rows are staged in LDS as split planes (one
-  // coalesced float4 per thread each, split once) and the state fragments come straight
-  // from global memory; both are loaded into registers one step ahead.
-  constexpr int LDR = 40;  // stride (bf16) of a staged 32-column slice plane
-  static_assert(8 * C * LDR <= 6 * C * LDB, "the staged slices fit the X / dX / M1 region");
-  bf16_t* const sDOh = sR;
-  bf16_t* const sDOl = sR + C * LDR;
-  bf16_t* const sDVh = sR + 2 * C * LDR;
-  bf16_t* const sDVl = sR + 3 * C * LDR;
-  bf16_t* const sVNh = sR + 4 * C * LDR;
-  bf16_t* const sVNl = sR + 5 * C * LDR;
-  bf16_t* const sVh = sR + 6 * C * LDR;  // v: exact in bf16 unless the inputs are fp32
-  bf16_t* const sVl = sR + 7 * C * LDR;
-  const int srow = tid >> 3, sc4 = 4 * (tid & 7);  // this thread's staged item
-  float4 pf_do, pf_dv, pf_vn;
-  typename Vec4<In>::type pf_v;
-  // the chunk's valid rows of dO, dV_new, V_new and v (zeros past them)
-  const unsigned rows_b = (unsigned)(nvalid * rs);  // elements
-  const auto rDO = buf_rsrc(dOb, 4u * rows_b), rDV = buf_rsrc(dVnb, 4u * rows_b);
-  const auto rVN = buf_rsrc(Vnb, 4u * rows_b), rV = buf_rsrc(vb, (unsigned)sizeof(In) * rows_b);
-  auto load_rows = [&](int u) {
-    const unsigned off = (unsigned)(srow * rs + 32 * u + sc4);
-    pf_do = bload4(rDO, 4u * off, (const float*)nullptr);
-    pf_dv = bload4(rDV, 4u * off, (const float*)nullptr);
-    pf_vn = bload4(rVN, 4u * off, (const float*)nullptr);
-    pf_v = bload4(rV, (unsigned)sizeof(In) * off, (const In*)nullptr);
-  };
-  auto f4 = [](float4 x) { return f32x4{x.x, x.y, x.z, x.w}; };
-  auto store_rows = [&]() {
-    const int o = srow * LDR + sc4;
-    put_row4(sDOh, sDOl, o, f4(pf_do));
-    put_row4(sDVh, sDVl, o, f4(pf_dv));
-    put_row4(sVNh, sVNl, o, f4(pf_vn));
-    if constexpr (F32) put_row4(sVh, sVl, o, f4(to_f4(pf_v)));
-    else *(u32x2*)(sVh + o) = *(const u32x2*)&pf_v;
-  };
-  float sfr[NKB][8], dfr[NKB][8];  // state fragments (the states are column-major)
-  float sds = 0.f;  // sum of dS_end * S over the state (each element is loaded once here)
-  auto load_state = [&](int u) {
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
-      // unconditional (a block past NCB reloads the last one, unused): see the dv loop
-      const int cb = wave + CW * kb < NCB ? wave + CW * kb : NCB - 1;
-      gfrag_col(Sg, DK, 16 * cb + lr, 32 * u, sfr[kb]);
-      gfrag_col(dSg, DK, 16 * cb + lr, 32 * u, dfr[kb]);
-    }
-  };
-  float4 pf_x[C * 16 / CNT];  // X, staged after the last step
-  f32x4 dw[NKB][4], dp[2], dxa[2];
-#pragma unroll
-  for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dq[kb][i] = dk[kb][i] = dw[kb][i] = zero4();
-#pragma unroll
-  for (int j = 0; j < 2; ++j) dp[j] = dxa[j] = zero4();
-  const int bi = wave & 3, half = wave >> 2;  // row block and column-block pair
-  // P and Lg at this wavefront's tiles (bi, 2 half + jj), used elementwise after the
-  // products over dv.  fp32 inputs read them from the preparation kernel's matrices; bf16
-  // inputs form them after the products over dv from the staged K and Q rows.
-  float pP[2][4], pLg[2][4];
-  if constexpr (F32) {
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int o = (16 * bi + 4 * lq + v) * C + 16 * (2 * half + jj) + lr;
-        pP[jj][v] = xb[kXlpgP + o];
-        pLg[jj][v] = xb[kXlpgLg + o];
-      }
-  }
   // ---------------------------------------------------------------- stage
   // K and Q rows in 16-byte items, every load issued (with the first step's) before any
-  // store, so the workgroup waits for one memory round trip rather than one per item
+  // store, so the workgroup waits for one memory round trip rather than one per item.  The
+  // chunk's valid rows only (zeros past them, no branch: see bload4).
+  const unsigned rows_b = (unsigned)(nvalid * rs);  // elements
+  const long long ro = t0 * rs + (long long)h * DV;
+  const auto rDO = buf_rsrc(p.dO + ro, 4u * rows_b), rDR = buf_rsrc(p.drows + ro, 4u * rows_b);
+  const auto rVN = buf_rsrc(p.vnew + ro, 4u * rows_b);
+  const auto rV = buf_rsrc((const In*)p.v + ro, (unsigned)sizeof(In) * rows_b);
+  const auto rDV = buf_rsrc((In*)p.dv + ro, (unsigned)sizeof(In) * rows_b);
+  constexpr int EPI = 16 / (int)sizeof(KT);  // elements per item
+  constexpr int PER = C * DK / EPI;          // items per matrix
+  constexpr int NIT = 2 * PER / CNT;
+  static_assert(NIT * CNT == 2 * PER && PER % CNT == 0, "staging split");
+  u32x4 st[NIT];
   {
-    constexpr int EPI = 16 / (int)sizeof(KT);  // elements per item
-    constexpr int PER = C * DK / EPI;          // items per matrix
-    constexpr int NIT = 2 * PER / CNT;
-    static_assert(NIT * CNT == 2 * PER, "staging split");
-    // the chunk's valid rows only (zeros past them, no branch: see bload4)
-    static_assert(PER % CNT == 0, "an item's matrix follows from m alone");
     const auto kr = buf_rsrc((const KT*)p.ks + t0 * p.ks_ld + (long long)hk * DK,
                              (unsigned)(nvalid * p.ks_ld * (long long)sizeof(KT)));
     const auto qr = buf_rsrc((const KT*)p.qs + t0 * p.qs_ld + (long long)hk * DK,
                              (unsigned)(nvalid * p.qs_ld * (long long)sizeof(KT)));
-    u32x4 st[NIT];
 #pragma unroll
     for (int m = 0; m < NIT; ++m) {
       const int which = m * CNT / PER;  // uniform: K items, then Q items
@@ -909,338 +848,361 @@ __global__ __launch_bounds__(CNT) void cgrad_kernel(BwdParams p) {
       st[m] = __builtin_amdgcn_raw_buffer_load_b128(which ? qr : kr,
                                                     (unsigned)((row * ld + c) * (long long)sizeof(KT)), 0, 0);
     }
-    load_rows(0);
-    load_state(0);
-    if (tid < C) {
-      sG[tid] = xb[kXlpgG + tid];
-      sBt[tid] = ((const float*)(p.rec + ((size_t)ci * Hv + h) * rec_stride + kRecG))[kGateBeta * C + tid];
-    }
-    sRowG[wave][l] = 0.f;
-    sColG[wave][l] = 0.f;
-    sRowB[wave][l] = 0.f;
-    sRowT[wave][l] = 0.f;
-    sRP[wave][l] = 0.f;
-#pragma unroll
-    for (int m = 0; m < NIT; ++m) {
-      const int it = tid + m * CNT;
-      const int which = it / PER, rem = it % PER;
-      const int row = rem / (DK / EPI), c = EPI * (rem % (DK / EPI));
-      *(u32x4*)((which ? sQ : sK) + row * LDK + c) = st[m];
-    }
   }
+  // the thread's staged items of a 32-column step: rows srow and srow + 32, 4 columns each
+  constexpr int NRI = C * 8 / CNT;
+  const int srow = tid >> 3, sc4 = 4 * (tid & 7);
+  float4 pf_do[NRI], pf_dr[NRI], pf_vn[NRI];
+  typename Vec4<In>::type pf_v[NRI];
+  // element offset of the thread's item of row srow; the step's columns go in the scalar
+  // offset (a row past the end is past the range without them)
+  const unsigned roff = (unsigned)srow * (unsigned)rs + sc4;
+  auto load_rows = [&](int u) {
+#pragma unroll
+    for (int m = 0; m < NRI; ++m) {
+      const unsigned off = roff + m * (CNT / 8) * (unsigned)rs;
+      pf_do[m] = bload4(rDO, 4u * off, (const float*)nullptr, 4 * 32 * u);
+      pf_dr[m] = bload4(rDR, 4u * off, (const float*)nullptr, 4 * 32 * u);
+      pf_vn[m] = bload4(rVN, 4u * off, (const float*)nullptr, 4 * 32 * u);
+      pf_v[m] = bload4(rV, (unsigned)sizeof(In) * off, (const In*)nullptr, (int)sizeof(In) * 32 * u);
+    }
+  };
+  // state fragments (the states are column-major, [dv][dk]): row dk_row(t, lr), 8
+  // consecutive dv
+  float sfr[NKB][8], dfr[NKB][8];
+  const auto rS = buf_rsrc(p.states + ((size_t)ci * Hv + h) * DK * DV, 4u * DK * DV);
+  const auto rDS = buf_rsrc(p.dstates + ((size_t)ci * Hv + h) * DK * DV, 4u * DK * DV);
+  const unsigned soff = 4u * (8 * lq * DK + dk_row(0, lr));
+  auto load_state = [&](__amdgpu_buffer_rsrc_t r, int u, float (&x)[NKB][8]) {
+    // opaque at each use: hoisted out of the loop, every load's offset would hold a register
+    // of its own instead of being the instruction's immediate
+    unsigned so = soff;
+    asm volatile("" : "+v"(so));
+#pragma unroll
+    for (int t = 0; t < NKB; ++t)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        x[t][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, so + 4u * (e * DK + 4 * t), 4 * 32 * u * DK, 0));
+  };
+  load_rows(0);
+  load_state(rS, 0, sfr);
+  if (tid < C) {
+    sG[tid] = xb[kXlpgG + tid];
+    sBt[tid] = ((const float*)(p.rec + ((size_t)ci * Hv + h) * rec_stride + kRecG))[kGateBeta * C + tid];
+  }
+#pragma unroll
+  for (int m = 0; m < NIT; ++m) {
+    const int it = tid + m * CNT;
+    const int which = it / PER, rem = it % PER;
+    const int row = rem / (DK / EPI), c = EPI * (rem % (DK / EPI));
+    *(u32x4*)((which ? sQ : sK) + row * LDK + c) = st[m];
+  }
+
+  // ---------------------------------------------------------------- products over dv
+  // accumulators [dk][token]: tile t, token block i; lane (q, r) holds dk_own(t) .. +3 of
+  // token 16 i + r
+  f32x4 aq[NKB][4], az[NKB][4], ay[NKB][4];  // dO S^T, dR S^T, V_new dS^T, transposed
+#pragma unroll
+  for (int t = 0; t < NKB; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) aq[t][i] = az[t][i] = ay[t][i] = zero4();
+  // tiles (rp, j) of dO V_new^T and (rl, j) of dR V_new^T at or below the diagonal: of both
+  // for j < 2 (a tile past the diagonal is not formed), of one of them for j >= 2
+  const int rp = wave, rl = 3 - wave;
+  const bool upper = wave >= 2;  // rp >= 2: the tiles j >= 2 are dP's, else dL's
+  f32x4 tp[2], tl[2], tx[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) tp[j] = tl[j] = tx[j] = zero4();
+  float sds = 0.f;                     // sum of dS * S (each element is loaded once here)
+  float rv[NRI];                       // dR . v of the thread's rows, its columns
+#pragma unroll
+  for (int m = 0; m < NRI; ++m) rv[m] = 0.f;
+  auto f4 = [](float4 x) { return f32x4{x.x, x.y, x.z, x.w}; };
   // (the barrier at the top of the first step orders the staging before every read)
-  // not unrolled: with every fragment a plain LDS read, an unrolled loop lets the
-  // scheduler hoist the reads of several steps and run out of registers
 #pragma unroll 1
   for (int u = 0; u < DV / 32; ++u) {
-    // (every barrier in this kernel orders LDS accesses only, as in the reverse scan)
+    // every barrier in this kernel orders LDS accesses only, as in the reverse scan
     lds_barrier();  // the previous step's readers are done
-    store_rows();
-    Op bs[NKB], bd[NKB];
 #pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
-      bs[kb] = split8(sfr[kb]);
-      bd[kb] = split8(dfr[kb]);
-      if (wave + CW * kb < NCB) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sds += sfr[kb][e] * dfr[kb][e];
-      }
+    for (int m = 0; m < NRI; ++m) {
+      const int row = srow + m * (CNT / 8), o = row * LDR + sc4;
+      put_row4(sDOh, sDOl, o, f4(pf_do[m]));
+      put_row4(sDRh, sDRl, o, f4(pf_dr[m]));
+      put_row4(sVNh, sVNl, o, f4(pf_vn[m]));
+      // dv = diag(beta) dR, written here in whole row pieces (rows past the end dropped)
+      const float4 d = pf_dr[m], v4 = to_f4(pf_v[m]);
+      rv[m] += d.x * v4.x + d.y * v4.y + d.z * v4.z + d.w * v4.w;
+      const float bt = sBt[row];
+      const unsigned off = (unsigned)sizeof(In) * (roff + m * (CNT / 8) * (unsigned)rs + 32 * u);
+      if constexpr (F32)
+        __builtin_amdgcn_raw_buffer_store_b128(
+            u32x4{__float_as_uint(bt * d.x), __float_as_uint(bt * d.y), __float_as_uint(bt * d.z),
+                  __float_as_uint(bt * d.w)}, rDV, off, 0, 0);
+      else
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16(bt * d.x, bt * d.y), pack_bf16(bt * d.z, bt * d.w)},
+                                              rDV, off, 0, 0);
     }
-    // The next step's loads, issued after this step's values are consumed (split and summed
-    // above) and unconditionally (the last step reloads its own slices, unused; X's rows,
-    // needed after the loop, load every step): loaded under a branch or hoisted above that
-    // use, they would need other registers than the ones the loop carries, and the copies at
-    // the end of the step would wait for them, turning the prefetch into a stall.
+    Op bs[NKB];
+#pragma unroll
+    for (int t = 0; t < NKB; ++t) bs[t] = split8(sfr[t]);
+    // The next step's loads, each issued after this step's values are consumed and
+    // unconditionally (the last step reloads its own slices, unused): loaded under a branch
+    // or hoisted above that use, they would need other registers than the ones the loop
+    // carries, and the copies at the end of the step would wait for them.
     __builtin_amdgcn_sched_barrier(0);
-    {
-      const int un = u + 1 < DV / 32 ? u + 1 : u;
-      load_rows(un);
-      load_state(un);
-#pragma unroll
-      for (int m = 0; m < C * 16 / CNT; ++m) {
-        const int it = tid + m * CNT;
-        pf_x[m] = load4(xb + kXlpgX + (it >> 4) * C + 4 * (it & 15));
-      }
-    }
+    const int un = u + 1 < DV / 32 ? u + 1 : u;
+    load_rows(un);
+    load_state(rDS, u, dfr);  // this step's, used after the products with S
     lds_barrier();
-    const Op ow = op_vec(sDOh, sDOl, LDR, 16 * bi, 0);  // dO and dV_new rows of block bi
-    const Op vw = op_vec(sDVh, sDVl, LDR, 16 * bi, 0);
+    // the products with S, then those with dS, then the tiles: few operands live at a time
+    // (all of them at once spilled accumulators, whose reloads waited for every load)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const Op ao = op_vec(sDOh, sDOl, LDR, 16 * i, 0);
-      const Op adv = op_vec(sDVh, sDVl, LDR, 16 * i, 0);
-      const Op avn = op_vec(sVNh, sVNl, LDR, 16 * i, 0);
+      const Op ar = op_vec(sDRh, sDRl, LDR, 16 * i, 0);
+      if (active) {
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-        if (wave + CW * kb >= NCB) continue;
-        dq[kb][i] = mm3<true, true>(dq[kb][i], ao, bs[kb]);    // dO S^T
-        dw[kb][i] = mm3<true, true>(dw[kb][i], adv, bs[kb]);   // dV_new S^T
-        dk[kb][i] = mm3<true, true>(dk[kb][i], avn, bd[kb]);   // V_new dS^T
+        for (int t = 0; t < NKB; ++t) {
+          aq[t][i] = mm3<true, true>(aq[t][i], bs[t], ao);
+          az[t][i] = mm3<true, true>(az[t][i], bs[t], ar);
+        }
       }
-      if ((i >> 1) == half) {
-        const Op av = op_vec<F32>(sVh, sVl, LDR, 16 * i, 0);
-        dxa[i & 1] = mm3<true, F32>(dxa[i & 1], vw, av);              // dV_new v^T
-        if (i <= bi) dp[i & 1] = mm3<true, true>(dp[i & 1], ow, avn);  // dO V_new^T
-      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-  }
-  lds_barrier();  // every read of the staged slices is done: the region now holds X
+    Op bd[NKB];
 #pragma unroll
-  for (int m = 0; m < C * 16 / CNT; ++m) {
-    const int it = tid + m * CNT;
-    put_row4(sXh, sXl, (it >> 4) * LDB + 4 * (it & 15), f4(pf_x[m]));
-  }
-  if constexpr (!F32) {
-    // P = lower(scale Q K^T * Gamma) and Lg = strict_lower(K K^T * Gamma) at this
-    // wavefront's tiles, with the preparation kernel's arithmetic (the exact bf16 products
-    // summed by the same MFMA over the same dk blocks in the same order, then
-    // scale * acc * 2^{min(G_i log2 e - G_m log2 e, 0)} * mask), so they are the values it
-    // left in its matrices, without storing and reloading 32 KiB per (chunk, value head)
+    for (int t = 0; t < NKB; ++t) {
+      float x[8];
+      op_values(bs[t], x);
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int bj = 2 * half + jj;
-      f32x4 kk = zero4(), qk = zero4();
+      for (int e = 0; e < 8; ++e) sds += x[e] * dfr[t][e];
+      bd[t] = split8(dfr[t]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load_state(rS, un, sfr);
 #pragma unroll
-      for (int s2 = 0; s2 < DK / 32; ++s2) {
-        const u32x4 km = frag_bf16((const bf16_t*)sK, LDK, 16 * bj, 32 * s2);
-        kk = mma16(frag_bf16((const bf16_t*)sK, LDK, 16 * bi, 32 * s2), km, kk);
-        qk = mma16(frag_bf16((const bf16_t*)sQ, LDK, 16 * bi, 32 * s2), km, qk);
+    for (int j = 0; j < 4; ++j) {
+      const Op av = op_vec(sVNh, sVNl, LDR, 16 * j, 0);
+      if (active) {
+#pragma unroll
+        for (int t = 0; t < NKB; ++t) ay[t][j] = mm3<true, true>(ay[t][j], bd[t], av);
       }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const Op op = op_vec(sDOh, sDOl, LDR, 16 * rp, 0), ol = op_vec(sDRh, sDRl, LDR, 16 * rl, 0);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * bi + 4 * lq + v, col = 16 * bj + lr;
-        const float e = __builtin_amdgcn_exp2f(
-            fminf(sG[row] * 1.4426950408889634f - sG[col] * 1.4426950408889634f, 0.f));
-        pLg[jj][v] = kk[v] * e * (float)(row > col);
-        pP[jj][v] = scale * qk[v] * e * (float)(row >= col);
+    for (int j = 0; j < 4; ++j) {
+      const Op av = op_vec(sVNh, sVNl, LDR, 16 * j, 0);
+      if (j < 2) {
+        if (j <= rp) tp[j] = mm3<true, true>(tp[j], op, av);
+        if (j <= rl) tl[j] = mm3<true, true>(tl[j], ol, av);
+      } else if (upper) {
+        if (j <= rp) tx[j - 2] = mm3<true, true>(tx[j - 2], op, av);
+      } else {
+        if (j <= rl) tx[j - 2] = mm3<true, true>(tx[j - 2], ol, av);
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 #pragma unroll
-  for (int kb = 0; kb < NKB; ++kb) {
-    const int cb = wave + CW * kb;
-    if (cb >= NCB) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f32x4 gx, rr;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * i + 4 * lq + v, col = 16 * cb + lr;
-        dq[kb][i][v] *= eg(row);                           // X1 = diag(e^G) dO S^T
-        gx[v] = scale * ldx(sQ + row * LDK + col) * dq[kb][i][v];
-        const float e = el(row);
-        rr[v] = dk[kb][i][v] * ldx(sK + row * LDK + col) * e;  // dkdec * kdec
-        dk[kb][i][v] *= e;
-      }
-      put_ct(sDWh, sDWl, LDB, 16 * i, 16 * cb, -dw[kb][i]);  // dW = -dV_new S^T
-      add_rows(rowG, i, gx);
-      add_rows(rP, i, rr);
-    }
+  for (int m = 0; m < NRI; ++m) {  // the row's 8 threads
+    const float s = group_sum_dpp<8>(rv[m]);
+    if ((tid & 7) == 0) sRV[srow + m * (CNT / 8)] = s;
   }
-#pragma unroll
-  for (int jj = 0; jj < 2; ++jj) {
-    const int bj = 2 * half + jj;
-    f32x4 pdp, dpg;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = 16 * bi + 4 * lq + v, col = 16 * bj + lr;
-      const float d = row >= col ? dp[jj][v] : 0.f;
-      pdp[v] = d * pP[jj][v];
-      dpg[v] = d * gam(row, col);                          // dPg = dP * Gamma
-    }
-    put_ct(sDPh, sDPl, LDB, 16 * bi, 16 * bj, dpg);
-    add_rows(rowG, bi, pdp);
-    add_cols(colG, bj, -pdp);
-  }
-  // sum of dS_end * S over the state (the e^{G_last} S term of the state update)
   sds = wave_sum(sds);
-  if (l == 0) sRed[wave] = sds;
-  lds_barrier();
+  if (l == 0) sRed[wave] = active ? sds : 0.f;
+  lds_barrier();  // every read of the staged slices is done: the region now holds dPg and Qm
 
-  // ---------------------------------------------------------------- dX = dU vb^T + dW kbe^T
-  {
+  // ---------------------------------------------------------------- rows over dk
+  auto k4 = [&](const KT* m, int row, int col) { return to_f4(*(const typename Vec4<KT>::type*)(m + row * LDK + col)); };
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int bj = 2 * half + jj;
-      f32x4 acc = zero4();
+  for (int i = 0; i < 4; ++i) {
+    const int row = 16 * i + lr;
+    const float eg = __expf(sG[row]), el = row == C - 1 ? 1.f : __expf(sG[C - 1] - sG[row]);
+    float x1 = 0.f, z = 0.f, y = 0.f;
+    if (active) {
 #pragma unroll
-      for (int s = 0; s < DK / 32; ++s)
-        acc = mm3<true, F32>(acc, op_tr(sDWh, sDWl, LDB, 16 * bi, 32 * s),
-                             kq_row<false>(sK, LDK, 16 * bj, 32 * s));
-      const int col = 16 * bj + lr;
-      const float bc = sBt[col], ec = eg(col);
-      f32x4 dx;
+      for (int t = 0; t < NKB; ++t) {
+        const float4 q4 = k4(sQ, row, dk_own(t)), kk = k4(sK, row, dk_own(t));
+        const float qa[4] = {q4.x, q4.y, q4.z, q4.w}, ka[4] = {kk.x, kk.y, kk.z, kk.w};
+        const float bz = sBt[row] * eg;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) dx[v] = bc * (dxa[jj][v] + ec * acc[v]);
-      put_ct(sDXh, sDXl, LDB, 16 * bi, 16 * bj, dx);
-    }
-  }
-  lds_barrier();
-
-  // ---------------------------------------------------------------- dvb = X^T dU, dkbe = X^T dW
-#pragma unroll
-  for (int kv = 0; kv < NVW; ++kv) {
-    const int cv = wave + CW * kv;
-    if (cv >= NVB) continue;
-    // the column's dV_new fragments (one per 32-token half, shared by every row block).
-    // dvb is formed transposed, dvb^T = dV_new^T X (the fragments serve as A operands and
-    // the X^T rows as B operands), so a lane holds 4 consecutive columns of one row: v is
-    // read and dv written 4 columns at a time.
-    Op bo[2];
-    {
-      float b[8];
-      gfrag_col_b(rDV, (unsigned)rs, 16 * cv + lr, 0, b);
-      bo[0] = split8(b);
-      gfrag_col_b(rDV, (unsigned)rs, 16 * cv + lr, 32, b);
-      bo[1] = split8(b);
-    }
-    typename Vec4<In>::type vv4[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 16 * i + lr;
-      vv4[i] = bload4(rV, (unsigned)sizeof(In) * (unsigned)(row * rs + 16 * cv + 4 * lq), (const In*)nullptr);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f32x4 acc = zero4();
-#pragma unroll
-      for (int p2 = i / 2; p2 < 2; ++p2)
-        acc = mm3<true, true>(acc, bo[p2], op_vec(sXh, sXl, LDB, 16 * i, 32 * p2));
-      const int row = 16 * i + lr;
-      const float4 vf = to_f4(vv4[i]);
-      const f32x4 vd = f32x4{vf.x * acc[0], vf.y * acc[1], vf.z * acc[2], vf.w * acc[3]};
-      const float bt = sBt[row];
-      if (row < nvalid) {
-        In* dvo = (In*)p.dv + (t0 + row) * rs + (long long)h * DV + 16 * cv + 4 * lq;
-        if constexpr (F32) *(float4*)dvo = float4{bt * acc[0], bt * acc[1], bt * acc[2], bt * acc[3]};
-        else *(u32x2*)dvo = u32x2{pack_bf16(bt * acc[0], bt * acc[1]), pack_bf16(bt * acc[2], bt * acc[3])};
-      }
-      add_cols(rowB, i, vd);  // row 16 i + r of the chunk: the transposed tile's column r
-    }
-  }
-#pragma unroll
-  for (int kb = 0; kb < NKB; ++kb) {
-    const int cb = wave + CW * kb;
-    if (cb >= NCB) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f32x4 acc = zero4();
-#pragma unroll
-      for (int p2 = i / 2; p2 < 2; ++p2)
-        acc = mm3<true, true>(acc, op_vec(sXh, sXl, LDB, 16 * i, 32 * p2),
-                              op_vec(sDWh, sDWl, LDB, 16 * cb, 32 * p2));
-      f32x4 kt;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * i + 4 * lq + v, col = 16 * cb + lr;
-        kt[v] = ldx(sK + row * LDK + col) * acc[v];
-        dk[kb][i][v] += sBt[row] * eg(row) * acc[v];
-      }
-      add_rows(rowT, i, kt);
-    }
-  }
-  // M1 = X^T dX
-  {
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int bj = 2 * half + jj;
-      f32x4 acc = zero4();
-      for (int p2 = bi / 2; p2 < 2; ++p2)  // X^T is upper triangular
-        acc = mm3<true, true>(acc, op_vec(sXh, sXl, LDB, 16 * bi, 32 * p2),
-                              op_vec(sDXh, sDXl, LDB, 16 * bj, 32 * p2));
-      put_ct(sMh, sMl, LDB, 16 * bi, 16 * bj, acc);
-    }
-  }
-  lds_barrier();  // M1 complete (a row block's two halves come from two wavefronts)
-  // ---------------------------------------------------------------- dL = -strict_lower(M1 X^T)
-  {
-    f32x4 dl[2];
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int bj = 2 * half + jj;
-      f32x4 acc = zero4();
-      if (bj <= bi) {
-#pragma unroll
-        for (int p2 = 0; p2 < 2; ++p2)  // B: rows of X
-          if (p2 <= bj / 2)
-            acc = mm3<true, true>(acc, op_tr(sMh, sMl, LDB, 16 * bi, 32 * p2),
-                                  op_tr(sXh, sXl, LDB, 16 * bj, 32 * p2));
-      }
-      dl[jj] = acc;
-    }
-    lds_barrier();  // every read of M1 is complete before its rows are overwritten
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int bj = 2 * half + jj;
-      f32x4 lb, ld, qm;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * bi + 4 * lq + v, col = 16 * bj + lr;
-        const float d = row > col ? -dl[jj][v] : 0.f;
-        const float lg = pLg[jj][v];
-        lb[v] = d * lg;
-        ld[v] = d * sBt[row] * lg;                      // dL * L
-        qm[v] = sBt[row] * d * gam(row, col);           // Qm = diag(beta) (dL * Gamma)
-      }
-      put_ct(sMh, sMl, LDB, 16 * bi, 16 * bj, qm);
-      add_rows(rowB, bi, lb);
-      add_rows(rowG, bi, ld);
-      add_cols(colG, bj, -ld);
-    }
-  }
-  lds_barrier();
-
-  // ---------------------------------------------------------------- (Qm + Qm^T) k, dPg^T qs, dPg k
-#pragma unroll
-  for (int kb = 0; kb < NKB; ++kb) {
-    const int cb = wave + CW * kb;
-    if (cb >= NCB) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f32x4 a_k = dk[kb][i], a_q = dq[kb][i], a_t = zero4();
-#pragma unroll
-      for (int p2 = 0; p2 < 2; ++p2) {
-        const Op bk = kq_col<false>(sK, LDK, 16 * cb, 32 * p2);
-        // (Qm + Qm^T) k as Qm k + Qm^T k
-        a_k = mm3<true, F32>(a_k, op_tr(sMh, sMl, LDB, 16 * i, 32 * p2), bk);
-        a_k = mm3<true, F32>(a_k, op_vec(sMh, sMl, LDB, 16 * i, 32 * p2), bk);
-        if (p2 <= i / 2)  // dPg is lower triangular
-          a_q = mm3<true, F32>(a_q, op_tr(sDPh, sDPl, LDB, 16 * i, 32 * p2), bk);
-        if (p2 >= i / 2)  // dPg^T is upper triangular
-          a_t = mm3<true, F32>(a_t, op_vec(sDPh, sDPl, LDB, 16 * i, 32 * p2),
-                               kq_col<false>(sQ, LDK, 16 * cb, 32 * p2));
-      }
-      // per value head rows at the input precision: the q/k finalisation sums them and
-      // rounds to that precision anyway
-      KT* dqo = (KT*)p.dqh + (t0 * Hv + h) * (long long)DK;
-      KT* dko = (KT*)p.dkh + (t0 * Hv + h) * (long long)DK;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * i + 4 * lq + v, col = 16 * cb + lr;
-        if (row < nvalid) {
-          dqo[(long long)row * Hv * DK + col] = from_f32<KT>(scale * a_q[v]);
-          dko[(long long)row * Hv * DK + col] = from_f32<KT>(a_k[v] + scale * a_t[v]);
+        for (int v = 0; v < 4; ++v) {
+          aq[t][i][v] *= eg;
+          ay[t][i][v] *= el;
+          x1 += qa[v] * aq[t][i][v];
+          z += ka[v] * az[t][i][v];
+          y += ka[v] * ay[t][i][v];
+          ay[t][i][v] -= bz * az[t][i][v];  // dk so far
         }
       }
     }
+    // over the lane groups, which hold the same token's other dk
+    auto rows4 = [&](float s) {
+      const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+      s = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+      const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+      return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    };
+    x1 = rows4(x1);
+    z = rows4(z);
+    y = rows4(y);
+    if (lq == 0) {
+      sX1[wave][row] = scale * x1;
+      sZ[wave][row] = z;
+      sY[wave][row] = y;
+    }
+  }
+  // ---------------------------------------------------------------- dP and dL tiles
+  // P = lower(scale Q K^T * Gamma) and Lg = strict_lower(K K^T * Gamma) at this wavefront's
+  // tiles: fp32 inputs read them from the preparation kernel's matrices, bf16 inputs form
+  // them with its arithmetic (the same products summed by the same MFMA over the same dk
+  // blocks in the same order)
+  {
+    f32x4 rowp = zero4(), rowl = zero4(), rowb = zero4();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x4 cg = zero4();
+      const int col = 16 * j + lr;
+      const float gc = sG[col] * 1.4426950408889634f;
+      if (j <= rp) {  // uniform
+        const f32x4 d4 = j < 2 ? tp[j] : tx[j - 2];
+        f32x4 pp = zero4(), dpg;
+        if constexpr (!F32) {
+#pragma unroll
+          for (int s2 = 0; s2 < DK / 32; ++s2)
+            pp = mma16(frag_bf16((const bf16_t*)sQ, LDK, 16 * rp, 32 * s2),
+                       frag_bf16((const bf16_t*)sK, LDK, 16 * j, 32 * s2), pp);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = 16 * rp + 4 * lq + v;
+          const float e = __builtin_amdgcn_exp2f(fminf(sG[row] * 1.4426950408889634f - gc, 0.f));
+          const float d = row >= col ? d4[v] : 0.f;
+          const float x = d * (F32 ? xb[kXlpgP + row * C + col] : scale * pp[v] * e);
+          rowp[v] += x;
+          cg[v] += x;
+          dpg[v] = d * e;                                // dPg = dP * Gamma
+        }
+        put_ct(sDPh, sDPl, LDB, 16 * rp, 16 * j, dpg);
+      }
+      if (j <= rl) {  // uniform
+        const f32x4 d4 = j < 2 ? tl[j] : tx[j - 2];
+        f32x4 kk = zero4(), qm;
+        if constexpr (!F32) {
+#pragma unroll
+          for (int s2 = 0; s2 < DK / 32; ++s2)
+            kk = mma16(frag_bf16((const bf16_t*)sK, LDK, 16 * rl, 32 * s2),
+                       frag_bf16((const bf16_t*)sK, LDK, 16 * j, 32 * s2), kk);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = 16 * rl + 4 * lq + v;
+          const float e = __builtin_amdgcn_exp2f(fminf(sG[row] * 1.4426950408889634f - gc, 0.f));
+          const float d = row > col ? -d4[v] : 0.f;      // dL
+          const float x = d * (F32 ? xb[kXlpgLg + row * C + col] : kk[v] * e);
+          const float y = sBt[row] * x;                  // dL * L
+          rowb[v] += x;
+          rowl[v] += y;
+          cg[v] += y;
+          qm[v] = sBt[row] * d * e;                      // Qm = diag(beta) (dL * Gamma)
+        }
+        put_ct(sQMh, sQMl, LDB, 16 * rl, 16 * j, qm);
+      }
+      set_cols(sCol[wave], j, cg);
+    }
+    set_rows(sRowP, rp, rowp);
+    set_rows(sRowL, rl, rowl);
+    set_rows(sRowB, rl, rowb);
+    // the tiles above the diagonal that complete the block pairs of row blocks 0 and 2
+    if (wave < 2) put_ct(sDPh, sDPl, LDB, 32 * wave, 32 * wave + 16, zero4());
+    else put_ct(sQMh, sQMl, LDB, 32 * (wave - 2), 32 * (wave - 2) + 16, zero4());
   }
   lds_barrier();
+
+  // ---------------------------------------------------------------- dPg K, (Qm + Qm^T) K, dPg^T Q
+  if (active) {
+    Op ko[NKB][2], qo[NKB][2];  // K and Q columns dk_row(t, .), slots over 32 tokens
+#pragma unroll
+    for (int t = 0; t < NKB; ++t)
+#pragma unroll
+      for (int p2 = 0; p2 < 2; ++p2) {
+        if constexpr (F32) {
+          float x[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[e] = sK[(32 * p2 + 8 * lq + e) * LDK + dk_row(t, lr)];
+          ko[t][p2] = split8(x);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[e] = sQ[(32 * p2 + 8 * lq + e) * LDK + dk_row(t, lr)];
+          qo[t][p2] = split8(x);
+        } else {
+          // source lane s of a 16-lane group points at row s / 4 and the 4 columns of row
+          // group s % 4 (see ds_read_tr)
+          const int o = (32 * p2 + 8 * lq + (lr >> 2)) * LDK + dk_row(t, 4 * (lr & 3));
+          const u32x2 a = ds_read_tr((const bf16_t*)sK + o), b = ds_read_tr((const bf16_t*)sK + o + 4 * LDK);
+          const u32x2 c = ds_read_tr((const bf16_t*)sQ + o), d = ds_read_tr((const bf16_t*)sQ + o + 4 * LDK);
+          ko[t][p2].h = ko[t][p2].l = u32x4{a[0], a[1], b[0], b[1]};
+          qo[t][p2].h = qo[t][p2].l = u32x4{c[0], c[1], d[0], d[1]};
+        }
+      }
+    // per value head rows at the input precision: the q/k finalisation sums them and
+    // rounds to that precision anyway
+    const long long oo = (t0 * Hv + h) * (long long)DK;
+    const unsigned ob = (unsigned)(nvalid * (long long)Hv * DK * (long long)sizeof(KT));
+    const auto rdq = buf_rsrc((KT*)p.dqh + oo, ob), rdk = buf_rsrc((KT*)p.dkh + oo, ob);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f32x4 a_t[NKB];
+#pragma unroll
+      for (int t = 0; t < NKB; ++t) a_t[t] = zero4();
+#pragma unroll
+      for (int p2 = 0; p2 < 2; ++p2) {
+        if (p2 <= i / 2) {  // lower triangular: rows of block i
+          const Op b = op_tr(sQMh, sQMl, LDB, 16 * i, 32 * p2), d = op_tr(sDPh, sDPl, LDB, 16 * i, 32 * p2);
+#pragma unroll
+          for (int t = 0; t < NKB; ++t) {
+            ay[t][i] = mm3<F32, true>(ay[t][i], ko[t][p2], b);
+            aq[t][i] = mm3<F32, true>(aq[t][i], ko[t][p2], d);
+          }
+        }
+        if (p2 >= i / 2) {  // transposes: upper triangular
+          const Op b = op_vec(sQMh, sQMl, LDB, 16 * i, 32 * p2), d = op_vec(sDPh, sDPl, LDB, 16 * i, 32 * p2);
+#pragma unroll
+          for (int t = 0; t < NKB; ++t) {
+            ay[t][i] = mm3<F32, true>(ay[t][i], ko[t][p2], b);
+            a_t[t] = mm3<F32, true>(a_t[t], qo[t][p2], d);
+          }
+        }
+      }
+      // token 16 i + r, the lane's consecutive dk (rows past the end dropped)
+      const unsigned off = (unsigned)(((16 * i + lr) * (long long)Hv * DK + dk_own(0)) * (long long)sizeof(KT));
+      float xq[4 * NKB], xk[4 * NKB];
+#pragma unroll
+      for (int t = 0; t < NKB; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          xq[4 * t + v] = scale * aq[t][i][v];
+          xk[4 * t + v] = ay[t][i][v] + scale * a_t[t][v];
+        }
+      store_row<KT, 4 * NKB>(rdq, off, xq);
+      store_row<KT, 4 * NKB>(rdk, off, xk);
+    }
+  }
 
   // ---------------------------------------------------------------- dG, dbeta, dg
   if (wave == 0) {
     const int i = l;
-    float rg = 0.f, rt = 0.f, rb = 0.f, rp = 0.f;
+    float rg = sRowP[i] + sRowL[i], rz = 0.f, ry = 0.f;
 #pragma unroll
     for (int w = 0; w < CW; ++w) {
-      rg += sRowG[w][i] + sColG[w][i] - sRP[w][i];
-      rt += sRowT[w][i];
-      rb += sRowB[w][i];
-      rp += sRP[w][i];
+      rg += sX1[w][i] - sCol[w][i];
+      rz += sZ[w][i];
+      ry += sY[w][i];
     }
-    const float t = __expf(sG[i]) * rt;
-    float dG = rg + sBt[i] * t;
-    const float db = rb + t;
-    const float rsum = wave_sum(rp);
+    const float t = -__expf(sG[i]) * rz;  // of -diag(e^G) K S in R
+    float dG = rg - ry + sBt[i] * t;
+    const float db = sRV[i] + sRowB[i] + t;
+    const float rsum = wave_sum(ry);
     float sds = 0.f;
 #pragma unroll
     for (int w = 0; w < CW; ++w) sds += sRed[w];

@@ -99,11 +99,11 @@ ChunkWs chunk_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64
 
 // Workspace of the backward pass: the forward's (records, normalised q/k, chunk
 // offsets), then the prep's fp32 X, Lg, P, G per (chunk slot, value head), the state
-// entering and the state gradient leaving every chunk, V_new and its gradient, and the
+// entering and the state gradient leaving every chunk, V_new and X^T dV_new, and the
 // per-value-head gradients of the normalised q and k.
 struct BwdWs {
   ChunkWs f;
-  size_t xlpg, states, dstates, vnew, dvnew, dqh, dkh, total;
+  size_t xlpg, states, dstates, vnew, drows, dqh, dkh, total;
 };
 
 BwdWs bwd_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64_t dv, int64_t N,
@@ -122,7 +122,7 @@ BwdWs bwd_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64_t d
   o += align_up(slots * (size_t)(Hv * dk * dv) * 4, 256);
   w.vnew = o;
   o += align_up(tokens * (size_t)(Hv * dv) * 4, 256);
-  w.dvnew = o;
+  w.drows = o;
   o += align_up(tokens * (size_t)(Hv * dv) * 4, 256);
   w.dqh = o;
   o += align_up(tokens * (size_t)(Hv * dk) * 4, 256);
@@ -860,7 +860,7 @@ int chunk_bwd_core(const char* fn, const void* q, const void* k, const void* v, 
   b.v = v; b.dO = d_o; b.dht = d_final_state; b.rec = p.rec; b.xlpg = p.xlpg;
   b.states = p.states; b.vnew = p.vnew;
   b.dstates = (float*)(base + ws.dstates);
-  b.dvnew = (float*)(base + ws.dvnew);
+  b.drows = (float*)(base + ws.drows);
   b.dh0 = d_initial_state;
   b.dqh = base + ws.dqh;  // sized for fp32; bf16 inputs use the first half
   b.dkh = base + ws.dkh;
@@ -1122,7 +1122,7 @@ int prefill_bwd_core(const char* fn, const void* mixed_qkv, const void* z, const
   bp.v = lp.v; bp.dO = lp.dO; bp.dht = d_final_state; bp.rec = p.rec; bp.xlpg = p.xlpg;
   bp.states = p.states; bp.vnew = p.vnew;
   bp.dstates = (float*)(base + ws.c.dstates);
-  bp.dvnew = (float*)(base + ws.c.dvnew);
+  bp.drows = (float*)(base + ws.c.drows);
   bp.dh0 = d_initial_state;
   bp.dqh = base + ws.c.dqh;
   bp.dkh = base + ws.c.dkh;

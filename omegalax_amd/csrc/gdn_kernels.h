@@ -115,7 +115,7 @@ struct BwdParams {
   const float* states;         // state entering each chunk [slot][Hv][DV][dk]
   const float* vnew;           // V_new
   float* dstates;              // gradient of the state leaving each chunk [slot][Hv][DV][dk]
-  float* dvnew;                // gradient of V_new [tokens][Hv][DV]
+  float* drows;                // X^T times the gradient of V_new [tokens][Hv][DV]
   float* dh0;                  // [N][Hv][dk][DV] or null
   void* dqh;                   // per value head gradient of the normalised q [tokens][Hv][dk],
                                // at the input precision (bf16 or fp32)
