@@ -331,7 +331,8 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
   // loaders' writes to one from the compute wavefronts' reads of the other.
   __shared__ __align__(16) KT sK0[C * LDK], sK1[LDR ? C * LDK : 8];
   __shared__ __align__(16) KT sQ0[C * LDK], sQ1[LDR ? C * LDK : 8];
-  // dO (this block's 64 columns), X^T and (fp32 inputs) P, row-major, as bf16 hi / lo planes
+  // dO (this block's 64 columns), X (fp32 inputs: X^T) and (fp32 inputs) P, row-major, as
+  // bf16 hi / lo planes
   __shared__ __align__(16) bf16_t sDO0[2 * C * LDB], sDO1[LDR ? 2 * C * LDB : 8];
   __shared__ __align__(16) bf16_t sX0[2 * C * LDB], sX1[LDR ? 2 * C * LDB : 8];
   __shared__ __align__(16) bf16_t sP[PREC ? 8 : 2 * C * LDB];
@@ -400,9 +401,12 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
   // chunk step later.
   constexpr int NKQ = 2 * C * (DK / 4) / NT;
   static_assert(NKQ * NT == 2 * C * (DK / 4), "item split");
+  constexpr int NXP = 2 * kNPairs * 64 / NT;  // (PREC) 16-byte pieces of the record's X
+  static_assert(NXP * NT == 2 * kNPairs * 64, "record pieces");
   struct Pf {
     typename Vec4<KT>::type pkq[NKQ];
-    float4 pdo[C * 16 / NT], pxp[(PREC ? 1 : 2) * C * 16 / NT];
+    float4 pdo[C * 16 / NT], pxp[PREC ? 1 : 2 * C * 16 / NT];
+    u32x4 px[PREC ? NXP : 1];
     float pgate, pg;
   };
   // chunk jj into f; every call issues the same loads (a chunk before the sequence's first
@@ -433,15 +437,21 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
       const int row = it >> 4, c4 = 4 * (it & 15);
       f.pdo[m] = bload4(dr, (unsigned)(4 * (row * rs + c4)), (const float*)nullptr);
     }
-    const float* xb = p.xlpg + ((size_t)sl * p.Hv + h) * kXlpgFloats;
+    const float* xb = p.xlpg + ((size_t)sl * p.Hv + h) * xlpg_floats(F32);
+    const unsigned char* rec = p.rec + ((size_t)sl * p.Hv + h) * rec_stride;
+    if constexpr (PREC) {
 #pragma unroll
-    for (int m = 0; m < (PREC ? 1 : 2) * C * 16 / NT; ++m) {
-      const int it = st + m * NT;
-      const int which = it / (C * 16), rem = it % (C * 16);
-      f.pxp[m] = load4(xb + (which ? kXlpgP : kXlpgX) + (rem >> 4) * C + 4 * (rem & 15));
+      for (int m = 0; m < NXP; ++m) f.px[m] = *(const u32x4*)(rec + kRecT + 16 * (st + m * NT));
+      f.pg = xb[kXlpgG + (st & (C - 1))];
+    } else {
+#pragma unroll
+      for (int m = 0; m < 2 * C * 16 / NT; ++m) {
+        const int it = st + m * NT;
+        const int which = it / (C * 16), rem = it % (C * 16);
+        f.pxp[m] = load4(xb + (which ? kXlpgP : kXlpgX) + (rem >> 4) * C + 4 * (rem & 15));
+      }
     }
-    if constexpr (PREC) f.pg = xb[kXlpgG + (st & (C - 1))];
-    f.pgate = ((const float*)(p.rec + ((size_t)sl * p.Hv + h) * rec_stride + kRecG))[st];
+    f.pgate = ((const float*)(rec + kRecG))[st];
   };
   auto store_chunk = [&](const Pf& f, const Buf& bf) {
     bf16_t* const sDOh = bf.DO;
@@ -460,13 +470,26 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
       const int it = st + m * NT;
       put_row4(sDOh, sDOl, (it >> 4) * LDB + 4 * (it & 15), f32x4{f.pdo[m].x, f.pdo[m].y, f.pdo[m].z, f.pdo[m].w});
     }
+    if constexpr (PREC) {
+      // piece 2x + part of the record's T part: lane (q, r) of pair x = (ib, jp) holds
+      // X[16 ib + r][32 jp + 4q .. +3] and [32 jp + 16 + 4q .. +3], hi (part 0) or lo
 #pragma unroll
-    for (int m = 0; m < (PREC ? 1 : 2) * C * 16 / NT; ++m) {
-      const int it = st + m * NT;
-      const int which = it / (C * 16), rem = it % (C * 16);
-      const f32x4 v = f32x4{f.pxp[m].x, f.pxp[m].y, f.pxp[m].z, f.pxp[m].w};
-      if (which) put_row4(sPh, sPl, (rem >> 4) * LDB + 4 * (rem & 15), v);
-      else put_row4(sXh, sXl, (rem >> 4) * LDB + 4 * (rem & 15), v);
+      for (int m = 0; m < NXP; ++m) {
+        const int piece = (st >> 6) + m * (NT / 64), x = piece >> 1;  // uniform per wavefront
+        const int ib = x < 3 ? x : x == 3 ? 2 : 3, jp = x == 3 || x == 5;
+        bf16_t* d = (piece & 1 ? sXl : sXh) + (16 * ib + lr) * LDB + 32 * jp + 4 * lq;
+        *(u32x2*)d = u32x2{f.px[m][0], f.px[m][1]};
+        *(u32x2*)(d + 16) = u32x2{f.px[m][2], f.px[m][3]};
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < 2 * C * 16 / NT; ++m) {
+        const int it = st + m * NT;
+        const int which = it / (C * 16), rem = it % (C * 16);
+        const f32x4 v = f32x4{f.pxp[m].x, f.pxp[m].y, f.pxp[m].z, f.pxp[m].w};
+        if (which) put_row4(sPh, sPl, (rem >> 4) * LDB + 4 * (rem & 15), v);
+        else put_row4(sXh, sXl, (rem >> 4) * LDB + 4 * (rem & 15), v);
+      }
     }
     if constexpr (PREC)
       if (st < C) bf.Gl[st] = f.pg;
@@ -621,8 +644,8 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
       f32x4 acc = zero4();
       dr[i] = zero4();
 #pragma unroll
-      for (int p2 = i / 2; p2 < 2; ++p2) {  // X^T is upper triangular; X^T rows (stored transposed)
-        const Op x = op_pair(sXh, sXl, LDB, 16 * i, 32 * p2);
+      for (int p2 = i / 2; p2 < 2; ++p2) {  // X^T is upper triangular
+        const Op x = PREC ? op_tr_pair(sXh, sXl, LDB, 16 * i, 32 * p2) : op_pair(sXh, sXl, LDB, 16 * i, 32 * p2);
         acc = mm3<true, true>(acc, x, dvp[p2]);
         dr[i] = mm3<true, true>(dr[i], dvp[p2], x);
       }
@@ -809,7 +832,7 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (nvalid <= 0) return;
   const int gqa = Hv / p.Hk, hk = h / gqa;
   const size_t rec_stride = (size_t)rec_bytes(rec_mode(F32), true);
-  const float* xb = p.xlpg + ((size_t)ci * Hv + h) * kXlpgFloats;
+  const float* xb = p.xlpg + ((size_t)ci * Hv + h) * xlpg_floats(F32);
   const long long rs = (long long)Hv * DV;  // row stride of dO, V_new, dR, v
   const float scale = p.scale;
 

@@ -98,7 +98,7 @@ ChunkWs chunk_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64
 }
 
 // Workspace of the backward pass: the forward's (records, normalised q/k, chunk
-// offsets), then the prep's fp32 X, Lg, P, G per (chunk slot, value head), the state
+// offsets), then the prep's G (and, fp32 inputs, X, Lg, P) per (chunk slot, value head), the state
 // entering and the state gradient leaving every chunk, V_new and X^T dV_new, and the
 // per-value-head gradients of the normalised q and k.
 struct BwdWs {
@@ -115,7 +115,7 @@ BwdWs bwd_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64_t d
   const size_t slots = (tokens + 63) / 64 + (size_t)N;
   size_t o = w.f.total;
   w.xlpg = o;
-  o += align_up(slots * (size_t)Hv * omx::kXlpgFloatsHost * 4, 256);
+  o += align_up(slots * (size_t)Hv * omx::xlpg_floats_host(mode == omx::kModeF32) * 4, 256);
   w.states = o;
   o += align_up(slots * (size_t)(Hv * dk * dv) * 4, 256);
   w.dstates = o;

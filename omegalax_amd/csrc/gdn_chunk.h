@@ -43,14 +43,15 @@ constexpr int kRecBytesF32 = kRecPL + kNPairs * kPairBytes;  // 25600
 // replaced by e^{G_last}), beta
 constexpr int kGateEG = 0, kGateEGS = 1, kGateEL = 2, kGateBeta = 3;
 
-// backward extras per (chunk slot, value head), fp32 row-major 64x64 matrices:
-// X^T (X = (I + L)^-1, upper triangular as stored), Lg = strict_lower(K K^T * Gamma)
-// (L = diag(beta) Lg), P, then G.  Lg and P are written for fp32 inputs only: with bf16
-// inputs the backward kernels form the Lg and P tiles they need from K, Q and G
+// backward extras per (chunk slot, value head): G, then, for fp32 inputs only, the fp32
+// row-major 64x64 matrices X^T (X = (I + L)^-1, upper triangular as stored), Lg =
+// strict_lower(K K^T * Gamma) (L = diag(beta) Lg) and P.  With bf16 inputs the backward
+// kernels form the Lg and P tiles they need from K, Q and G, and read X from the record,
+// whose T part then holds X itself (without diag(beta)) as bf16 hi + lo
 constexpr int kXlpgMat = kC * kC;
-constexpr int kXlpgX = 0, kXlpgLg = kXlpgMat, kXlpgP = 2 * kXlpgMat, kXlpgG = 3 * kXlpgMat;
-constexpr int kXlpgFloats = 3 * kXlpgMat + kC;
-static_assert(kXlpgFloats == kXlpgFloatsHost, "backward extras layout");
+constexpr int kXlpgG = 0, kXlpgX = kC, kXlpgLg = kC + kXlpgMat, kXlpgP = kC + 2 * kXlpgMat;
+constexpr int xlpg_floats(bool f32) { return xlpg_floats_host(f32); }
+static_assert(kC == 64 && xlpg_floats(true) == kC + 3 * kXlpgMat, "backward extras layout");
 
 // Layer mode with dk = 128 (the scan's direct-load path): the value channels' conv +
 // SiLU runs in the scan's helper wavefronts, so the prep forms the q and k rows only.

@@ -726,7 +726,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
       tl[x] = *(const u32x4*)(tp + kPairBytes);
     }
     // R = V - diag(e^G) K S at rows 16i + 4lq + v, column 16w + lr (diag(beta) is
-    // folded into the record's T)
+    // folded into the record's T, except in a bf16 backward's, where it enters R here)
     f32x4 R[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -735,6 +735,10 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
       R[i][1] = vv[i][1] - eg.y * KS[i][1];
       R[i][2] = vv[i][2] - eg.z * KS[i][2];
       R[i][3] = vv[i][3] - eg.w * KS[i][3];
+      if constexpr (BWD && !IS) {
+        const float4 bt = *(const float4*)(sGate + kGateBeta * C + 16 * i + 4 * lq);
+        R[i] = f32x4{bt.x * R[i][0], bt.y * R[i][1], bt.z * R[i][2], bt.w * R[i][3]};
+      }
     }
 
     // ------------------------------------------------------------ V_new = T diag(beta) R

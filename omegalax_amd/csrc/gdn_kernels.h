@@ -96,7 +96,8 @@ struct ChunkParams {
   const void* vs;
   long long ks_ld, qs_ld, vs_ld;
   // backward pass only (the backward variants of the two kernels write them)
-  float* xlpg;                 // prep: per (chunk slot, value head) X^T, Lg, P [64][64], G [64]
+  float* xlpg;                 // prep: per (chunk slot, value head) G [64] (fp32 inputs: and
+                               // X^T, Lg, P [64][64])
   float* states;               // scan: the state entering each chunk [slot][Hv][DV][dk]
   float* vnew;                 // scan: V_new [tokens][Hv][DV]
 };
@@ -134,8 +135,9 @@ struct BwdParams {
   float scale;
 };
 
-// floats of the backward extras per (chunk slot, value head): X, Lg, P [64][64], G [64]
-constexpr int kXlpgFloatsHost = 3 * 64 * 64 + 64;
+// floats of the backward extras per (chunk slot, value head): G [64], and for fp32 inputs
+// X^T, Lg, P [64][64]
+constexpr int xlpg_floats_host(bool f32) { return 64 + (f32 ? 3 * 64 * 64 : 0); }
 
 // kernel modes of the chunked prefill (template arguments of both kernels)
 constexpr int kModeBF16 = 0, kModeF32 = 1, kModeLayer = 2;

@@ -254,9 +254,12 @@ __device__ __forceinline__ void put_f32_tile(float* m, int bi, int bj, f32x4 a) 
   *(float4*)(m + (16 * bi + (l & 15)) * kC + 16 * bj + 4 * (l >> 4)) = float4{a[0], a[1], a[2], a[3]};
 }
 
-// BWD: also writes, per (chunk, value head), the fp32 matrices the backward pass reads
-// (X^T with X = (I + L)^-1, Lg = strict_lower(K K^T * Gamma), P, and G; layout in
-// gdn_chunk.h).
+// BWD: also writes, per (chunk, value head), G and (fp32 inputs) the fp32 matrices the
+// backward pass reads (X^T with X = (I + L)^-1, Lg = strict_lower(K K^T * Gamma) and P;
+// layout in gdn_chunk.h).  With bf16 inputs the record's T part holds X itself, which both
+// the recompute scan (with diag(beta) on its right-hand side) and the reverse scan read, so
+// that X is not written a second time: at C1 the backward's prep 112 -> 90 us, the recompute
+// scan 296 -> 285 us, the reverse scan 320 -> 308 us.
 template <int DK, int MODE, bool BWD = false>
 __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_kernel(ChunkParams p) {
   using Q_ = PrepCfg<DK, MODE>;
@@ -426,15 +429,15 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
     for (int gg = 0; gg < gqa; ++gg) {
       const int h = hk * gqa + gg;
       const auto rec = buf_rsrc(p.rec + ((size_t)ci * p.Hv + h) * rec_stride, (unsigned)rec_stride);
-      float* xb = BWD ? p.xlpg + ((size_t)ci * p.Hv + h) * kXlpgFloats : nullptr;
-      if constexpr (BWD) {
-        // the lower tiles of X^T and (fp32 inputs) the upper tiles of Lg and P are zero
-        for (int z = wave; z < (IS ? 18 : 6); z += 4) {
+      float* xb = BWD ? p.xlpg + ((size_t)ci * p.Hv + h) * xlpg_floats(IS) : nullptr;
+      if constexpr (BWD && IS) {
+        // the lower tiles of X^T and the upper tiles of Lg and P are zero
+        for (int z = wave; z < 18; z += 4) {
           const int mat = z / 6, u = z % 6;
           const int bi = u < 3 ? 0 : (u < 5 ? 1 : 2);
           const int bj = u < 3 ? u + 1 : (u < 5 ? u - 1 : 3);
           if (mat == 0) put_f32_tile(xb + kXlpgX, bj, bi, zero4());
-          else if (IS) put_f32_tile(xb + mat * kXlpgMat, bi, bj, zero4());
+          else put_f32_tile(xb + kXlpgX + mat * kXlpgMat, bi, bj, zero4());
         }
       }
 
@@ -577,10 +580,11 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
             const u32x2 th = pack_hi4(Ta), tl = pack_lo4(Ta);
             sTd[(2 * bi) * 64 + l] = th;  // A fragments of T_ww for the other waves
             sTd[(2 * bi + 1) * 64 + l] = tl;
-            // the record holds T diag(beta): column 16 bi + 4 lq + v scaled by its beta
-            const f32x4 Tb = Ta * col_beta(gw, bi);
+            // the record holds T diag(beta): column 16 bi + 4 lq + v scaled by its beta (a
+            // bf16 backward's, T itself: its reverse scan reads T^T from there)
+            const f32x4 Tb = BWD && !IS ? Ta : Ta * col_beta(gw, bi);
             put_tile(rec, rec_t_off(bi, bi), pack_hi4(Tb));
-            if constexpr (BWD) put_f32_tile(xb + kXlpgX, bi, bi, Tc);  // X^T: the C layout
+            if constexpr (BWD && IS) put_f32_tile(xb + kXlpgX, bi, bi, Tc);  // X^T: the C layout
             put_tile(rec, rec_t_off(bi, bi) + kPairBytes, pack_lo4(Tb));
             if ((bi & 1) == 0) {
               // the zero upper tile (bi, bi + 1) that completes row block bi's last pair
@@ -644,9 +648,9 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
           const f32x4 TijT = mm3k16(zero4(), xh, xl, th, tl);
           Th[i] = pack_hi4(Tij);
           Tl[i] = pack_lo4(Tij);
-          const f32x4 Tb = TijT * col_beta(gw, j);  // T_ij diag(beta), A layout
+          const f32x4 Tb = BWD && !IS ? TijT : TijT * col_beta(gw, j);  // T_ij diag(beta), A layout
           put_tile(rec, rec_t_off(i, j), pack_hi4(Tb));
-          if constexpr (BWD) put_f32_tile(xb + kXlpgX, j, i, Tij);  // X^T: the C layout
+          if constexpr (BWD && IS) put_f32_tile(xb + kXlpgX, j, i, Tij);  // X^T: the C layout
           put_tile(rec, rec_t_off(i, j) + kPairBytes, pack_lo4(Tb));
         }
       }
