@@ -7,15 +7,15 @@
 //   o = chunk_gated_delta_rule(q, k, v, g, beta) (fp32);
 //   out = w_n * o * rsqrt(mean(o^2) + eps) * silu(z).
 // Kernels here, in the order the backward runs them:
-//   conv_silu_split_kernel  y from x and w, as the forward's prep computes it, into
-//                           separate q, k, v rows for the rule's backward;
-//   gates_kernel            g and beta per (token, value head);
+//   fwd_pieces_kernel       y from x and w, as the forward's prep computes it, into
+//                           separate q, k, v rows for the rule's backward, and g and beta
+//                           per (token, value head);
 //   norm_bwd_kernel         the gated RMSNorm's adjoint: do, dz and per-workgroup partial
 //                           sums of dw_n (o comes from the rule's recompute scan);
-//   gates_bwd_kernel        da, db and per-workgroup partial sums of dA_log, d dt_bias;
-//   conv_bwd_kernel         du = dy silu'(u), dx (the transposed conv) and per-token-block
+//   tail_bwd_kernel         da, db and per-workgroup partial sums of dA_log, d dt_bias;
+//                           du = dy silu'(u), dx (the transposed conv) and per-token-block
 //                           partial sums of dw;
-//   col_reduce_kernel       the partial sums in a fixed order (deterministic results).
+//   reduce_kernel           all partial sums in a fixed order (deterministic results).
 // Dtype casts are differentiated as the identity, as autodiff does.
 #include "gdn_chunk.h"
 #include "gdn_kernels.h"
@@ -88,10 +88,9 @@ __device__ __forceinline__ float silu_grad(float u) {
 // 3-token halo).
 constexpr int kConvFwdTB = 16;
 
-__global__ __launch_bounds__(NT) void conv_silu_split_kernel(LayerBwdParams p) {
+__device__ __forceinline__ void conv_silu_split(const LayerBwdParams& p, long long idx) {
   const int G = p.conv_dim / 8;
   const long long nblk = (p.tokens + kConvFwdTB - 1) / kConvFwdTB;
-  const long long idx = (long long)blockIdx.x * NT + threadIdx.x;
   if (idx >= nblk * G) return;
   const long long tb = (idx / G) * kConvFwdTB;
   const long long te = tb + kConvFwdTB < p.tokens ? tb + kConvFwdTB : p.tokens;
@@ -144,12 +143,18 @@ __global__ __launch_bounds__(NT) void conv_silu_split_kernel(LayerBwdParams p) {
 }
 
 // one thread per (token, value head): g and beta as the forward's prep forms them
-__global__ __launch_bounds__(NT) void gates_kernel(LayerBwdParams p) {
-  const long long idx = (long long)blockIdx.x * NT + threadIdx.x;
+__device__ __forceinline__ void gates(const LayerBwdParams& p, long long idx) {
   if (idx >= p.tokens * p.Hv) return;
   const int h = (int)(idx % p.Hv);
   p.g[idx] = -expf(p.A_log[h]) * softplusf_(bf2f(p.a[idx]) + p.dt_bias[h]);
   p.beta[idx] = round_bf(sigmoidf_(bf2f(p.b[idx])));
+}
+
+// The first gate_blocks workgroups form the gates, the rest the conv: one launch, so the
+// gates cost no launch and drain of their own (4.8 us at 3,001 tokens).
+__global__ __launch_bounds__(NT) void fwd_pieces_kernel(LayerBwdParams p, unsigned gate_blocks) {
+  if (blockIdx.x < gate_blocks) gates(p, (long long)blockIdx.x * NT + threadIdx.x);
+  else conv_silu_split(p, (long long)(blockIdx.x - gate_blocks) * NT + threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------- gated RMSNorm
@@ -218,19 +223,19 @@ __global__ __launch_bounds__(NT) void norm_bwd_kernel(LayerBwdParams p) {
 
 // ---------------------------------------------------------------------------- gates
 
-// Workgroup w takes a contiguous token range; thread (j, h) = (tid / Hv, tid % Hv) walks its
+// Workgroup w of the gate part takes a contiguous token range; thread (j, h) = (tid / Hv, tid % Hv) walks its
 // tokens j, j + R, ... (R = 256 / Hv) for value head h.
 //   da = dg A sigmoid(a + dt_bias), A = -exp(A_log); db = dbeta sigmoid(b)(1 - sigmoid(b));
 //   dA_log = sum dg g, d dt_bias = sum da.
-__global__ __launch_bounds__(NT) void gates_bwd_kernel(LayerBwdParams p, long long per) {
-  __shared__ float sacc[NT][2];
+__device__ __forceinline__ void gates_bwd(const LayerBwdParams& p, long long blk, long long per,
+                                          float (*sacc)[2]) {
   const int Hv = p.Hv, tid = threadIdx.x;
   const int R = NT / Hv;
   const int h = tid % Hv, j = tid / Hv;
   float sA = 0.f, sdt = 0.f;
   if (j < R) {
     const float A = -expf(p.A_log[h]), dtb = p.dt_bias[h];
-    const long long t0 = (long long)blockIdx.x * per;
+    const long long t0 = blk * per;
     const long long t1 = t0 + per < p.tokens ? t0 + per : p.tokens;
     for (long long t = t0 + j; t < t1; t += R) {
       const long long i = t * Hv + h;
@@ -252,197 +257,259 @@ __global__ __launch_bounds__(NT) void gates_bwd_kernel(LayerBwdParams p, long lo
       a0 += sacc[jj * Hv + tid][0];
       a1 += sacc[jj * Hv + tid][1];
     }
-    p.part_gates[(size_t)blockIdx.x * 2 * Hv + tid] = a0;
-    p.part_gates[(size_t)blockIdx.x * 2 * Hv + Hv + tid] = a1;
+    p.part_gates[(size_t)blk * 2 * Hv + tid] = a0;
+    p.part_gates[(size_t)blk * 2 * Hv + Hv + tid] = a1;
   }
 }
 
 // ---------------------------------------------------------------------------- conv + SiLU
 
-// One thread per (64-token block, 8-channel group).  du = dy silu'(u) with u recomputed;
-// dx[s] = sum_d wt[d] du[s + d] over s + d inside s's sequence (the transposed conv);
-// dwt[d] = sum_t du[t] x[t - d] (x = 0 before the sequence start), written per token block.
-constexpr int kConvTB = 64;
+// One workgroup per (64 tokens, 256 channels): wavefront w takes tokens 16w .. 16w + 15 of
+// the block, a lane 4 channels.  du = dy silu'(u) with u recomputed;
+//   dx[s] = sum_d wt[d] du[s + d], dwt[d] = sum_t du[t] x[t - d],
+// both over the pairs (t, d) whose token t - d lies in t's sequence.  Token t's du enters
+// dx[t - d], so the wavefront also forms du of the three tokens after its own.
+//
+// Every row it needs (22 of x, 19 of dy) is loaded before the first use, and the 4 x 256
+// channels of a workgroup make 1,500 workgroups of 3,001 tokens x 8,192 channels: with one
+// thread walking 64 tokens with a one-row prefetch the kernel waited for one row after the
+// other (188 workgroups, 61 us there, and 21 us for the gates in a launch of their own; now
+// 40 us for both, 147 MB at 3.7 TB/s).  The four wavefronts' dwt are summed in LDS, so the
+// partial sums stay one per 64 tokens.
+constexpr int kConvTB = 64;  // tokens per workgroup
+constexpr int kConvSB = 16;  // tokens per wavefront
 
-__global__ __launch_bounds__(NT) void conv_bwd_kernel(LayerBwdParams p) {
-  const int G = p.conv_dim / 8;
-  const long long nblk = (p.tokens + kConvTB - 1) / kConvTB;
-  const long long idx = (long long)blockIdx.x * NT + threadIdx.x;
-  if (idx >= nblk * G) return;
-  const long long blk = idx / G;
-  const int c0 = 8 * (int)(idx % G);
-  const int kd = p.Hk * p.dk;
-  const long long vd = (long long)p.Hv * p.dv;
-  const bf16_t* dys;
-  long long dy_ld;
-  int dy_c;
-  if (c0 < kd) { dys = p.grad_q; dy_ld = kd; dy_c = c0; }
-  else if (c0 < 2 * kd) { dys = p.grad_k; dy_ld = kd; dy_c = c0 - kd; }
-  else { dys = p.grad_v; dy_ld = vd; dy_c = c0 - 2 * kd; }
-  float wt[8][4];
-  conv_w8(p.conv_w, c0, wt);
-  const long long tb = blk * kConvTB;
-  const long long te = tb + kConvTB < p.tokens ? tb + kConvTB : p.tokens;
-  float dwt[8][4];
+__device__ __forceinline__ void conv_bwd(const LayerBwdParams& p, long long bid, float (*sdw)[64][16]) {
+  const int nchg = (p.conv_dim + 255) / 256;
+  const long long blk = bid / nchg;
+  const int l = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cg = 256 * (int)(bid % nchg), c0 = cg + 4 * l;
+  const bool in = c0 < p.conv_dim;
+  const int cc = in ? c0 : p.conv_dim - 4;  // lanes past the channels load the last ones
+  const long long tb = blk * kConvTB + wave * kConvSB;
+  float dwt[4][4];  // [channel][d]
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
+  for (int e = 0; e < 4; ++e)
 #pragma unroll
     for (int d = 0; d < 4; ++d) dwt[e][d] = 0.f;
-  // rolling windows: xs[d] = x[t - d]; dus[d] = du[t - d] (the last four du computed)
-  float xs[4][8], dus[4][8];
+  if (tb < p.tokens) {  // uniform
+    const int kd = p.Hk * p.dk;
+    const long long vd = (long long)p.Hv * p.dv;
+    const bf16_t* dys;
+    long long dy_ld;
+    if (cc < kd) { dys = p.grad_q + cc; dy_ld = kd; }
+    else if (cc < 2 * kd) { dys = p.grad_k + (cc - kd); dy_ld = kd; }
+    else { dys = p.grad_v + (cc - 2 * kd); dy_ld = vd; }
+    const long long last = p.tokens - 1;
+    // rows outside the tokens reload one inside; the masks below leave them out
+    u32x2 xr[kConvSB + 6], dyr[kConvSB + 3];
 #pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    zero8(xs[d]);
-    zero8(dus[d]);
-  }
-  long long cs0, cs1;  // sequence of the current token t
-  token_seq(p.cu_seqlens, p.N, p.T, tb, cs0, cs1);
-#pragma unroll
-  for (int d = 1; d < 4; ++d)
-    if (tb - d >= cs0) load8(p.x + (tb - d) * p.conv_dim + c0, xs[d]);
-  // ends[d]: the end of token t - d's sequence (the rows a dx term may reach)
-  long long ends[4] = {cs1, cs1, cs1, cs1};
-  const long long tend = te + 3 < p.tokens ? te + 3 : p.tokens;
-  // The next token's x and dy rows are loaded one iteration ahead, unconditionally (the
-  // last iteration reloads its own row), and every iteration stores one dx row (see
-  // below): no memory operation sits under a per-thread branch, which would leave the
-  // count of outstanding operations unknown and make each wait for a load cover the
-  // stores as well.  The loads before the loop have landed.
-  u32x4 nx = *(const u32x4*)(p.x + tb * p.conv_dim + c0);
-  u32x4 ndy = *(const u32x4*)(dys + tb * dy_ld + dy_c);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  for (long long t = tb; t < tend; ++t) {
-    const u32x4 cx = nx, cdy = ndy;
-    {
-      const long long tn = t + 1 < tend ? t + 1 : t;
-      nx = *(const u32x4*)(p.x + tn * p.conv_dim + c0);
-      ndy = *(const u32x4*)(dys + tn * dy_ld + dy_c);
-    }
-    if (t >= cs1) {  // a new sequence starts at t: no history
-      token_seq(p.cu_seqlens, p.N, p.T, t, cs0, cs1);
-#pragma unroll
-      for (int d = 1; d < 4; ++d) zero8(xs[d]);
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the lookup's loads end here
+    for (int k = 0; k < kConvSB + 6; ++k) {
+      long long t = tb - 3 + k;
+      t = t < 0 ? 0 : (t > last ? last : t);
+      xr[k] = *(const u32x2*)(p.x + t * p.conv_dim + cc);
     }
 #pragma unroll
-    for (int d = 3; d > 0; --d) ends[d] = ends[d - 1];
-    ends[0] = cs1;
-    unpack8<false>(&cx, xs[0]);
-    float dy[8];
-    unpack8<false>(&cdy, dy);
-    float du[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      du[e] = dy[e] * silu_grad(conv_u(wt[e], xs[0][e], xs[1][e], xs[2][e], xs[3][e]));
-    if (t < te) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-#pragma unroll
-        for (int d = 0; d < 4; ++d) dwt[e][d] += du[e] * xs[d][e];
+    for (int k = 0; k < kConvSB + 3; ++k) {
+      const long long t = tb + k < last ? tb + k : last;
+      dyr[k] = *(const u32x2*)(dys + t * dy_ld);
     }
-    // shift the du window; a sequence boundary cuts it (du of another sequence is 0 here)
+    float wt[4][4];
+    uint32_t w01[4], w23[4];
 #pragma unroll
-    for (int d = 3; d > 0; --d)
+    for (int e = 0; e < 4; ++e) {
+      const float4 w = *(const float4*)(p.conv_w + (size_t)(cc + e) * 4);
+      w01[e] = pack_bf16(w.w, w.z);  // the forward's bf16 weights; wt[e][d]: d tokens back
+      w23[e] = pack_bf16(w.y, w.x);
+      wt[e][0] = __uint_as_float(w01[e] << 16);
+      wt[e][1] = __uint_as_float(w01[e] & 0xffff0000u);
+      wt[e][2] = __uint_as_float(w23[e] << 16);
+      wt[e][3] = __uint_as_float(w23[e] & 0xffff0000u);
+    }
+    // bit k of back[d]: token tb + k - d lies in token tb + k's sequence.  A sequence that
+    // starts at token b clears bits b - tb .. b - tb + d - 1 of back[d].
+    unsigned back[4];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) dus[d][e] = dus[d - 1][e];
+    for (int d = 0; d < 4; ++d) back[d] = 0xffffffffu;
+    auto start_at = [&](long long b) {
+      const int k = (int)(b - tb);  // -2 .. kConvSB + 2
 #pragma unroll
-    for (int e = 0; e < 8; ++e) dus[0][e] = du[e];
-    // dx[s] for s = t - 3 needs du[s .. s + 3] = dus[3 .. 0]; terms past s's sequence end
-    // are dropped (tokens s + d >= end(s) belong to the next sequence)
-    // (s < te always: t < te + 3.)  Rows s < tb (the first three iterations) store to
-    // row tb instead, which this thread writes again later (here or in the tail below),
-    // so the store need not sit under a branch.
-    const long long s = t - 3;
-    {
-      const long long ss1 = ends[3];  // end of s's sequence
-      float dx[8];
+      for (int d = 1; d < 4; ++d)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float acc = 0.f;
-#pragma unroll
-        for (int d = 0; d < 4; ++d)
-          if (s + d < ss1) acc += wt[e][d] * dus[3 - d][e];
-        dx[e] = acc;
+        for (int m = 0; m < d; ++m)
+          if (k + m >= 0) back[d] &= ~(1u << (k + m));
+    };
+    const long long t2 = tb > 2 ? tb - 2 : 0, tend = tb + kConvSB + 3;
+    if (p.cu_seqlens) {
+      int lo = 0, hi = p.N;  // the last sequence with cu[n] <= t2
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (p.cu_seqlens[mid] <= t2) lo = mid;
+        else hi = mid;
       }
-      const long long sw = s >= tb ? s : tb;
-      *(u32x4*)(p.dx + sw * p.conv_dim + c0) = pack8(dx);
+      for (int n = lo; n < p.N; ++n) {
+        const long long b = p.cu_seqlens[n];
+        if (b >= tend) break;
+        if (b >= t2) start_at(b);
+      }
+    } else {
+      for (long long b = (t2 + p.T - 1) / p.T * p.T; b < tend; b += p.T) start_at(b);
     }
+    // the rows this wavefront owns (rows past the tokens and lanes past the channels are
+    // outside the range: dropped, no branch)
+    const long long rows = p.tokens - tb < kConvSB ? p.tokens - tb : kConvSB;
+    const auto dxr = buf_rsrc(p.dx + tb * p.conv_dim, 2u * (unsigned)(rows * p.conv_dim));
+    const unsigned drop = 0xffffffffu;
+    float xf[4][4];  // [d][channel]: x[t - d]
 #pragma unroll
-    for (int d = 3; d > 0; --d)
+    for (int d = 1; d < 4; ++d)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) xs[d][e] = xs[d - 1][e];
-  }
-  // the block's last tokens whose du window runs past the end of all tokens
-  for (long long s = (te - 3 > tb ? te - 3 : tb); s < te; ++s) {
-    if (s + 3 < tend) continue;  // already written in the loop
-    long long ss0, ss1;
-    token_seq(p.cu_seqlens, p.N, p.T, s, ss0, ss1);
-    const long long last = tend - 1;  // dus[0] holds du[last]
-    float dx[8];
+      for (int e = 0; e < 4; ++e) xf[d][e] = __uint_as_float(e & 1 ? xr[3 - d][e >> 1] & 0xffff0000u : xr[3 - d][e >> 1] << 16);
+    float dx[4][4];  // [d][channel]: dx[t - d] so far
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float acc = 0.f;
+    for (int d = 0; d < 4; ++d)
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const long long tt = s + d;
-        const int back = (int)(last - tt);
-        if (tt < ss1 && tt <= last && back < 4) {
-          float v = 0.f;
+      for (int e = 0; e < 4; ++e) dx[d][e] = 0.f;
 #pragma unroll
-          for (int b = 0; b < 4; ++b)
-            if (b == back) v = dus[b][e];
-          acc += wt[e][d] * v;
+    for (int k = 0; k < kConvSB + 3; ++k) {
+      if (tb + k < p.tokens) {  // uniform
+        u32x2 x1 = xr[k + 2], x2 = xr[k + 1], x3 = xr[k];
+        const u32x2 x0 = xr[k + 3];
+        const u32x2 zero = {0u, 0u};
+        if (!(back[1] >> k & 1)) x1 = zero;
+        if (!(back[2] >> k & 1)) x2 = zero;
+        if (!(back[3] >> k & 1)) x3 = zero;
+        float du[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const unsigned sel = e & 1 ? 0x07060302u : 0x05040100u;
+          const float u = round_bf(dot4_bf16(w01[e], w23[e], __builtin_amdgcn_perm(x1[e >> 1], x0[e >> 1], sel),
+                                             __builtin_amdgcn_perm(x3[e >> 1], x2[e >> 1], sel)));
+          xf[0][e] = __uint_as_float(e & 1 ? x0[e >> 1] & 0xffff0000u : x0[e >> 1] << 16);
+          du[e] = __uint_as_float(e & 1 ? dyr[k][e >> 1] & 0xffff0000u : dyr[k][e >> 1] << 16) * silu_grad(u);
+        }
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          if (back[d] >> k & 1) {  // uniform
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              dx[d][e] += wt[e][d] * du[e];
+              if (k < kConvSB) dwt[e][d] += du[e] * xf[d][e];
+            }
+          }
         }
       }
-      dx[e] = acc;
-    }
-    *(u32x4*)(p.dx + s * p.conv_dim + c0) = pack8(dx);
-  }
-  // partial dw in [c][k] order (k = 3 - d)
-  float* part = p.part_conv + (size_t)blk * p.conv_dim * 4 + (size_t)c0 * 4;
+      if (k >= 3)
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16(dx[3][0], dx[3][1]), pack_bf16(dx[3][2], dx[3][3])}, dxr,
+                                              in ? 2u * (unsigned)((k - 3) * p.conv_dim + c0) : drop, 0, 0);
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
-    *(float4*)(part + 4 * e) = float4{dwt[e][3], dwt[e][2], dwt[e][1], dwt[e][0]};
+      for (int d = 3; d > 0; --d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          dx[d][e] = dx[d - 1][e];
+          xf[d][e] = xf[d - 1][e];
+        }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dx[0][e] = 0.f;
+    }
+  }
+  // dw in [c][tap] order (tap = 3 - d), the wavefronts' sums in order
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    *(float4*)&sdw[wave][l][4 * e] = float4{dwt[e][3], dwt[e][2], dwt[e][1], dwt[e][0]};
+  __syncthreads();
+  const int c = cg + (int)threadIdx.x;
+  if (c < p.conv_dim) {
+    float4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kConvTB / kConvSB; ++w) {
+      const float4 v = *(const float4*)&sdw[w][threadIdx.x >> 2][4 * (threadIdx.x & 3)];
+      t = float4{t.x + v.x, t.y + v.y, t.z + v.z, t.w + v.w};
+    }
+    *(float4*)(p.part_conv + ((size_t)blk * p.conv_dim + c) * 4) = t;
+  }
 }
 
-// out[c] = sum over rows r of part[r * stride + off + c], c < ncols: COLS columns per
-// workgroup and NT / COLS row groups (rows r = rg mod NT/COLS), each summing its rows into
-// four accumulators; the partial sums are combined in a fixed order, so the result does not
+// The first gate_blocks workgroups take the gates, the rest the conv (one launch for both)
+__global__ __launch_bounds__(NT) void tail_bwd_kernel(LayerBwdParams p, unsigned gate_blocks, long long per) {
+  __shared__ __align__(16) float sdw[kConvTB / kConvSB][64][16];
+  if (blockIdx.x < gate_blocks) gates_bwd(p, blockIdx.x, per, (float (*)[2])sdw);
+  else conv_bwd(p, blockIdx.x - gate_blocks, sdw);
+}
+
+// out[c] = sum over rows r of part[r * stride + c], c < ncols: COLS columns per workgroup
+// and NT / COLS row groups (rows r = rg mod NT/COLS), each summing its rows into sixteen
+// accumulators, so that sixteen loads are in flight (the norm's 4,096 rows bound the launch:
+// 20.6 us with four); the partial sums are combined in a fixed order, so the result does not
 // depend on timing.
+struct ReduceJob {
+  const float* part;
+  float* out;
+  long long nrows;
+  int stride, ncols;
+  unsigned blocks;  // workgroups of this job
+};
+struct ReduceJobs {
+  ReduceJob j[4];
+};
+
 template <int COLS>
-__global__ __launch_bounds__(NT) void col_reduce_kernel(const float* part, long long nrows,
-                                                        int stride, int off, int ncols, float* out) {
+__device__ __forceinline__ void col_reduce(const ReduceJob& q, unsigned blk, float* s_part) {
   constexpr int RG = NT / COLS;
-  __shared__ float s_part[RG][COLS];
   const int cl = threadIdx.x % COLS, rg = threadIdx.x / COLS;
-  const int c = blockIdx.x * COLS + cl;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  if (c < ncols) {
-    long long r = rg;
-    for (; r + 3 * RG < nrows; r += 4 * RG) {
+  const int c = (int)blk * COLS + cl;
+  constexpr int U = 16;
+  float acc[U];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) acc[u] += part[(r + u * RG) * stride + off + c];
+  for (int u = 0; u < U; ++u) acc[u] = 0.f;
+  if (c < q.ncols) {
+    long long r = rg;
+    for (; r + (U - 1) * RG < q.nrows; r += U * RG) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc[u] += q.part[(r + u * RG) * q.stride + c];
     }
-    for (; r < nrows; r += RG) acc[0] += part[r * stride + off + c];
+    for (; r + 3 * RG < q.nrows; r += 4 * RG) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[u] += q.part[(r + u * RG) * q.stride + c];
+    }
+    for (; r < q.nrows; r += RG) acc[0] += q.part[r * q.stride + c];
   }
-  s_part[rg][cl] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+  for (int w = U / 2; w > 0; w >>= 1)
+#pragma unroll
+    for (int u = 0; u < w; ++u) acc[u] += acc[u + w];
+  s_part[threadIdx.x] = acc[0];
   __syncthreads();
-  if (rg == 0 && c < ncols) {
+  if (rg == 0 && c < q.ncols) {
     float t = 0.f;
-    for (int g = 0; g < RG; ++g) t += s_part[g][cl];
-    out[c] = t;
+    for (int g = 0; g < RG; ++g) t += s_part[g * COLS + cl];
+    q.out[c] = t;
   }
 }
 
 // narrow column groups (more row groups) for the few-column reductions
-void launch_col_reduce(const float* part, long long nrows, int stride, int off, int ncols,
-                       float* out, hipStream_t stream) {
-  if (ncols <= 2048)
-    hipLaunchKernelGGL((col_reduce_kernel<8>), dim3((ncols + 7) / 8), dim3(NT), 0, stream, part,
-                       nrows, stride, off, ncols, out);
-  else
-    hipLaunchKernelGGL((col_reduce_kernel<32>), dim3((ncols + 31) / 32), dim3(NT), 0, stream, part,
-                       nrows, stride, off, ncols, out);
+constexpr int kReduceNarrow = 2048;
+
+// All four parameter gradients in one launch (each launch and drain of its own cost about
+// 4.7 us at 3,001 tokens)
+__global__ __launch_bounds__(NT) void reduce_kernel(ReduceJobs jobs) {
+  __shared__ float s_part[NT];
+  unsigned b = blockIdx.x;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const ReduceJob& q = jobs.j[i];
+    if (b < q.blocks) {  // uniform
+      if (q.ncols <= kReduceNarrow) col_reduce<8>(q, b, s_part);
+      else col_reduce<32>(q, b, s_part);
+      return;
+    }
+    b -= q.blocks;
+  }
+}
+
+ReduceJob reduce_job(const float* part, long long nrows, int stride, int ncols, float* out) {
+  const int cols = ncols <= kReduceNarrow ? 8 : 32;
+  return ReduceJob{part, out, nrows, stride, ncols, (unsigned)((ncols + cols - 1) / cols)};
 }
 
 }  // namespace
@@ -451,39 +518,39 @@ int layer_bwd_norm_blocks() { return 4096; }
 
 long long layer_bwd_conv_blocks(long long tokens) { return (tokens + kConvTB - 1) / kConvTB; }
 
+// about four tokens per thread at 32 value heads; at 256 tokens per workgroup the gates of
+// 3,001 tokens ran on 12 workgroups (21 us)
 int layer_bwd_gate_blocks(long long tokens) {
-  const long long b = (tokens + 255) / 256;
+  const long long b = (tokens + 31) / 32;
   return (int)(b < 1024 ? (b < 1 ? 1 : b) : 1024);
 }
 
 hipError_t launch_layer_fwd_pieces(const LayerBwdParams& p, hipStream_t stream) {
   const long long n1 = (p.tokens + kConvFwdTB - 1) / kConvFwdTB * (p.conv_dim / 8);
   if (n1 > 0) {
-    hipLaunchKernelGGL(conv_silu_split_kernel, dim3((unsigned)((n1 + NT - 1) / NT)), dim3(NT), 0,
-                       stream, p);
-    const long long n2 = p.tokens * p.Hv;
-    hipLaunchKernelGGL(gates_kernel, dim3((unsigned)((n2 + NT - 1) / NT)), dim3(NT), 0, stream, p);
+    const unsigned gb = (unsigned)((p.tokens * p.Hv + NT - 1) / NT);
+    hipLaunchKernelGGL(fwd_pieces_kernel, dim3(gb + (unsigned)((n1 + NT - 1) / NT)), dim3(NT), 0, stream, p, gb);
   }
   return hipGetLastError();
 }
 
 hipError_t launch_layer_norm_bwd(const LayerBwdParams& p, hipStream_t stream) {
   hipLaunchKernelGGL(norm_bwd_kernel, dim3(layer_bwd_norm_blocks()), dim3(NT), 0, stream, p);
-  launch_col_reduce(p.part_norm, layer_bwd_norm_blocks(), p.dv, 0, p.dv, p.d_norm_w, stream);
   return hipGetLastError();
 }
 
 hipError_t launch_layer_tail_bwd(const LayerBwdParams& p, hipStream_t stream) {
   const int gb = layer_bwd_gate_blocks(p.tokens);
   const long long per = (p.tokens + gb - 1) / gb;
-  hipLaunchKernelGGL(gates_bwd_kernel, dim3(gb), dim3(NT), 0, stream, p, per);
-  launch_col_reduce(p.part_gates, gb, 2 * p.Hv, 0, p.Hv, p.dA_log, stream);
-  launch_col_reduce(p.part_gates, gb, 2 * p.Hv, p.Hv, p.Hv, p.d_dt_bias, stream);
   const long long nblk = layer_bwd_conv_blocks(p.tokens);
-  const long long n = nblk * (p.conv_dim / 8);
-  if (n > 0)
-    hipLaunchKernelGGL(conv_bwd_kernel, dim3((unsigned)((n + NT - 1) / NT)), dim3(NT), 0, stream, p);
-  launch_col_reduce(p.part_conv, nblk, p.conv_dim * 4, 0, p.conv_dim * 4, p.d_conv_w, stream);
+  const unsigned cb = (unsigned)(nblk * ((p.conv_dim + 255) / 256));
+  hipLaunchKernelGGL(tail_bwd_kernel, dim3((unsigned)gb + cb), dim3(NT), 0, stream, p, (unsigned)gb, per);
+  const ReduceJobs jobs{{reduce_job(p.part_conv, nblk, p.conv_dim * 4, p.conv_dim * 4, p.d_conv_w),
+                         reduce_job(p.part_norm, layer_bwd_norm_blocks(), p.dv, p.dv, p.d_norm_w),
+                         reduce_job(p.part_gates, gb, 2 * p.Hv, p.Hv, p.dA_log),
+                         reduce_job(p.part_gates + p.Hv, gb, 2 * p.Hv, p.Hv, p.d_dt_bias)}};
+  const unsigned rb = jobs.j[0].blocks + jobs.j[1].blocks + jobs.j[2].blocks + jobs.j[3].blocks;
+  hipLaunchKernelGGL(reduce_kernel, dim3(rb), dim3(NT), 0, stream, jobs);
   return hipGetLastError();
 }
 

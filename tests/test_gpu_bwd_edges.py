@@ -1,0 +1,60 @@
+"""GPU parity of the backward kernels at the edges of their tiles, against the fp64 oracle.
+
+The gradient kernel works on 16-token row blocks of 64-token chunks and forms dbeta without
+dividing by beta (beta = 0 is a padding token's gate); the layer tail's conv adjoint gives a
+wavefront 16 tokens and masks the taps at every sequence start.  Tolerances as in
+tests/test_gpu_bwd.py and tests/test_gpu_layer_bwd.py, whose inputs these reuse.
+"""
+import numpy as np
+import pytest
+
+import test_gpu_bwd as core
+import test_gpu_layer_bwd as layer
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,dk,dv,dtype", [
+    (15, 128, 128, "bf16"), (16, 128, 64, "bf16"), (17, 64, 128, "bf16"), (63, 128, 128, "bf16"),
+    (65, 128, 128, "bf16"), (79, 64, 64, "bf16"), (17, 64, 64, "f32"), (65, 32, 64, "f32"),
+])
+def test_core_backward_at_row_block_edges(T, dk, dv, dtype):
+    core.say(f"bwd edges T={T} dk={dk} dv={dv} {dtype}")
+    args = core.make(7000 + T + dk, 2, T, 2, 4, dk, dv, dtype)
+    core.check(core.run_gpu(*args, dtype), core.run_ref(*args, dtype), dtype)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_core_backward_with_zero_and_one_beta(dtype):
+    """dbeta of a token with beta = 0 is its derivative, not 0 / 0."""
+    core.say(f"bwd beta in {{0, 1}} {dtype}")
+    args = list(core.make(7100, 1, 90, 1, 2, 64, 64, dtype))
+    beta = args[4]
+    beta[:, ::3] = 0.0
+    beta[:, 1::3] = 1.0
+    got = core.run_gpu(*args, dtype)
+    assert all(np.isfinite(x).all() for x in got)
+    core.check(got, core.run_ref(*args, dtype), dtype)
+
+
+@pytest.mark.parametrize("lens,Hk,Hv,dk,dv", [
+    ([1], 1, 1, 64, 64),                              # one token; 192 channels (not a multiple of 256)
+    ([2, 1, 1, 3], 1, 2, 64, 64),                     # sequences shorter than the conv window
+    ([15, 1, 2, 14, 17, 15], 1, 1, 64, 128),          # starts on both sides of 16-token edges
+    ([62, 1, 1, 3, 64, 0, 5], 2, 4, 128, 128),        # starts around a 64-token edge, one empty
+])
+def test_layer_backward_at_conv_edges(lens, Hk, Hv, dk, dv):
+    layer.say(f"layer bwd edges lens={lens}")
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    dims = dict(Hk=Hk, dk=dk, Hv=Hv, dv=dv)
+    d = layer.make(7200 + len(lens), 1, int(cu[-1]), Hk, Hv, dk, dv, N=len(lens))
+    layer.check(layer.run_gpu(d, dims, cu=cu), layer.run_ref(d, dims, cu=cu))
+
+
+@pytest.mark.parametrize("B,T", [(3, 16), (2, 19), (5, 1)])
+def test_layer_backward_of_batch_rows_at_conv_edges(B, T):
+    layer.say(f"layer bwd edges B={B} T={T}")
+    dims = dict(Hk=1, dk=64, Hv=2, dv=64)
+    d = layer.make(7300 + T, B, T, 1, 2, 64, 64)
+    layer.check(layer.run_gpu(d, dims), layer.run_ref(d, dims))
