@@ -6,7 +6,7 @@
 // HBM (64 MiB at C1) for a few MFLOP of work, twice.  This kernel reads each hidden row
 // once and forms both outputs from it: a memory-bound skinny product.
 //
-// Work mapping: one workgroup per 64 token rows, wavefront w owning rows 16 (w % 4) ..
+// Work mapping (many rows; few rows: ab_proj_small_kernel): one workgroup per 64 token rows, wavefront w owning rows 16 (w % 4) ..
 // +15 of contraction part w / 4 (one or two parts, the partial sums added at the end);
 // each part runs its chunks of KC.  A chunk's weight rows (both matrices, 2 x 16 NT rows,
 // rows past Hv zero) are staged once per part in LDS (rows padded by 16 bytes, so the 16
@@ -181,14 +181,87 @@ __global__ __launch_bounds__(256 * KS) void ab_proj_kernel(const bf16_t* __restr
   }
 }
 
+// Few rows: one workgroup of eight wavefronts per (16 rows, 16 output columns of one
+// matrix), the contraction dealt over the wavefronts in 64-wide steps and their partial sums
+// added through LDS in order.  A decode step's rows are one workgroup of ab_proj_kernel,
+// which walks the whole contraction behind one chunk's latency after the other: latency
+// bounds it, so here every load of up to four steps is in flight at once and the columns run
+// side by side (each rereads its rows, from L2).  D=2048, Hv=32:
+// 17 rows 12.7 -> 5.6 us (launch included), 1,024 rows 15.4 -> 5.9 us.
+constexpr int kSmallWaves = 8, kSmallSteps = 4;
+
+__global__ __launch_bounds__(64 * kSmallWaves) void ab_proj_small_kernel(const bf16_t* __restrict__ x,
+                                                                        const bf16_t* __restrict__ wa,
+                                                                        const bf16_t* __restrict__ wb,
+                                                                        bf16_t* __restrict__ a,
+                                                                        bf16_t* __restrict__ b, long long M,
+                                                                        int D, int Hv, bool vec_out) {
+  __shared__ f32x4 sum[kSmallWaves][64];
+  const int l = threadIdx.x & 63, lq = l >> 4, lr = l & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int T = (Hv + 15) / 16;  // column tiles per matrix
+  const int ct = blockIdx.x % (2 * T), m = ct / T, t = ct % T;
+  const long long row = (long long)(blockIdx.x / (2 * T)) * 16 + lr;
+  // rows past M and columns past Hv load the last one, in bounds, and are not stored
+  const bf16_t* xr = x + (row < M ? row : M - 1) * D;
+  const int h = 16 * t + lr < Hv ? 16 * t + lr : Hv - 1;
+  const bf16_t* wr = (m == 0 ? wa : wb) + (long long)h * D;
+  const u32x4 z4 = {0u, 0u, 0u, 0u};
+  f32x4 acc = zero4();
+  for (int k0 = 64 * wave; k0 < D; k0 += 64 * kSmallWaves * kSmallSteps) {
+    u32x4 xv[2 * kSmallSteps], wv[2 * kSmallSteps];
+#pragma unroll
+    for (int j = 0; j < 2 * kSmallSteps; ++j) {
+      const int k = k0 + 64 * kSmallWaves * (j >> 1) + 16 * lq + 8 * (j & 1);
+      const int kc = k < D ? k : 0;  // past D: element 0, and zeros in x
+      xv[j] = *(const u32x4*)(xr + kc);
+      wv[j] = *(const u32x4*)(wr + kc);
+    }
+#pragma unroll
+    for (int j = 0; j < 2 * kSmallSteps; ++j) {
+      const int k = k0 + 64 * kSmallWaves * (j >> 1) + 16 * lq + 8 * (j & 1);
+      acc = mma16(wv[j], k < D ? xv[j] : z4, acc);
+    }
+  }
+  sum[wave][l] = acc;
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int w = 1; w < kSmallWaves; ++w) acc += sum[w][l];
+  if (row >= M) return;
+  bf16_t* out = (m == 0 ? a : b) + row * Hv;
+  const int cc = 16 * t + 4 * lq;
+  if (vec_out) {
+    if (cc < Hv) *(uint2*)(out + cc) = make_uint2(pack_bf16(acc[0], acc[1]), pack_bf16(acc[2], acc[3]));
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (cc + v < Hv) out[cc + v] = f2bf(acc[v]);
+  }
+}
+
+// whether both outputs take one 8-byte store per lane
+bool vector_out(const void* a, const void* b, int Hv) {
+  return Hv % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 8 == 0 && reinterpret_cast<uintptr_t>(b) % 8 == 0;
+}
+
+long long small_blocks(long long M, int Hv) { return (M + 15) / 16 * 2 * ((Hv + 15) / 16); }
+
+hipError_t launch_small(const void* x, const void* wa, const void* wb, void* a, void* b, long long M,
+                        int D, int Hv, hipStream_t stream) {
+  hipLaunchKernelGGL(ab_proj_small_kernel, dim3((unsigned)small_blocks(M, Hv)), dim3(64 * kSmallWaves), 0, stream,
+                     (const bf16_t*)x, (const bf16_t*)wa, (const bf16_t*)wb, (bf16_t*)a, (bf16_t*)b, M, D, Hv,
+                     vector_out(a, b, Hv));
+  return hipGetLastError();
+}
+
 template <int NT>
 hipError_t launch_nt(const void* x, const void* wa, const void* wb, void* a, void* b, long long M,
                      int D, int Hv, hipStream_t stream) {
   constexpr int KS = proj_split<NT>();
   const long long blocks = (M + kProjRows - 1) / kProjRows;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  const bool vec_out = Hv % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 8 == 0 &&
-                       reinterpret_cast<uintptr_t>(b) % 8 == 0;
+  const bool vec_out = vector_out(a, b, Hv);
   hipLaunchKernelGGL((ab_proj_kernel<NT, KS>), dim3((unsigned)blocks), dim3(256 * KS), 0, stream,
                      (const bf16_t*)x, (const bf16_t*)wa, (const bf16_t*)wb, (bf16_t*)a,
                      (bf16_t*)b, M, D, Hv, vec_out);
@@ -197,12 +270,20 @@ hipError_t launch_nt(const void* x, const void* wa, const void* wb, void* a, voi
 
 }  // namespace
 
+// The small kernel runs while its grid is at most one workgroup per CU: up to there it is
+// always the faster one (the most rows it takes, D=2048: Hv=8, 2,048 rows, 5.3 against
+// 11.7 us; Hv=32, 1,024 rows, 5.9 against 15.4 us; Hv=64, 512 rows, 5.9 against 21.5 us);
+// with twice the rows it ties (D=1024, Hv=32: 9.4 against 9.0 us), since each column tile
+// rereads the rows.
+constexpr long long kSmallBlocks = 256;
+
 int ab_proj_max_heads() { return 128; }
 
 hipError_t launch_ab_proj(const void* x, const void* wa, const void* wb, void* a, void* b,
                           long long M, int D, int Hv, hipStream_t stream) {
   if (M == 0) return hipSuccess;
   if (D <= 0 || D % 8 != 0 || Hv < 1 || Hv > 128) return hipErrorInvalidValue;
+  if (small_blocks(M, Hv) <= kSmallBlocks) return launch_small(x, wa, wb, a, b, M, D, Hv, stream);
   if (Hv <= 16) return launch_nt<1>(x, wa, wb, a, b, M, D, Hv, stream);
   if (Hv <= 32) return launch_nt<2>(x, wa, wb, a, b, M, D, Hv, stream);
   if (Hv <= 64) return launch_nt<4>(x, wa, wb, a, b, M, D, Hv, stream);

@@ -131,3 +131,11 @@ def test_layer_projections_outside_the_kernel_limits_use_library_gemms():
         _, _, a, b = _projections(params, cfg, x)
         torch.cuda.synchronize()
         assert torch.equal(a, F.linear(x, wa)) and torch.equal(b, F.linear(x, wb))
+
+
+@pytest.mark.parametrize("M,D,Hv", [(1, 8, 1), (15, 72, 16), (16, 2048, 32), (17, 1032, 17),
+                                    (33, 520, 128), (2048, 64, 16), (2049, 64, 16)])
+def test_ab_projections_of_few_rows(M, D, Hv):
+    """The few-row kernel's edges: rows and columns past a tile, a contraction shorter than its
+    eight wavefronts' first step and one ending inside a step, and its largest row count."""
+    test_ab_projections_match_fp64_and_library_gemms(M, D, Hv)
