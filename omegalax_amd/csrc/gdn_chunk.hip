@@ -66,13 +66,14 @@ struct Cfg {
   static constexpr int RAWW = IS ? 2 : 1;       // u32x4 words per 8-element input segment
   static constexpr int LDK = DK + 8;            // row stride of [token][dk] arrays
   static constexpr int SEGS = DK / 8;           // 8-element segments per q/k row
-  static constexpr int NI_KQ = 2 * C * SEGS / NT;
-  static constexpr int NI_V = C * (BV / 8) / NT;
+  static constexpr int NST = 256;               // threads that stage rows through registers
+  static constexpr int NI_KQ = 2 * C * SEGS / NST;
+  static constexpr int NI_V = C * (BV / 8) / NST;
   static constexpr int REC = rec_bytes(MODE, BWD_);
   static constexpr int NREC16 = REC / 16;
   // 16-byte pieces read per chunk: a backward scan that forms no o skips P's lo parts
   static constexpr int NREC16_NO_O = rec_bytes(MODE) / 16;
-  static constexpr int NI_R = (NREC16 + NT - 1) / NT;
+  static constexpr int NI_R = (NREC16 + NST - 1) / NST;
   // bf16 rows with dk = 128 are loaded straight from global memory into one of two
   // LDS buffers (no register staging): unpadded rows with XOR-swizzled 16-byte
   // segments.  fp32 inputs (split on staging) and dk = 64 stage through registers
@@ -91,19 +92,28 @@ struct Cfg {
   // C4 2.663-2.666 -> 2.605-2.639 ms), one elsewhere.  In the forward scan's 64-column
   // workgroups the second loader measured slower (C1 core call 0.311-0.319 against
   // 0.292-0.297 ms).
-  static constexpr int NL = DIRECT ? (MODE == MODE_BF16 && (BWD_ || NWC_ < 4) ? 2 : 1) : 0;
-  static constexpr int NTH = DIRECT ? NT + 64 * (NL + NH) : NT;
-  static constexpr int WPE = (NTH / 64 + 3) / 4;
-  static constexpr int NBUF = DIRECT ? 2 : 1;
   static constexpr int SZK = DIRECT ? C * DK : NS * C * LDK;  // elements of a K or Q buffer
   static constexpr int SZV = DIRECT ? C * BV : NS * C * LDT;  // elements of a V buffer
-  static constexpr int TOTAL = NBUF * (2 * SZK * 2 + SZV * 2 + REC);
+  static constexpr int BUF = 2 * SZK * 2 + SZV * 2 + REC;     // bytes of one set of buffers
+  // Register staging: where two sets of buffers fit (dk <= 64), four loader wavefronts hold
+  // the chunk after next in registers and store the next chunk into the free set, while the
+  // compute wavefronts work on the other: one barrier per chunk, and neither the rows' waits
+  // nor their conversion (fp32 rows are split on staging) sit on the state's chain.  Otherwise
+  // (fp32 inputs at dk = 128) the compute wavefronts stage the rows themselves, between two
+  // barriers.  fp32 inputs at d = 64 (B=2, T=512, H=4):
+  // the scan 30.1 -> 23.6 us; layer rows at d = 64 (B=4, T=500, Hv=16): 22.1 -> 18.0 us.
+  static constexpr bool LSTAGE = !DIRECT && 2 * BUF <= 160 * 1024;
+  static constexpr int NL = DIRECT ? (MODE == MODE_BF16 && (BWD_ || NWC_ < 4) ? 2 : 1) : (LSTAGE ? NST / 64 : 0);
+  static constexpr int NTH = NT + 64 * (NL + NH);
+  static constexpr int WPE = (NTH / 64 + 3) / 4;
+  static constexpr int NBUF = DIRECT || LSTAGE ? 2 : 1;
+  static constexpr int TOTAL = NBUF * BUF;
   static_assert(TOTAL <= 160 * 1024, "LDS budget");
   static_assert(!DIRECT || REC % 1024 == 0, "direct loads move the record in 1 KiB pieces");
   static_assert(DK % 32 == 0 && DK <= 128, "dk");
   static_assert(DIRECT || NWC == 4, "register staging runs four column wavefronts");
-  static_assert(NI_KQ * NT == 2 * C * SEGS && (C * SEGS) % NT == 0, "item split");
-  static_assert(NI_V * NT == C * (BV / 8), "item split");
+  static_assert(DIRECT || (NI_KQ * NST == 2 * C * SEGS && (C * SEGS) % NST == 0), "item split");
+  static_assert(DIRECT || NI_V * NST == C * (BV / 8), "item split");
   static_assert(!VCONV || DIRECT, "the helper wavefronts run beside the direct loads");
   static_assert(!VCONV || (BV / 8) * (C / (BV / 16)) == 64 * NH, "one V task per helper lane");
 };
@@ -124,12 +134,11 @@ struct Prefetch {
 template <int DK, int MODE, bool BWD>
 __device__ __forceinline__ void prefetch(const ChunkParams& p, Prefetch<DK, MODE, BWD>& pf,
                                          long long t0, int nvalid, const unsigned char* rec,
-                                         int hk, int h, int col0) {
+                                         int hk, int h, int col0, const int tid) {
   using Q_ = Cfg<DK, MODE, 4, BWD>;
-  constexpr int NT = Q_::NT, BV = Q_::BV;
+  constexpr int NT = Q_::NST, BV = Q_::BV;
   constexpr bool F32 = MODE == MODE_F32;
   using In = typename std::conditional<F32, float, bf16_t>::type;
-  const int tid = threadIdx.x;
   const int nrec16 = BWD && !p.o ? Q_::NREC16_NO_O : Q_::NREC16;
 #pragma unroll
   for (int k = 0; k < Q_::NI_R; ++k) {
@@ -157,6 +166,65 @@ __device__ __forceinline__ void prefetch(const ChunkParams& p, Prefetch<DK, MODE
     const unsigned rr = full ? r : (r < nvalid ? r : nvalid - 1);
     if (which == 0) load_raw<F32>(kb, rr * ksl + seg * 8u, pf.kq[k]);
     else load_raw<F32>(qb, rr * qsl + seg * 8u, pf.kq[k]);
+  }
+}
+
+// A prefetched chunk's rows and record into the LDS buffers, by thread tid of NST.
+template <int DK, int MODE, bool BWD>
+__device__ __forceinline__ void stage(const ChunkParams& p, const Prefetch<DK, MODE, BWD>& pf, int nvalid,
+                                      bf16_t* sK, bf16_t* sQ, bf16_t* sV, unsigned char* sRec, const int tid) {
+  using Q_ = Cfg<DK, MODE, 4, BWD>;
+  constexpr int NT = Q_::NST, BV = Q_::BV, LDK = Q_::LDK, SEGS = Q_::SEGS;
+  constexpr bool F32 = MODE == MODE_F32;
+  constexpr int K_LO = C * LDK, V_LO = C * LDT;
+  const bool full = nvalid == C;  // uniform: only a sequence's last chunk has padded rows
+#pragma unroll
+  for (int k = 0; k < Q_::NI_KQ; ++k) {
+    constexpr int PER = C * SEGS;
+    const int which = (k * NT) / PER;
+    const int rem2 = (k * NT) % PER + tid;
+    const int r = rem2 / SEGS, seg = rem2 % SEGS;
+    bf16_t* dst = (which == 0 ? sK : sQ) + r * LDK + seg * 8;
+    if constexpr (F32) {
+      float x[8];
+      unpack8<true>(pf.kq[k], x);
+      const float keep = (float)(r < nvalid);  // padded rows are zero
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] *= keep;
+      *(u32x4*)dst = pack8(x);
+      *(u32x4*)(dst + K_LO) = pack8_lo(x);
+    } else if (full) {
+      *(u32x4*)dst = pf.kq[k][0];
+    } else {
+      const unsigned keep = r < nvalid ? 0xffffffffu : 0u;  // padded rows are zero
+      *(u32x4*)dst = pf.kq[k][0] & keep;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < Q_::NI_V; ++k) {
+    const int it = tid + k * NT;
+    const int r = it / (BV / 8), seg = it % (BV / 8);
+    bf16_t* dst = sV + r * LDT + seg * 8;
+    if constexpr (F32) {
+      float x[8];
+      unpack8<true>(pf.v[k], x);
+      const float keep = (float)(r < nvalid);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] *= keep;
+      *(u32x4*)dst = pack8(x);
+      *(u32x4*)(dst + V_LO) = pack8_lo(x);
+    } else if (full) {
+      *(u32x4*)dst = pf.v[k][0];
+    } else {
+      const unsigned keep = r < nvalid ? 0xffffffffu : 0u;
+      *(u32x4*)dst = pf.v[k][0] & keep;
+    }
+  }
+  const int nrec16 = BWD && !p.o ? Q_::NREC16_NO_O : Q_::NREC16;
+#pragma unroll
+  for (int k = 0; k < Q_::NI_R; ++k) {
+    const int it = tid + k * NT;
+    if (it < nrec16) ((u32x4*)sRec)[it] = pf.rec[k];
   }
 }
 
@@ -421,9 +489,8 @@ template <int DK, int MODE, bool BWD = false, int NWC_ = 4, bool FUSE = false>
 __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amdgpu_waves_per_eu(Cfg<DK, MODE, NWC_, BWD>::WPE, Cfg<DK, MODE, NWC_, BWD>::WPE))) void scan_kernel(ChunkParams p) {
   using Q_ = Cfg<DK, MODE, NWC_, BWD>;
   constexpr int NWC = Q_::NWC, BV = Q_::BV, NT = Q_::NT;
-  constexpr int LDK = Q_::LDK, SEGS = Q_::SEGS;
+  constexpr int LDK = Q_::LDK;
   constexpr bool IS = Q_::IS, OS = Q_::OS;
-  constexpr bool F32 = MODE == MODE_F32;
   // Each buffer is its own __shared__ object, so the compiler can tell their
   // accesses apart and overlap loads of one with stores to another.
   constexpr bool DIRECT = Q_::DIRECT;
@@ -431,10 +498,11 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
   // below is unrolled by two so that every access names its buffer statically: the
   // compiler can then tell that the next chunk's loads into one buffer do not touch
   // the other, and does not wait for them before this chunk's LDS reads.
-  __shared__ __align__(16) bf16_t sK0[Q_::SZK], sK1[DIRECT ? Q_::SZK : 8];
-  __shared__ __align__(16) bf16_t sQ0[Q_::SZK], sQ1[DIRECT ? Q_::SZK : 8];
-  __shared__ __align__(16) bf16_t sV0[Q_::SZV], sV1[DIRECT ? Q_::SZV : 8];
-  __shared__ __align__(16) unsigned char sRec0[Q_::REC], sRec1[DIRECT ? Q_::REC : 16];
+  constexpr bool LSTAGE = Q_::LSTAGE, TWO = Q_::NBUF == 2;
+  __shared__ __align__(16) bf16_t sK0[Q_::SZK], sK1[TWO ? Q_::SZK : 8];
+  __shared__ __align__(16) bf16_t sQ0[Q_::SZK], sQ1[TWO ? Q_::SZK : 8];
+  __shared__ __align__(16) bf16_t sV0[Q_::SZV], sV1[TWO ? Q_::SZV : 8];
+  __shared__ __align__(16) unsigned char sRec0[Q_::REC], sRec1[TWO ? Q_::REC : 16];
   // (layer, direct loads) the compute wavefronts' row sums of o^2, by chunk parity: chunk
   // j's are written after the barrier that opens chunk j + 1 (so no wavefront waits for
   // the write before a barrier); the loader adds them up after the barrier of chunk j + 2
@@ -451,7 +519,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
 
   const int tid = threadIdx.x, l = tid & 63, lq = l >> 4, lr = l & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool loader = DIRECT && wave >= NWC && wave < NWC + Q_::NL;  // loads, computes nothing
+  const bool loader = wave >= NWC && wave < NWC + Q_::NL;  // loads, computes nothing
   const bool helper = Q_::VCONV && wave >= NWC + Q_::NL;  // forms the V rows (layer, direct loads)
   const bool compute = wave < NWC;             // owns 16 state columns
   // XCD-aware work item (scan_item): a key head's workgroups share one XCD's L2, and
@@ -506,8 +574,8 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
                             (lds_bf16*)sV0, (lds_u8*)sRec0);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): landed before the first barrier
       }
-    } else {
-      prefetch<DK, MODE, BWD>(p, pf, s0, nv0, rec_of(0), hk, h, col0);
+    } else if constexpr (!LSTAGE) {
+      prefetch<DK, MODE, BWD>(p, pf, s0, nv0, rec_of(0), hk, h, col0, tid);
     }
   }
 
@@ -576,66 +644,21 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
       }
       // (FUSE) z of the chunk normalised at the end of this step, in flight meanwhile
       if constexpr (FUSE) z_load(j - kFin);
+    } else if constexpr (LSTAGE) {
+      // the loaders have stored chunk j, and chunk j-1, the last reader of the other set,
+      // is finished everywhere
+      lds_barrier();
     } else {
     __syncthreads();  // the previous chunk's readers are done with the shared arrays
 
-    // ------------------------------------------------------------ stage the chunk
-    const bool full = nvalid == C;  // uniform: only a sequence's last chunk has padded rows
-#pragma unroll
-    for (int k = 0; k < Q_::NI_KQ; ++k) {
-      constexpr int PER = C * SEGS;
-      const int which = (k * NT) / PER;
-      const int rem2 = (k * NT) % PER + tid;
-      const int r = rem2 / SEGS, seg = rem2 % SEGS;
-      bf16_t* dst = (which == 0 ? sK : sQ) + r * LDK + seg * 8;
-      if constexpr (F32) {
-        float x[8];
-        unpack8<true>(pf.kq[k], x);
-        const float keep = (float)(r < nvalid);  // padded rows are zero
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] *= keep;
-        *(u32x4*)dst = pack8(x);
-        *(u32x4*)(dst + K_LO) = pack8_lo(x);
-      } else if (full) {
-        *(u32x4*)dst = pf.kq[k][0];
-      } else {
-        const unsigned keep = r < nvalid ? 0xffffffffu : 0u;  // padded rows are zero
-        *(u32x4*)dst = pf.kq[k][0] & keep;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < Q_::NI_V; ++k) {
-      const int it = tid + k * NT;
-      const int r = it / (BV / 8), seg = it % (BV / 8);
-      bf16_t* dst = sV + r * LDT + seg * 8;
-      if constexpr (F32) {
-        float x[8];
-        unpack8<true>(pf.v[k], x);
-        const float keep = (float)(r < nvalid);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] *= keep;
-        *(u32x4*)dst = pack8(x);
-        *(u32x4*)(dst + V_LO) = pack8_lo(x);
-      } else if (full) {
-        *(u32x4*)dst = pf.v[k][0];
-      } else {
-        const unsigned keep = r < nvalid ? 0xffffffffu : 0u;
-        *(u32x4*)dst = pf.v[k][0] & keep;
-      }
-    }
-    const int nrec16 = BWD && !p.o ? Q_::NREC16_NO_O : Q_::NREC16;
-#pragma unroll
-    for (int k = 0; k < Q_::NI_R; ++k) {
-      const int it = tid + k * NT;
-      if (it < nrec16) ((u32x4*)sRec)[it] = pf.rec[k];
-    }
+    stage<DK, MODE, BWD>(p, pf, nvalid, sK, sQ, sV, sRec, tid);
     __syncthreads();
 
     // issue the next chunk's loads; they land during the rest of this chunk
     if (j + 1 < nchunks) {
       const long long tn = t0 + C;
       prefetch<DK, MODE, BWD>(p, pf, tn, (int)((s1 - tn) < C ? (s1 - tn) : C), rec_of(j + 1), hk, h,
-                         col0);
+                         col0, tid);
     }
     }
 
@@ -1201,6 +1224,40 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
           sSS[(nchunks - 1) & 1][wave][16 * lq + lr] = ss_prev;
           lds_barrier();
         }
+      }
+    }
+  } else if constexpr (LSTAGE) {
+    if (loader) {
+      // chunk j's rows are loaded two steps before the step that reads them and stored one
+      // before it, into the set that chunk j - 2 has left; one barrier per chunk
+      const int st = tid - NT;
+      auto rows = [&](int c, long long& tc) {
+        tc = s0 + (long long)c * C;
+        return (int)((s1 - tc) < C ? (s1 - tc) : C);
+      };
+      long long tc;
+      auto load = [&](int c) {
+        const int nvc = rows(c, tc);
+        prefetch<DK, MODE, BWD>(p, pf, tc, nvc, rec_of(c), hk, h, col0, st);
+      };
+      if (nchunks > 0) {
+        load(0);
+        stage<DK, MODE, BWD>(p, pf, rows(0, tc), sK0, sQ0, sV0, sRec0, st);
+        if (nchunks > 1) load(1);
+      }
+      auto step = [&](int j, bf16_t* nK, bf16_t* nQ, bf16_t* nV, unsigned char* nRec) {
+        lds_barrier();
+        if (j + 1 < nchunks) stage<DK, MODE, BWD>(p, pf, rows(j + 1, tc), nK, nQ, nV, nRec, st);
+        if (j + 2 < nchunks) load(j + 2);
+      };
+      for (int j = 0; j < nchunks; j += 2) {
+        step(j, sK1, sQ1, sV1, sRec1);
+        if (j + 1 < nchunks) step(j + 1, sK0, sQ0, sV0, sRec0);
+      }
+    } else {
+      for (int j = 0; j < nchunks; j += 2) {
+        run_chunk(j, sK0, sQ0, sV0, sRec0);
+        if (j + 1 < nchunks) run_chunk(j + 1, sK1, sQ1, sV1, sRec1);
       }
     }
   } else {
