@@ -319,8 +319,13 @@ __device__ __forceinline__ constexpr int ptile_index(int mb, int nb) { return mb
 // staged, the other buffer is free), one publishes the P tiles.  fp32 K and Q rows leave
 // no room for a second buffer, so with fp32 inputs the compute wavefronts stage the rows
 // themselves from a register prefetch two chunks deep.
-template <int DK, bool F32>
-__global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
+//
+// NWC compute wavefronts of 16 columns each (as the forward scan's workgroups: four, or two
+// or one where 64-column workgroups would leave CUs idle; fp32 inputs take four).
+template <int DK, bool F32, int NWC>
+__global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdParams p) {
+  static_assert(!F32 || NWC == 4, "fp32 inputs: the four compute wavefronts stage the rows");
+  constexpr int BV = 16 * NWC;  // columns of dv per workgroup
   using KT = typename std::conditional<F32, float, bf16_t>::type;
   constexpr int LDK = DK + (F32 ? 4 : 8);
   constexpr int LDB = C + 8;  // stride (bf16) of a split plane
@@ -331,7 +336,7 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
   // loaders' writes to one from the compute wavefronts' reads of the other.
   __shared__ __align__(16) KT sK0[C * LDK], sK1[LDR ? C * LDK : 8];
   __shared__ __align__(16) KT sQ0[C * LDK], sQ1[LDR ? C * LDK : 8];
-  // dO (this block's 64 columns), X (fp32 inputs: X^T) and (fp32 inputs) P, row-major, as
+  // dO (this block's columns), X (fp32 inputs: X^T) and (fp32 inputs) P, row-major, as
   // bf16 hi / lo planes
   __shared__ __align__(16) bf16_t sDO0[2 * C * LDB], sDO1[LDR ? 2 * C * LDB : 8];
   __shared__ __align__(16) bf16_t sX0[2 * C * LDB], sX1[LDR ? 2 * C * LDB : 8];
@@ -356,12 +361,12 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
 
   const int tid = threadIdx.x, l = tid & 63, lq = l >> 4, lr = l & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool loader = LDR && wave >= NT / 64;  // (LDR) waves 4-7: rows and P tiles only
-  const int st = loader ? tid - NT : tid;       // index among the threads that stage rows
+  const bool loader = LDR && wave >= NWC;      // (LDR) the last four: rows and P tiles only
+  const int st = loader ? tid - 64 * NWC : tid;  // index among the NT threads that stage rows
   const ScanItem item = scan_item(p.seq_order, p.N, p.Hk, p.Hv, p.nb);
   const int blk = item.blk, h = item.h, n = item.n;
   const int gqa = p.Hv / p.Hk, hk = h / gqa;
-  const int DV = p.DV, col0 = 64 * blk, c = 16 * wave;
+  const int DV = p.DV, col0 = BV * blk, c = 16 * wave;
   long long s0, s1;
   seq_range(p.cu_seqlens, n, p.T, s0, s1);
   const int nchunks = (int)((s1 - s0 + C - 1) / C);
@@ -405,7 +410,7 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
   static_assert(NXP * NT == 2 * kNPairs * 64, "record pieces");
   struct Pf {
     typename Vec4<KT>::type pkq[NKQ];
-    float4 pdo[C * 16 / NT], pxp[PREC ? 1 : 2 * C * 16 / NT];
+    float4 pdo[C * BV / 4 / NT], pxp[PREC ? 1 : 2 * C * 16 / NT];
     u32x4 px[PREC ? NXP : 1];
     float pgate, pg;
   };
@@ -432,9 +437,9 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
       f.pkq[m] = bload4(which ? qr : kr, (unsigned)((row * ld + c4) * (long long)sizeof(KT)), (const KT*)nullptr);
     }
 #pragma unroll
-    for (int m = 0; m < C * 16 / NT; ++m) {
+    for (int m = 0; m < C * BV / 4 / NT; ++m) {
       const int it = st + m * NT;
-      const int row = it >> 4, c4 = 4 * (it & 15);
+      const int row = it / (BV / 4), c4 = 4 * (it % (BV / 4));
       f.pdo[m] = bload4(dr, (unsigned)(4 * (row * rs + c4)), (const float*)nullptr);
     }
     const float* xb = p.xlpg + ((size_t)sl * p.Hv + h) * xlpg_floats(F32);
@@ -466,9 +471,9 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
       store4((which ? bf.Q : bf.K) + row * LDK + c4, f.pkq[m]);
     }
 #pragma unroll
-    for (int m = 0; m < C * 16 / NT; ++m) {
+    for (int m = 0; m < C * BV / 4 / NT; ++m) {
       const int it = st + m * NT;
-      put_row4(sDOh, sDOl, (it >> 4) * LDB + 4 * (it & 15), f32x4{f.pdo[m].x, f.pdo[m].y, f.pdo[m].z, f.pdo[m].w});
+      put_row4(sDOh, sDOl, (it / (BV / 4)) * LDB + 4 * (it % (BV / 4)), f32x4{f.pdo[m].x, f.pdo[m].y, f.pdo[m].z, f.pdo[m].w});
     }
     if constexpr (PREC) {
       // piece 2x + part of the record's T part: lane (q, r) of pair x = (ib, jp) holds
@@ -515,7 +520,7 @@ __global__ __launch_bounds__(F32 ? NT : 2 * NT) void rscan_kernel(BwdParams p) {
   };
   // (LDR) the ten tiles, dealt over the four loaders (t = lw, lw + 4, lw + 8), into sPT
   auto form_ptiles = [&](const Buf& bf) {
-    const int lw = wave - NT / 64;
+    const int lw = wave - NWC;
     for (int t = lw; t < 10; t += 4) {  // uniform per wavefront
       const int mb = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3;
       const int nb = t - mb * (mb + 1) / 2;
@@ -1293,11 +1298,27 @@ __global__ __launch_bounds__(NT) void qk_final_kernel(BwdParams p, long long row
   }
 }
 
+// p.nb (64-column blocks) is replaced by the scan's own count in a copy of the parameters
+template <int DK, bool F32, int NWC>
+hipError_t launch_rscan(const BwdParams& p, hipStream_t stream) {
+  BwdParams q = p;
+  q.nb = p.DV / (16 * NWC);
+  hipLaunchKernelGGL((rscan_kernel<DK, F32, NWC>), dim3((unsigned)(q.N * q.Hv * q.nb)),
+                     dim3(F32 ? NT : 64 * NWC + NT), 0, stream, q);
+  return hipGetLastError();
+}
+
 template <int DK, bool F32>
 hipError_t launch_bwd_dk(const BwdParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL((rscan_kernel<DK, F32>), dim3((unsigned)(p.N * p.Hv * p.nb)), dim3(F32 ? NT : 2 * NT), 0,
-                     stream, p);
-  hipError_t e = hipGetLastError();
+  hipError_t e;
+  if constexpr (F32) {
+    e = launch_rscan<DK, F32, 4>(p, stream);
+  } else {
+    const int tiles = scan_column_tiles(p.N, p.Hv, p.DV);
+    e = tiles == 1   ? launch_rscan<DK, F32, 1>(p, stream)
+        : tiles == 2 ? launch_rscan<DK, F32, 2>(p, stream)
+                     : launch_rscan<DK, F32, 4>(p, stream);
+  }
   if (e != hipSuccess) return e;
   const unsigned grid = (unsigned)((long long)p.n_rec * p.Hv);
   if (grid > 0) {

@@ -52,9 +52,9 @@ constexpr int C = kC;
 constexpr int LDT = kLDT;
 constexpr int kBlockCols = 64;  // dv columns per block of the other kernels (nb = dv / 64)
 
-// NWC_: 16-column state tiles (compute wavefronts) per workgroup.  Four on every path;
-// the direct-load path also runs with two or one, so that sequences x heads x dv / 16 tiles
-// fill the chip when 64-column workgroups would leave CUs idle.
+// NWC_: 16-column state tiles (compute wavefronts) per workgroup: four, or two or one, so
+// that sequences x heads x dv / 16 tiles fill the chip when 64-column workgroups would leave
+// CUs idle (where loader wavefronts stage the rows; see scan_column_tiles).
 template <int DK, int MODE, int NWC_ = 4, bool BWD_ = false>
 struct Cfg {
   static constexpr int NWC = NWC_;
@@ -68,7 +68,8 @@ struct Cfg {
   static constexpr int SEGS = DK / 8;           // 8-element segments per q/k row
   static constexpr int NST = 256;               // threads that stage rows through registers
   static constexpr int NI_KQ = 2 * C * SEGS / NST;
-  static constexpr int NI_V = C * (BV / 8) / NST;
+  static constexpr int VITEMS = C * (BV / 8);   // 8-element items of a V chunk
+  static constexpr int NI_V = (VITEMS + NST - 1) / NST;
   static constexpr int REC = rec_bytes(MODE, BWD_);
   static constexpr int NREC16 = REC / 16;
   // 16-byte pieces read per chunk: a backward scan that forms no o skips P's lo parts
@@ -111,17 +112,17 @@ struct Cfg {
   static_assert(TOTAL <= 160 * 1024, "LDS budget");
   static_assert(!DIRECT || REC % 1024 == 0, "direct loads move the record in 1 KiB pieces");
   static_assert(DK % 32 == 0 && DK <= 128, "dk");
-  static_assert(DIRECT || NWC == 4, "register staging runs four column wavefronts");
+  static_assert(DIRECT || LSTAGE || NWC == 4, "staging by the compute wavefronts takes four");
   static_assert(DIRECT || (NI_KQ * NST == 2 * C * SEGS && (C * SEGS) % NST == 0), "item split");
-  static_assert(DIRECT || NI_V * NST == C * (BV / 8), "item split");
+  static_assert(VITEMS % 64 == 0, "whole wavefronts of V items");
   static_assert(!VCONV || DIRECT, "the helper wavefronts run beside the direct loads");
   static_assert(!VCONV || (BV / 8) * (C / (BV / 16)) == 64 * NH, "one V task per helper lane");
 };
 
 // Per-thread register prefetch of one chunk's inputs.
-template <int DK, int MODE, bool BWD>
+template <int DK, int MODE, int NWC, bool BWD>
 struct Prefetch {
-  using Q_ = Cfg<DK, MODE, 4, BWD>;
+  using Q_ = Cfg<DK, MODE, NWC, BWD>;
   u32x4 kq[Q_::NI_KQ][Q_::RAWW];
   u32x4 v[Q_::NI_V][Q_::RAWW];
   u32x4 rec[Q_::NI_R];
@@ -131,11 +132,11 @@ struct Prefetch {
 // chunk-uniform base (scalar registers) plus a per-thread 32-bit offset that does not
 // change from chunk to chunk; only a sequence's last, partial chunk clamps its rows
 // (rows past the end load the last valid row, in bounds, and staging zeroes them).
-template <int DK, int MODE, bool BWD>
-__device__ __forceinline__ void prefetch(const ChunkParams& p, Prefetch<DK, MODE, BWD>& pf,
+template <int DK, int MODE, int NWC, bool BWD>
+__device__ __forceinline__ void prefetch(const ChunkParams& p, Prefetch<DK, MODE, NWC, BWD>& pf,
                                          long long t0, int nvalid, const unsigned char* rec,
                                          int hk, int h, int col0, const int tid) {
-  using Q_ = Cfg<DK, MODE, 4, BWD>;
+  using Q_ = Cfg<DK, MODE, NWC, BWD>;
   constexpr int NT = Q_::NST, BV = Q_::BV;
   constexpr bool F32 = MODE == MODE_F32;
   using In = typename std::conditional<F32, float, bf16_t>::type;
@@ -155,7 +156,8 @@ __device__ __forceinline__ void prefetch(const ChunkParams& p, Prefetch<DK, MODE
     const int it = tid + k * NT;
     const int r = it / (BV / 8), seg = it % (BV / 8);
     const unsigned rr = full ? r : (r < nvalid ? r : nvalid - 1);
-    load_raw<F32>(vb, rr * vsl + seg * 8u, pf.v[k]);
+    if (Q_::VITEMS % NT == 0 || it < Q_::VITEMS)  // uniform per wavefront
+      load_raw<F32>(vb, rr * vsl + seg * 8u, pf.v[k]);
   }
 #pragma unroll
   for (int k = 0; k < Q_::NI_KQ; ++k) {
@@ -170,10 +172,10 @@ __device__ __forceinline__ void prefetch(const ChunkParams& p, Prefetch<DK, MODE
 }
 
 // A prefetched chunk's rows and record into the LDS buffers, by thread tid of NST.
-template <int DK, int MODE, bool BWD>
-__device__ __forceinline__ void stage(const ChunkParams& p, const Prefetch<DK, MODE, BWD>& pf, int nvalid,
+template <int DK, int MODE, int NWC, bool BWD>
+__device__ __forceinline__ void stage(const ChunkParams& p, const Prefetch<DK, MODE, NWC, BWD>& pf, int nvalid,
                                       bf16_t* sK, bf16_t* sQ, bf16_t* sV, unsigned char* sRec, const int tid) {
-  using Q_ = Cfg<DK, MODE, 4, BWD>;
+  using Q_ = Cfg<DK, MODE, NWC, BWD>;
   constexpr int NT = Q_::NST, BV = Q_::BV, LDK = Q_::LDK, SEGS = Q_::SEGS;
   constexpr bool F32 = MODE == MODE_F32;
   constexpr int K_LO = C * LDK, V_LO = C * LDT;
@@ -203,6 +205,7 @@ __device__ __forceinline__ void stage(const ChunkParams& p, const Prefetch<DK, M
 #pragma unroll
   for (int k = 0; k < Q_::NI_V; ++k) {
     const int it = tid + k * NT;
+    if (Q_::VITEMS % NT != 0 && it >= Q_::VITEMS) break;  // uniform per wavefront
     const int r = it / (BV / 8), seg = it % (BV / 8);
     bf16_t* dst = sV + r * LDT + seg * 8;
     if constexpr (F32) {
@@ -565,7 +568,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
   const unsigned o_elem = (unsigned)lr * o_rs + 16u * wave + 4u * lq;
   const unsigned o_lane = 4u * o_elem, o_lane_h = 2u * o_elem;  // bytes: fp32 o, bf16 o
 
-  Prefetch<DK, MODE, BWD> pf;
+  Prefetch<DK, MODE, NWC, BWD> pf;
   if (nchunks > 0) {
     const int nv0 = (int)((s1 - s0) < C ? (s1 - s0) : C);
     if constexpr (DIRECT) {
@@ -575,7 +578,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): landed before the first barrier
       }
     } else if constexpr (!LSTAGE) {
-      prefetch<DK, MODE, BWD>(p, pf, s0, nv0, rec_of(0), hk, h, col0, tid);
+      prefetch<DK, MODE, NWC, BWD>(p, pf, s0, nv0, rec_of(0), hk, h, col0, tid);
     }
   }
 
@@ -651,13 +654,13 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
     } else {
     __syncthreads();  // the previous chunk's readers are done with the shared arrays
 
-    stage<DK, MODE, BWD>(p, pf, nvalid, sK, sQ, sV, sRec, tid);
+    stage<DK, MODE, NWC, BWD>(p, pf, nvalid, sK, sQ, sV, sRec, tid);
     __syncthreads();
 
     // issue the next chunk's loads; they land during the rest of this chunk
     if (j + 1 < nchunks) {
       const long long tn = t0 + C;
-      prefetch<DK, MODE, BWD>(p, pf, tn, (int)((s1 - tn) < C ? (s1 - tn) : C), rec_of(j + 1), hk, h,
+      prefetch<DK, MODE, NWC, BWD>(p, pf, tn, (int)((s1 - tn) < C ? (s1 - tn) : C), rec_of(j + 1), hk, h,
                          col0, tid);
     }
     }
@@ -1238,16 +1241,16 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
       long long tc;
       auto load = [&](int c) {
         const int nvc = rows(c, tc);
-        prefetch<DK, MODE, BWD>(p, pf, tc, nvc, rec_of(c), hk, h, col0, st);
+        prefetch<DK, MODE, NWC, BWD>(p, pf, tc, nvc, rec_of(c), hk, h, col0, st);
       };
       if (nchunks > 0) {
         load(0);
-        stage<DK, MODE, BWD>(p, pf, rows(0, tc), sK0, sQ0, sV0, sRec0, st);
+        stage<DK, MODE, NWC, BWD>(p, pf, rows(0, tc), sK0, sQ0, sV0, sRec0, st);
         if (nchunks > 1) load(1);
       }
       auto step = [&](int j, bf16_t* nK, bf16_t* nQ, bf16_t* nV, unsigned char* nRec) {
         lds_barrier();
-        if (j + 1 < nchunks) stage<DK, MODE, BWD>(p, pf, rows(j + 1, tc), nK, nQ, nV, nRec, st);
+        if (j + 1 < nchunks) stage<DK, MODE, NWC, BWD>(p, pf, rows(j + 1, tc), nK, nQ, nV, nRec, st);
         if (j + 2 < nchunks) load(j + 2);
       };
       for (int j = 0; j < nchunks; j += 2) {
@@ -1329,24 +1332,27 @@ int device_cus() {
   return cus[dev];
 }
 
-// Column tiles per workgroup for the direct-load scan: 4 (64 columns) when that gives a
-// workgroup per CU, else 2 or 1, the widest that still does.  The workgroups walk their
-// sequences' chunks in order, so a grid smaller than the chip leaves CUs idle for the
-// whole call; narrower workgroups also leave each CU's LDS to fewer wavefronts.
-int scan_tiles_per_wg(const ChunkParams& p) {
-  const long long tiles = (long long)p.N * p.Hv * (p.DV / 16);
+// Column tiles per workgroup: 4 (64 columns) when that gives a workgroup per CU, else 2 or
+// 1, the widest that still does.  The workgroups walk their sequences' chunks in order, so a
+// grid smaller than the chip leaves CUs idle for the whole call; narrower workgroups also
+// leave each CU's LDS to fewer wavefronts.  Against 64 columns: backward of B=1 T=2,548 Hv=32
+// d=128, recompute scan 112 -> 79 us and reverse scan 166 -> 135 us (256 workgroups of 16
+// columns for 64); fp32 inputs, B=2 T=512 H=4 d=64, 23.7 -> 19.3 us (32 for 8); layer rows,
+// B=8 T=1,000 Hv=16 d=64, 30.7 -> 27.7 us (256 of 32 columns for 128).
+int tiles_per_wg(long long tiles) {
   const long long cus = device_cus();
   if (tiles >= 4 * cus) return 4;
   if (tiles >= 2 * cus) return 2;
   return 1;
 }
+int scan_tiles_per_wg(const ChunkParams& p) { return tiles_per_wg((long long)p.N * p.Hv * (p.DV / 16)); }
 
-template <int DK, int MODE, bool FUSE = false>
-hipError_t launch_scan_direct(const ChunkParams& p, hipStream_t stream) {
+template <int DK, int MODE, bool BWD = false, bool FUSE = false>
+hipError_t launch_scan_tiles(const ChunkParams& p, hipStream_t stream) {
   switch (scan_tiles_per_wg(p)) {
-    case 1: return launch_scan_cfg<DK, MODE, false, 1, FUSE>(p, stream);
-    case 2: return launch_scan_cfg<DK, MODE, false, 2, FUSE>(p, stream);
-    default: return launch_scan_cfg<DK, MODE, false, 4, FUSE>(p, stream);
+    case 1: return launch_scan_cfg<DK, MODE, BWD, 1, FUSE>(p, stream);
+    case 2: return launch_scan_cfg<DK, MODE, BWD, 2, FUSE>(p, stream);
+    default: return launch_scan_cfg<DK, MODE, BWD, 4, FUSE>(p, stream);
   }
 }
 
@@ -1354,8 +1360,10 @@ hipError_t launch_scan_direct(const ChunkParams& p, hipStream_t stream) {
 
 int chunk_block_cols() { return kBlockCols; }
 
+int scan_column_tiles(int N, int Hv, int DV) { return tiles_per_wg((long long)N * Hv * (DV / 16)); }
+
 int layer_scan_blocks(const ChunkParams& p) {
-  return p.dk == 128 ? p.DV / (16 * scan_tiles_per_wg(p)) : p.DV / kBlockCols;
+  return p.DV / (16 * scan_tiles_per_wg(p));
 }
 
 // The layer scan applies the gated norm itself (FUSE) when it loads directly (dk = 128),
@@ -1386,34 +1394,34 @@ bool layer_scan_forms_v(int dk) { return layer_v_in_scan(dk); }
 
 hipError_t launch_scan_bwd(const ChunkParams& p, int mode, hipStream_t stream) {
   if (mode == MODE_F32) {
-    if (p.dk == 64) return launch_scan_cfg<64, MODE_F32, true>(p, stream);
-    if (p.dk == 32) return launch_scan_cfg<32, MODE_F32, true>(p, stream);
+    if (p.dk == 64) return launch_scan_tiles<64, MODE_F32, true>(p, stream);
+    if (p.dk == 32) return launch_scan_tiles<32, MODE_F32, true>(p, stream);
     return hipErrorInvalidValue;
   }
   if (mode == MODE_BF16) {
-    if (p.dk == 128) return launch_scan_cfg<128, MODE_BF16, true>(p, stream);
-    if (p.dk == 64) return launch_scan_cfg<64, MODE_BF16, true>(p, stream);
+    if (p.dk == 128) return launch_scan_tiles<128, MODE_BF16, true>(p, stream);
+    if (p.dk == 64) return launch_scan_tiles<64, MODE_BF16, true>(p, stream);
   }
   return hipErrorInvalidValue;
 }
 
 hipError_t launch_scan(const ChunkParams& p, int mode, hipStream_t stream) {
   if (mode == MODE_F32) {
-    if (p.dk == 64) return launch_scan_cfg<64, MODE_F32>(p, stream);
-    if (p.dk == 32) return launch_scan_cfg<32, MODE_F32>(p, stream);
+    if (p.dk == 64) return launch_scan_tiles<64, MODE_F32>(p, stream);
+    if (p.dk == 32) return launch_scan_tiles<32, MODE_F32>(p, stream);
     if (p.dk == 128) return launch_scan_cfg<128, MODE_F32>(p, stream);
     return hipErrorInvalidValue;
   }
   if (mode == MODE_LAYER) {
     if (p.dk == 128) {
-      if (layer_scan_fuses_norm(p)) return launch_scan_direct<128, MODE_LAYER, true>(p, stream);
-      return launch_scan_direct<128, MODE_LAYER>(p, stream);
+      if (layer_scan_fuses_norm(p)) return launch_scan_tiles<128, MODE_LAYER, false, true>(p, stream);
+      return launch_scan_tiles<128, MODE_LAYER>(p, stream);
     }
-    if (p.dk == 64) return launch_scan_cfg<64, MODE_LAYER>(p, stream);
+    if (p.dk == 64) return launch_scan_tiles<64, MODE_LAYER>(p, stream);
     return hipErrorInvalidValue;
   }
-  if (p.dk == 128) return launch_scan_direct<128, MODE_BF16>(p, stream);
-  if (p.dk == 64) return launch_scan_cfg<64, MODE_BF16>(p, stream);
+  if (p.dk == 128) return launch_scan_tiles<128, MODE_BF16>(p, stream);
+  if (p.dk == 64) return launch_scan_tiles<64, MODE_BF16>(p, stream);
   return hipErrorInvalidValue;
 }
 

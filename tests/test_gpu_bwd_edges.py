@@ -8,6 +8,8 @@ tests/test_gpu_bwd.py and tests/test_gpu_layer_bwd.py, whose inputs these reuse.
 import numpy as np
 import pytest
 
+from oracle import gdn_oracle as O
+
 import test_gpu_bwd as core
 import test_gpu_layer_bwd as layer
 
@@ -58,3 +60,28 @@ def test_layer_backward_of_batch_rows_at_conv_edges(B, T):
     dims = dict(Hk=1, dk=64, Hv=2, dv=64)
     d = layer.make(7300 + T, B, T, 1, 2, 64, 64)
     layer.check(layer.run_gpu(d, dims), layer.run_ref(d, dims))
+
+
+@pytest.mark.parametrize("B,Hk,Hv,dk,dv,dtype", [
+    (1, 2, 4, 64, 64, "f32"), (8, 8, 16, 64, 64, "f32"),      # 16- and 32-column workgroups
+    (8, 8, 16, 64, 64, "bf16"), (8, 16, 32, 64, 64, "bf16"),  # 32- and 64-column
+    (4, 8, 16, 128, 128, "bf16"), (8, 8, 16, 128, 128, "bf16"),
+])
+def test_scans_at_every_workgroup_width(B, Hk, Hv, dk, dv, dtype):
+    """Sequences x value heads x dv / 16 chooses the scans' 16-, 32- or 64-column workgroups;
+    the suite's small shapes all take the narrowest."""
+    from omegalax_amd import chunk_gated_delta_rule
+    core.say(f"scan widths B={B} Hk={Hk} Hv={Hv} dk={dk} dv={dv} {dtype}")
+    T = 150
+    q, k, v, g, beta, S0, do, dht = args = core.make(7400 + B + Hv + dk, B, T, Hk, Hv, dk, dv, dtype)
+    got = core.run_gpu(*args, dtype)
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    o, fs = chunk_gated_delta_rule(core.dev(q, tdt), core.dev(k, tdt), core.dev(v, tdt), core.dev(g),
+                                   core.dev(beta), initial_state=core.dev(S0), output_final_state=True)
+    # the last batch row against the oracle (rows are independent)
+    row = [x[-1:] for x in args]
+    core.check([x[-1:] for x in got], core.run_ref(*row, dtype), dtype)
+    act = O.round_bf16 if dtype == "bf16" else (lambda x: x)
+    ro, rs = O.chunk_gated_delta_rule(*row[:5], initial_state=row[5], output_final_state=True, act_round=act)
+    assert core.rel(core.np_(o[-1:]), ro) < (core.BF16_TOL if dtype == "bf16" else core.F32_TOL)
+    assert core.rel(core.np_(fs[-1:]), rs) < core.F32_TOL
