@@ -55,7 +55,7 @@ constexpr int kBlockCols = 64;  // dv columns per block of the other kernels (nb
 // NWC_: 16-column state tiles (compute wavefronts) per workgroup: four, or two or one, so
 // that sequences x heads x dv / 16 tiles fill the chip when 64-column workgroups would leave
 // CUs idle (where loader wavefronts stage the rows; see scan_column_tiles).
-template <int DK, int MODE, int NWC_ = 4, bool BWD_ = false>
+template <int DK, int MODE, int NWC_ = 4, bool BWD_ = false, bool FUSE_ = false>
 struct Cfg {
   static constexpr int NWC = NWC_;
   static constexpr int BV = 16 * NWC;  // state columns per workgroup
@@ -88,11 +88,14 @@ struct Cfg {
   // with the compute wavefronts, each may then hold at most half the register file
   // loader wavefronts: two in the backward's bf16 recompute (the chunk after next's K/Q
   // rows in one's registers, its V rows and record in the other's, so that the loads are
-  // not queued behind the state stores of the same step) and in the bf16 forward scan's
-  // narrow workgroups (where the second loader takes a SIMD no compute wavefront uses:
-  // C4 2.663-2.666 -> 2.605-2.639 ms), one elsewhere.  In the forward scan's 64-column
-  // workgroups the second loader measured slower (C1 core call 0.311-0.319 against
-  // 0.292-0.297 ms).
+  // not queued behind the state stores of the same step) and in narrow workgroups (where
+  // the second loader takes a SIMD no compute wavefront uses: C4 2.663-2.666 ->
+  // 2.605-2.639 ms; layer, B=1 T=1,900 Hv=32, whose one loader waited each step for its
+  // direct loads and for the norm's exchange: 87.8 us, with the second loader and XWAVE 81,
+  // with FWAVE too 68.6; T=4,000 Hv=64, 32 columns: 179 -> 154), one elsewhere.  In the
+  // forward scan's 64-column workgroups the second loader measured slower (C1 core call
+  // 0.311-0.319 against 0.292-0.297 ms), and so did an exchange wavefront of its own (B=4
+  // T=4,096: 240 -> 246 us).
   static constexpr int SZK = DIRECT ? C * DK : NS * C * LDK;  // elements of a K or Q buffer
   static constexpr int SZV = DIRECT ? C * BV : NS * C * LDT;  // elements of a V buffer
   static constexpr int BUF = 2 * SZK * 2 + SZV * 2 + REC;     // bytes of one set of buffers
@@ -104,8 +107,12 @@ struct Cfg {
   // barriers.  fp32 inputs at d = 64 (B=2, T=512, H=4):
   // the scan 30.1 -> 23.6 us; layer rows at d = 64 (B=4, T=500, Hv=16): 22.1 -> 18.0 us.
   static constexpr bool LSTAGE = !DIRECT && 2 * BUF <= 160 * 1024;
-  static constexpr int NL = DIRECT ? (MODE == MODE_BF16 && (BWD_ || NWC_ < 4) ? 2 : 1) : (LSTAGE ? NST / 64 : 0);
-  static constexpr int NTH = NT + 64 * (NL + NH);
+  static constexpr int NL = DIRECT ? ((MODE == MODE_BF16 && BWD_) || NWC_ < 4 ? 2 : 1) : (LSTAGE ? NST / 64 : 0);
+  // (layer, 16 and 32 columns) one more wavefront stores or (FUSE) exchanges the rows'
+  // partial sums, so that the loaders wait for nothing but their rows, and (FUSE) one
+  // normalises the finished chunks
+  static constexpr bool XWAVE = VCONV && NWC_ < 4, FWAVE = XWAVE && FUSE_;
+  static constexpr int NTH = NT + 64 * (NL + NH + XWAVE + FWAVE);
   static constexpr int WPE = (NTH / 64 + 3) / 4;
   static constexpr int NBUF = DIRECT || LSTAGE ? 2 : 1;
   static constexpr int TOTAL = NBUF * BUF;
@@ -417,8 +424,9 @@ __device__ __forceinline__ void put_kq(const KQRegs& r, lds_bf16* sK, lds_bf16* 
 static_assert(kRecP % 1024 == 0 && kRecG % 1024 == 0, "P fills whole 1 KiB record pieces");
 template <int MODE, int BV, bool BWD>
 struct VRRegs {
-  static constexpr int NV = BV / 8, NR = rec_bytes(MODE) / 1024, NRX = rec_bytes(MODE, BWD) / 1024;
-  u32x4 v[NV], r[NRX];
+  static constexpr bool HAS_V = MODE != MODE_LAYER;  // the layer's V rows: helper wavefronts
+  static constexpr int NV = HAS_V ? BV / 8 : 0, NR = rec_bytes(MODE) / 1024, NRX = rec_bytes(MODE, BWD) / 1024;
+  u32x4 v[HAS_V ? NV : 1], r[NRX];
 };
 template <int MODE, int BV, bool BWD>
 __device__ __forceinline__ void stage_vr(const ChunkParams& p, long long t0, int nvalid,
@@ -430,7 +438,7 @@ __device__ __forceinline__ void stage_vr(const ChunkParams& p, long long t0, int
   const bf16_t* vb = (const bf16_t*)p.vs + t0 * p.vs_ld + (long long)h * p.DV + col0;
   const unsigned vld = (unsigned)p.vs_ld;
 #pragma unroll
-  for (int mi = 0; mi < SV; ++mi) {
+  for (int mi = 0; mi < R_::NV; ++mi) {
     const int row = RPI * mi + l / SV;
     const unsigned rr = (unsigned)(row < nvalid ? row : nvalid - 1);
     const unsigned g = (unsigned)((l % SV) ^ swz_v<SV>(row));
@@ -489,8 +497,8 @@ template <int DK, int MODE, bool BWD = false, int NWC_ = 4, bool FUSE = false>
 // One workgroup per CU is the design point (the state fills the register file): the
 // compiler may use the whole file (half of it with a loader wavefront, which shares a
 // SIMD) instead of holding back for a second workgroup.
-__global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amdgpu_waves_per_eu(Cfg<DK, MODE, NWC_, BWD>::WPE, Cfg<DK, MODE, NWC_, BWD>::WPE))) void scan_kernel(ChunkParams p) {
-  using Q_ = Cfg<DK, MODE, NWC_, BWD>;
+__global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute__((amdgpu_waves_per_eu(Cfg<DK, MODE, NWC_, BWD, FUSE>::WPE, Cfg<DK, MODE, NWC_, BWD, FUSE>::WPE))) void scan_kernel(ChunkParams p) {
+  using Q_ = Cfg<DK, MODE, NWC_, BWD, FUSE>;
   constexpr int NWC = Q_::NWC, BV = Q_::BV, NT = Q_::NT;
   constexpr int LDK = Q_::LDK;
   constexpr bool IS = Q_::IS, OS = Q_::OS;
@@ -513,8 +521,12 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
   __shared__ float sSS[WG_SS ? 2 : 1][WG_SS ? NWC : 1][C];
   float ss_prev = 0.f;  // this lane's row sum of the previous chunk, not yet in sSS
   static_assert(!FUSE || WG_SS, "the fused norm runs on the layer's direct-load scan");
-  constexpr int kRing = 4;  // (FUSE) chunks of bf16 o kept per compute wavefront
-  constexpr int kFin = 3;   // (FUSE) steps from a chunk to its normalisation
+  constexpr bool XW = Q_::XWAVE, FW = Q_::FWAVE;
+  // (FUSE) chunks of bf16 o kept per compute wavefront: with a finalizing wavefront a chunk
+  // is read while a later one is written
+  constexpr int kRing = FW ? 8 : 4;
+  constexpr int kFin = FW ? 4 : 3;  // (FUSE) steps from a chunk to its normalisation
+  static_assert(kFin < kRing, "a chunk is normalised before its ring entry is rewritten");
   // (FUSE) lane l's 4 x 4 bf16 o values of row block i of chunk c, wave w: sO[c % 4][w][i][l]
   __shared__ __align__(16) u32x2 sO[FUSE ? kRing : 1][FUSE ? NWC : 1][FUSE ? 4 : 1][64];
   __shared__ float sRN[FUSE ? 2 : 1][C];  // (FUSE) 1/RMS of each row of a chunk
@@ -522,8 +534,22 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
 
   const int tid = threadIdx.x, l = tid & 63, lq = l >> 4, lr = l & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool loader = wave >= NWC && wave < NWC + Q_::NL;  // loads, computes nothing
-  const bool helper = Q_::VCONV && wave >= NWC + Q_::NL;  // forms the V rows (layer, direct loads)
+  // Roles of the other wavefronts: lw, hw are a loader's (loads, computes nothing) and a
+  // helper's (layer, direct loads: forms the V rows) number, or negative.  Wavefront i runs on
+  // SIMD i % 4; in the layer's narrow workgroups the compute wavefronts share theirs with the
+  // exchange and (32 columns) a loader, which issue little, and not with the helpers or the
+  // finalizing wavefront.
+  int lw = wave >= NWC && wave < NWC + Q_::NL ? wave - NWC : -1;
+  int hw = Q_::VCONV && wave >= NWC + Q_::NL && wave < NWC + Q_::NL + Q_::NH ? wave - NWC - Q_::NL : -1;
+  bool xwave = false, fwave = false;  // stores or exchanges the row partials; normalises
+  if constexpr (XW) {
+    static_assert(NWC <= 2 && Q_::NL == 2 && Q_::NH == 2, "the roles below");
+    lw = NWC == 1 ? (wave == 1 || wave == 2 ? wave - 1 : -1) : (wave == 5 || wave == 6 ? wave - 5 : -1);
+    hw = NWC == 1 ? (wave == 3 ? 0 : wave == 5 ? 1 : -1) : (wave == 2 || wave == 3 ? wave - 2 : -1);
+    xwave = wave == 4;
+    fwave = FW && wave == 5 + NWC;
+  }
+  const bool loader = lw >= 0, helper = hw >= 0;
   const bool compute = wave < NWC;             // owns 16 state columns
   // XCD-aware work item (scan_item): a key head's workgroups share one XCD's L2, and
   // packed sequences start longest first
@@ -572,7 +598,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
   if (nchunks > 0) {
     const int nv0 = (int)((s1 - s0) < C ? (s1 - s0) : C);
     if constexpr (DIRECT) {
-      if (loader && wave == NWC) {
+      if (lw == 0) {
         stage_all<DK, MODE, BV, BWD>(p, s0, nv0, rec_of(0), hk, h, col0, (lds_bf16*)sK0, (lds_bf16*)sQ0,
                             (lds_bf16*)sV0, (lds_u8*)sRec0);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): landed before the first barrier
@@ -587,9 +613,16 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
   // the step; out = w (o rn) silu(z), stored through a buffer whose range ends at the
   // chunk's last valid row.  The row offsets are in the lane offsets, which the range
   // check covers (a scalar offset is not relied on to be checked).  c < 0 does nothing.
-  u32x2 zf[4];
-  const float4 nw4 = FUSE ? *(const float4*)(p.norm_w + col0 + 16 * wave + 4 * lq)
-                          : make_float4(0.f, 0.f, 0.f, 0.f);
+  // (FW: on the finalizing wavefront, for the NWC compute wavefronts' columns)
+  constexpr int NF = FW ? NWC : 1;
+  u32x2 zf[NF][4];
+  float4 nw4[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+    nw4[f] = FUSE && (!FW || fwave) ? *(const float4*)(p.norm_w + col0 + 16 * (FW ? f : wave) + 4 * lq)
+                                    : make_float4(0.f, 0.f, 0.f, 0.f);
+  // element offset of row lr, columns 4 lq .. +3 of compute wavefront f's slice
+  auto f_elem = [&](int f) { return (unsigned)lr * o_rs + 16u * (FW ? f : wave) + 4u * lq; };
   auto chunk_rows = [&](int c, long long& tc) {
     tc = s0 + (long long)c * C;
     return (int)((s1 - tc) < C ? (s1 - tc) : C);
@@ -602,8 +635,10 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
       const auto zr = buf_rsrc((const bf16_t*)p.z + (tc * p.Hv + h) * (long long)DV + col0,
                                2u * nvc * o_rs);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        zf[i] = __builtin_amdgcn_raw_buffer_load_b64(zr, o_lane_h + 2u * 16u * i * o_rs, 0, 0);
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          zf[f][i] = __builtin_amdgcn_raw_buffer_load_b64(zr, 2u * (f_elem(f) + 16u * i * o_rs), 0, 0);
     }
   };
   auto finalize = [&](int c) {
@@ -613,19 +648,21 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
       const int nvc = chunk_rows(c, tc);
       const auto orr = buf_rsrc((bf16_t*)p.out + (tc * p.Hv + h) * (long long)DV + col0,
                                 2u * nvc * o_rs);
-      const float w[4] = {nw4.x, nw4.y, nw4.z, nw4.w};
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const u32x2 ow = sO[c % kRing][wave][i][l];
+        const float w[4] = {nw4[f].x, nw4[f].y, nw4[f].z, nw4[f].w};
+        const u32x2 ow = sO[c % kRing][FW ? f : wave][i][l];
         const float rn = sRN[c & 1][16 * i + lr];
         uint32_t r[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const float o0 = __uint_as_float(ow[e] << 16), o1 = __uint_as_float(ow[e] & 0xffff0000u);
-          const float z0 = __uint_as_float(zf[i][e] << 16), z1 = __uint_as_float(zf[i][e] & 0xffff0000u);
+          const float z0 = __uint_as_float(zf[f][i][e] << 16), z1 = __uint_as_float(zf[f][i][e] & 0xffff0000u);
           r[e] = pack_bf16(w[2 * e] * (o0 * rn) * silu_fast(z0), w[2 * e + 1] * (o1 * rn) * silu_fast(z1));
         }
-        __builtin_amdgcn_raw_buffer_store_b64(u32x2{r[0], r[1]}, orr, o_lane_h + 2u * 16u * i * o_rs, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{r[0], r[1]}, orr, 2u * (f_elem(f) + 16u * i * o_rs), 0, 0);
       }
     }
   };
@@ -646,7 +683,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
         if (j >= 1) sSS[(j - 1) & 1][wave][16 * lq + lr] = ss_prev;
       }
       // (FUSE) z of the chunk normalised at the end of this step, in flight meanwhile
-      if constexpr (FUSE) z_load(j - kFin);
+      if constexpr (FUSE && !FW) z_load(j - kFin);
     } else if constexpr (LSTAGE) {
       // the loaders have stored chunk j, and chunk j-1, the last reader of the other set,
       // is finished everywhere
@@ -953,7 +990,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
       for (int i = 0; i < 4; ++i)
         sO[j % kRing][wave][i][l] = u32x2{pack_bf16(o[i][0], o[i][1]), pack_bf16(o[i][2], o[i][3])};
       sSS[j & 1][wave][16 * lq + lr] = row_sq_scatter(o);
-      finalize(j - kFin);
+      if constexpr (!FW) finalize(j - kFin);
     } else {
       // unnormalised o in bf16; the epilogue kernel applies the norm, from the fp32 sums
       // of squares stored below
@@ -989,6 +1026,8 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
   if constexpr (DIRECT) {
     if (loader && Q_::NL == 2) {
       if constexpr (Q_::NL == 2) {
+        // (layer) the other wavefronts' steps after the last chunk
+        constexpr int DRAIN = WG_SS ? (FUSE ? kFin : 2) : 0;
         // one barrier per chunk, as the compute wavefronts: after the barrier at the top of
         // chunk j, buffer (j + 1) % 2 is free and receives chunk j + 1 from the registers,
         // which then receive chunk j + 2.  The two loaders run separate loops, so neither
@@ -997,7 +1036,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
           tc = s0 + (long long)c * C;
           return (int)((s1 - tc) < C ? (s1 - tc) : C);
         };
-        if (wave == NWC) {  // the K and Q rows
+        if (lw == 0) {  // the K and Q rows
           KQRegs r;
           long long tc;
           if (nchunks > 1) {
@@ -1036,8 +1075,9 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
             if (j + 1 < nchunks) step(j + 1, (lds_bf16*)sV0, (lds_u8*)sRec0);
           }
         }
+        for (int j = 0; nchunks > 0 && j < DRAIN; ++j) lds_barrier();
       }
-    } else if (loader) {
+    } else if (loader || xwave) {
       // one barrier per chunk, as the compute wavefronts: after the barrier at the top of
       // chunk j, buffer (j + 1) % 2 is free and receives chunk j + 1
       // (layer) lane l's row of chunk jj: the workgroup's partial, one per row, stored
@@ -1060,11 +1100,10 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
       // writes it again, kXchRing chunks later (a block writes chunk c + 4's partial only
       // after it has seen every block's partial of chunk c + 2, which they publish after
       // they have read chunk c's)
-      auto xch_rsrc = [&](int c, int s, unsigned bytes) {
-        return buf_rsrc(p.ss_xch + 2 * ((((size_t)n * p.Hv + h) * p.ss_xch_slots + s) * kXchRing +
-                                        c % kXchRing) * C,
-                        bytes);
-      };
+      // (one resource over the value head's ring; the entry goes in the scalar offset)
+      const auto xr = buf_rsrc(p.ss_xch + 2 * (((size_t)n * p.Hv + h) * p.ss_xch_slots) * kXchRing * C,
+                               8u * (unsigned)p.ss_xch_slots * kXchRing * C);
+      auto xch_off = [&](int c, int s) { return 8 * (s * kXchRing + c % kXchRing) * C; };
       // this workgroup's partial of chunk c's row l (its waves' partials, in sSS since the
       // barrier that opened this step), written through to memory with tag c + 1
       auto publish = [&](int c) {
@@ -1074,8 +1113,9 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
           float v[NWC];
 #pragma unroll
           for (int w = 0; w < NWC; ++w) v[w] = sSS[c & 1][w][l];
-          __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(ss_tree<NWC>(v)), (unsigned)c + 1u},
-                                                xch_rsrc(c, blk, 8u * nvc), 8u * l, 0, 17);
+          // rows past the chunk's end are given an offset past the range: dropped
+          __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(ss_tree<NWC>(v)), (unsigned)c + 1u}, xr,
+                                                l < nvc ? 8u * l : 0x80000000u, xch_off(c, blk), 17);
         }
       };
       // every block's partial of chunk c's row l, read past the caches (system scope)
@@ -1083,7 +1123,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
         if constexpr (FUSE) {
 #pragma unroll
           for (int s = 0; s < NBX; ++s)
-            if (s < p.nb) xv[s] = __builtin_amdgcn_raw_buffer_load_b64(xch_rsrc(c, s, 8u * C), 8u * l, 0, 17);
+            if (s < p.nb) xv[s] = __builtin_amdgcn_raw_buffer_load_b64(xr, 8u * l, xch_off(c, s), 17);
         }
       };
       // once every valid row's entries carry chunk c's tag: the row's sum over the blocks in the
@@ -1128,7 +1168,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
           const int nvn = (int)((s1 - tn) < C ? (s1 - tn) : C);
           stage_all<DK, MODE, BV, BWD>(p, tn, nvn, rec_of(j + 1), hk, h, col0, nK, nQ, nV, nRec);
         }
-        if constexpr (FUSE) {
+        if constexpr (FUSE && !XW) {
           // chunk j - 1's partial (its waves wrote sSS before this step's barrier), then
           // the partials of chunk j - 2 that every block published a step ago
           if (j >= 1 && j - 1 < nchunks) publish(j - 1);
@@ -1136,11 +1176,32 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
         }
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): landed before the next barrier
         if constexpr (FUSE) {
-          if (j >= 2 && j - 2 < nchunks) finish(j - 2);
+          if constexpr (!XW)
+            if (j >= 2 && j - 2 < nchunks) finish(j - 2);
         } else {
           if (j >= 2) store_ss(j - 2);  // written after barrier j - 1, visible after barrier j
         }
       };
+      if (XW && xwave) {
+        // The exchange (FUSE) on its own wavefront, a step deeper: at step j the partials of chunk
+        // j - 3, gathered a step ago, are summed; then chunk j - 1's is published and chunk
+        // j - 2's are gathered.  In that order a block that has published chunk c + 2's has
+        // read every partial of chunk c, and one that publishes chunk c + 4's has seen every
+        // block's of chunk c + 2: the ring of four still suffices.
+        if constexpr (FUSE) {
+          for (int j = 0; nchunks > 0 && j < nchunks + kFin; ++j) {
+            lds_barrier();
+            if (j >= 3 && j - 3 < nchunks) finish(j - 3);
+            if (j >= 1 && j - 1 < nchunks) publish(j - 1);
+            if (j >= 2 && j - 2 < nchunks) gather(j - 2);
+          }
+        } else {
+          for (int j = 0; nchunks > 0 && j < nchunks + 2; ++j) {
+            lds_barrier();
+            if (j >= 2) store_ss(j - 2);
+          }
+        }
+      } else {
       for (int j = 0; j < nchunks; j += 2) {
         load(j, (lds_bf16*)sK1, (lds_bf16*)sQ1, (lds_bf16*)sV1, (lds_u8*)sRec1);
         if (j + 1 < nchunks) load(j + 1, (lds_bf16*)sK0, (lds_bf16*)sQ0, (lds_bf16*)sV0, (lds_u8*)sRec0);
@@ -1157,6 +1218,16 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
           store_ss(nchunks - 1);
         }
       }
+      }
+    } else if (fwave) {
+      // chunk j - kFin, its z loaded a step ahead
+      if constexpr (FW) {
+        for (int j = 0; nchunks > 0 && j < nchunks + kFin; ++j) {
+          lds_barrier();
+          finalize(j - kFin);
+          if (j + 1 < nchunks + kFin) z_load(j + 1 - kFin);
+        }
+      }
     } else if (helper) {
       if constexpr (Q_::VCONV) {
         // one barrier per chunk, as the loader: after the barrier at the top of chunk j,
@@ -1169,7 +1240,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
         // are loaded one chunk step ahead (two register sets; loads past the last chunk
         // repeat it), so their latency is off the step.
         constexpr int SV = BV / 8, R = BV / 16;
-        const int hl = tid - 64 * (NWC + Q_::NL);
+        const int hl = 64 * hw + l;
         const int g = hl % SV, r0 = (hl / SV) * R;
         const int chu = 2 * p.Hk * DK + h * DV + col0;
         uint32_t wp[8][2];
@@ -1204,9 +1275,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
           }
         }
         if (nchunks > 0) {  // the loader's barriers after its loop
-          lds_barrier();
-          lds_barrier();
-          if constexpr (FUSE) lds_barrier();
+          for (int j = 0; j < (FUSE ? kFin : 2); ++j) lds_barrier();
         }
       }
     } else {
@@ -1218,8 +1287,10 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
         if (nchunks > 0)
           for (int j = nchunks; j < nchunks + kFin; ++j) {
             lds_barrier();
-            z_load(j - kFin);
-            finalize(j - kFin);
+            if constexpr (!FW) {
+              z_load(j - kFin);
+              finalize(j - kFin);
+            }
           }
       } else if constexpr (WG_SS) {  // the loader's two barriers after its loop
         if (nchunks > 0) {
@@ -1307,7 +1378,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD>::NTH)) __attribute__((amd
 // blocks) is replaced by the scan's own count in a copy of the parameters.
 template <int DK, int MODE, bool BWD = false, int NWC = 4, bool FUSE = false>
 hipError_t launch_scan_cfg(const ChunkParams& p, hipStream_t stream) {
-  using Q_ = Cfg<DK, MODE, NWC, BWD>;
+  using Q_ = Cfg<DK, MODE, NWC, BWD, FUSE>;
   ChunkParams q = p;
   q.nb = p.DV / Q_::BV;
   // (layer) row-sum partials per (token, value head): one per workgroup with direct
@@ -1316,20 +1387,6 @@ hipError_t launch_scan_cfg(const ChunkParams& p, hipStream_t stream) {
   const unsigned grid = (unsigned)(q.N * q.Hv * q.nb);
   hipLaunchKernelGGL((scan_kernel<DK, MODE, BWD, NWC, FUSE>), dim3(grid), dim3(Q_::NTH), 0, stream, q);
   return hipGetLastError();
-}
-
-// Compute units of the current device (queried once per device).
-int device_cus() {
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] == 0) {
-    int v = 0;
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
-      v = 256;
-    cus[dev] = v;
-  }
-  return cus[dev];
 }
 
 // Column tiles per workgroup: 4 (64 columns) when that gives a workgroup per CU, else 2 or
@@ -1357,6 +1414,20 @@ hipError_t launch_scan_tiles(const ChunkParams& p, hipStream_t stream) {
 }
 
 }  // namespace
+
+// Compute units of the current device (queried once per device).
+int device_cus() {
+  static int cus[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cus[dev] == 0) {
+    int v = 0;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
+      v = 256;
+    cus[dev] = v;
+  }
+  return cus[dev];
+}
 
 int chunk_block_cols() { return kBlockCols; }
 

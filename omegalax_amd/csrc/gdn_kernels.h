@@ -144,6 +144,7 @@ constexpr int kModeBF16 = 0, kModeF32 = 1, kModeLayer = 2;
 
 bool chunk_dims_supported(int dk, int dv, bool f32_inputs);
 int chunk_block_cols();
+int device_cus();  // compute units of the current device
 // 16-column tiles per workgroup (4, 2 or 1) of the forward and reverse scans
 int scan_column_tiles(int N, int Hv, int DV);
 bool layer_dims_supported(int dk, int dv);

@@ -1,0 +1,89 @@
+"""GPU parity of the forward kernels at the edges of their dispatch, against the fp64 oracle.
+
+The layer scan takes 16-, 32- or 64-column workgroups and either applies the gated norm itself
+or leaves it to the epilogue kernel, by the number of sequences x value heads x columns.
+The suite's small shapes all take the first of each.  Tolerances as in
+tests/test_gpu_layer.py, whose inputs these reuse.
+"""
+import numpy as np
+import pytest
+
+from omegalax_amd import workloads as W
+
+import test_gpu_layer as layer
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+ROWS = ("mixed_qkv", "z", "a", "b")
+
+
+def check_rows(B, T, dims, rows, seed):
+    """A batch on the GPU, the given rows of it (rows are independent) against the oracle."""
+    d = W.layer_inputs(B, T, **dims, seed=seed)
+    S0 = (0.02 * np.random.default_rng(seed).standard_normal(
+        (B, dims["Hv"], dims["dk"], dims["dv"]))).astype(np.float32)
+    out, S, conv = layer.gpu_prefill(W.to_device(d), dims, None, S0)
+    for n in rows:
+        one = {k: (v[n:n + 1] if k in ROWS else v) for k, v in d.items()}
+        ref, S_ref, conv_ref = layer.ref_prefill(one, dims, None, S0[n:n + 1])
+        assert layer.rel(layer.np_(out[n:n + 1]), ref) < layer.BF16_TOL
+        assert layer.rel(layer.np_(S[n:n + 1]), S_ref) < layer.STATE_TOL
+        assert np.array_equal(layer.np_(conv[n:n + 1]), conv_ref)
+
+
+@pytest.mark.parametrize("T", [1, 64, 65, 129, 200, 257, 385, 640])
+@pytest.mark.parametrize("B,Hk,Hv,dv", [
+    (1, 1, 2, 128),    # 16-column workgroups
+    (16, 2, 4, 128),   # 32-column, 256 workgroups
+])
+def test_layer_scan_pipeline_depth(B, Hk, Hv, dv, T):
+    """Sequences of one to ten chunks: the exchange and finalizing wavefronts run up to four
+    chunks behind the scan and drain it after the last one."""
+    layer.say(f"layer scan depth B={B} Hv={Hv} T={T}")
+    check_rows(B, T, dict(Hk=Hk, dk=128, Hv=Hv, dv=dv), (0, B - 1), 8000 + T)
+
+
+@pytest.mark.parametrize("B,Hk,Hv,dk,dv", [
+    (8, 1, 4, 128, 256),    # 32-column workgroups, eight to a value head, one round
+    (9, 1, 4, 128, 256),    # the same, past one round: the epilogue kernel
+    (24, 1, 4, 128, 128),   # 32-column, past one round
+    (25, 1, 4, 128, 128),   # the same, groups not a multiple of eight
+    (33, 1, 4, 128, 128),   # 64-column, past one round, groups not a multiple of eight
+    (40, 1, 4, 128, 128),   # 64-column, past one round
+    (24, 1, 3, 128, 256),   # 64-column, four to a value head, past one round
+    (40, 2, 4, 128, 64),    # one workgroup to a value head
+    (40, 1, 4, 64, 128),    # dk = 64
+])
+def test_layer_scan_at_every_workgroup_width(B, Hk, Hv, dk, dv):
+    layer.say(f"layer scan widths B={B} Hk={Hk} Hv={Hv} dk={dk} dv={dv}")
+    check_rows(B, 460, dict(Hk=Hk, dk=dk, Hv=Hv, dv=dv), (0, B // 2, B - 1), 8100 + B + dv)
+
+
+def test_layer_scan_of_many_packed_sequences():
+    """40 packed sequences, some of them empty, from their own states: past one round of the
+    chip, longest first."""
+    layer.say("layer scan: 40 packed sequences")
+    dims = dict(Hk=1, dk=128, Hv=4, dv=128)
+    rng = np.random.default_rng(8200)
+    lens = rng.integers(0, 1100, size=40)
+    lens[[0, 7, 39]] = 0
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    d = W.layer_inputs(1, int(cu[-1]), **dims, seed=8201)
+    S0 = (0.02 * rng.standard_normal((40, 4, 128, 128))).astype(np.float32)
+    out, S, conv = layer.gpu_prefill(W.to_device(d), dims, cu, S0)
+    ref, S_ref, conv_ref = layer.ref_prefill(d, dims, cu, S0)
+    assert layer.rel(layer.np_(out), ref) < layer.BF16_TOL
+    assert layer.rel(layer.np_(S), S_ref) < layer.STATE_TOL
+    assert np.array_equal(layer.np_(conv), conv_ref)
+
+
+def test_layer_of_no_tokens_keeps_the_states():
+    """T = 0 over more workgroups than the chip holds: no chunk to prepare, states copied."""
+    layer.say("layer T=0")
+    dims = dict(Hk=1, dk=128, Hv=4, dv=128)
+    d = W.layer_inputs(40, 1, **dims, seed=8300)
+    t = W.to_device({k: (v[:, :0] if k in ROWS else v) for k, v in d.items()})
+    S0 = np.random.default_rng(8301).standard_normal((40, 4, 128, 128)).astype(np.float32)
+    _, S, _ = layer.gpu_prefill(t, dims, None, S0)
+    assert np.array_equal(layer.np_(S), S0)
