@@ -118,6 +118,7 @@ __device__ __forceinline__ void l2norm8(float* x) {
 // One (chunk, key head) task: chunk ci of sequence n (tokens [t0, t0 + nvalid)).
 struct PrepTask {
   int ci, hk, n, nvalid;
+  int h0, nh;  // the value heads this workgroup takes
   long long s0, t0;
 };
 
@@ -214,20 +215,19 @@ __device__ __forceinline__ void load_task_inputs(const ChunkParams& p, const Pre
       if constexpr (F32) pf.raw[k * Q_::RAWW + 1] = src[1];
     }
   }
-  const int gqa = p.Hv / p.Hk;
-  const int gg = tid >> 6;  // this wavefront's value head within the key head
-  const long long g0 = t.t0 * p.Hv + (long long)t.hk * gqa;  // token t0, first value head
+  const int gg = tid >> 6;  // this wavefront's value head among the workgroup's
+  const long long g0 = t.t0 * p.Hv + t.h0;  // token t0, first value head
   pf.ga = 0.f;
   pf.gb = 0.f;
   pf.alog = 0.f;
   pf.dtb = 0.f;
   if constexpr (MODE == MODE_LAYER) {
-    if (gg < gqa) {
-      pf.alog = p.A_log[t.hk * gqa + gg];
-      pf.dtb = p.dt_bias[t.hk * gqa + gg];
+    if (gg < t.nh) {
+      pf.alog = p.A_log[t.h0 + gg];
+      pf.dtb = p.dt_bias[t.h0 + gg];
     }
   }
-  if (gg < gqa && l < t.nvalid) {
+  if (gg < t.nh && l < t.nvalid) {
     const unsigned lo = (unsigned)l * (unsigned)p.Hv;  // lane = token
     if constexpr (MODE == MODE_LAYER) {
       pf.ga = bf2f(*at_bytes((const bf16_t*)p.a + g0 + gg, 2u * lo));
@@ -261,7 +261,7 @@ __device__ __forceinline__ void put_f32_tile(float* m, int bi, int bj, f32x4 a) 
 // that X is not written a second time: at C1 the backward's prep 112 -> 90 us, the recompute
 // scan 296 -> 285 us, the reverse scan 320 -> 308 us.
 template <int DK, int MODE, bool BWD = false>
-__global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_kernel(ChunkParams p) {
+__global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_kernel(ChunkParams p, int parts) {
   using Q_ = PrepCfg<DK, MODE>;
   constexpr int LDK = Q_::LDK, SEGS = Q_::SEGS;
   constexpr bool IS = Q_::IS, F32 = MODE == MODE_F32;
@@ -276,24 +276,28 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
 
   const int tid = threadIdx.x, l = tid & 63, lq = l >> 4, lr = l & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int gqa = p.Hv / p.Hk;
-  // tasks: (chunk, key head) pairs, one per workgroup (the grid may hold spare ones)
+  // tasks: (chunk, key head) pairs, `parts` consecutive workgroups each, which take the key
+  // head's value heads in equal shares (the grid may hold spare ones)
   const int n_ci = p.chunk_off ? uniform_ld(p.chunk_off, p.N) : p.n_rec;
   const int total = n_ci * p.Hk;
-  const int task = (int)blockIdx.x;
+  const int task = (int)blockIdx.x / parts, part = (int)blockIdx.x % parts;
   if (task >= total) return;  // uniform
 
   PrepIn<DK, MODE> pf;
   {
-    const PrepTask tk = prep_task(p, task, n_ci);
+    PrepTask tk = prep_task(p, task, n_ci);
+    tk.nh = p.Hv / p.Hk / parts;
+    tk.h0 = (tk.hk * parts + part) * tk.nh;
     load_task_inputs<DK, MODE>(p, tk, pf);
+    const int nh = tk.nh, h0 = tk.h0;
+    const bool first = part == 0;  // writes the key head's q and k rows
     const int hk = tk.hk, ci = tk.ci, n = tk.n, nvalid = tk.nvalid;
     const long long s0 = tk.s0, t0 = tk.t0;
 
     // -------------------------------------------------------------- q, k, v rows
     if constexpr (MODE == MODE_LAYER) {
       // dk = 64: wave 0 forms the k rows, wave 1 the q rows, waves 2-3 the v channels of
-      // the gqa value heads (16 rows per item).  dk = 128, where the scan forms v: waves
+      // the workgroup's value heads (16 rows per item).  dk = 128, where the scan forms v: waves
       // 0 and 2 the k rows (top and bottom half of the chunk), waves 1 and 3 the q rows.
       // Lane = 8-channel group g + SEGS * row part; each lane streams its rows, and the
       // SEGS lanes of a row are adjacent, so the row's L2 norm is a DPP sum.
@@ -310,7 +314,7 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
         const unsigned ostride = (unsigned)(p.Hk * DK);
         const auto gout = buf_rsrc((bf16_t*)(which == 0 ? p.kn : p.qn) + t0 * (long long)p.Hk * DK +
                                        (long long)hk * DK,
-                                   2u * (unsigned)nvalid * ostride);
+                                   first ? 2u * (unsigned)nvalid * ostride : 0u);
         conv_rows<ROWS>(p, n, s0, t0, nvalid, r0, (which == 0 ? p.Hk * DK : 0) + hk * DK, 8 * g,
                         [&](int m, const u32x4& yw) {
           float y[8];
@@ -322,11 +326,11 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
           __builtin_amdgcn_raw_buffer_store_b128(hw, gout, 2u * ((unsigned)r * ostride + 8u * g), 0, 0);
         });
       } else if constexpr (!layer_v_in_scan(DK)) {
-        const int VG = gqa * p.DV / 8;  // 8-channel groups of v
-        const int vch0 = 2 * p.Hk * DK + hk * gqa * p.DV;
+        const int VG = nh * p.DV / 8;  // 8-channel groups of v
+        const int vch0 = 2 * p.Hk * DK + h0 * p.DV;
         const unsigned vstride = (unsigned)(p.Hv * p.DV);
         // rows past nvalid are dropped by the range (no store under a branch)
-        const auto vout = buf_rsrc((bf16_t*)p.vc + t0 * (long long)p.Hv * p.DV + (long long)hk * gqa * p.DV,
+        const auto vout = buf_rsrc((bf16_t*)p.vc + t0 * (long long)p.Hv * p.DV + (long long)h0 * p.DV,
                                    2u * (unsigned)nvalid * vstride);
         for (int it = tid - 128; it < VG * 4; it += 128) {
           const int g = it % VG, r0 = (it / VG) * 16;
@@ -368,7 +372,7 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
         if constexpr (IS) *(u32x4*)(dst + K_LO) = pack8_lo(x);
         if constexpr (F32) {  // fp32 rows are stored as they form (no register copy)
           void* out = which == 0 ? p.kn : p.qn;
-          if (out && (nvalid == C || r < nvalid)) {
+          if (out && first && (nvalid == C || r < nvalid)) {
             const long long o0 = t0 * (long long)p.Hk * DK + (long long)hk * DK;
             const unsigned lo = (unsigned)r * (unsigned)(p.Hk * DK) + 8u * seg;
             float4* d4 = (float4*)at_bytes((float*)out + o0, 4u * lo);
@@ -385,7 +389,7 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
           const int rem = (k * NT) % PER + tid;
           const int r = rem / SEGS, seg = rem % SEGS;
           void* out = which == 0 ? p.kn : p.qn;
-          if (out && (nvalid == C || r < nvalid)) {
+          if (out && first && (nvalid == C || r < nvalid)) {
             // row t0 of this key head (uniform) plus the lane's byte offset
             const long long o0 = t0 * (long long)p.Hk * DK + (long long)hk * DK;
             const unsigned lo = (unsigned)r * (unsigned)(p.Hk * DK) + 8u * seg;
@@ -426,8 +430,8 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
     float* gw = sGw + wave * 2 * C;  // this wave's G log2(e) [0, C) and beta [C, 2C)
     const size_t rec_stride = (size_t)rec_bytes(MODE, BWD);
 
-    for (int gg = 0; gg < gqa; ++gg) {
-      const int h = hk * gqa + gg;
+    for (int gg = 0; gg < nh; ++gg) {
+      const int h = h0 + gg;
       const auto rec = buf_rsrc(p.rec + ((size_t)ci * p.Hv + h) * rec_stride, (unsigned)rec_stride);
       float* xb = BWD ? p.xlpg + ((size_t)ci * p.Hv + h) * xlpg_floats(IS) : nullptr;
       if constexpr (BWD && IS) {
@@ -445,12 +449,12 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
       // inputs come from LDS only: a global load here, whose register the loop reuses,
       // would make every value head wait for all of the wavefront's outstanding memory
       // operations (this task's row and record stores).
-      if (gg >= kGatePf && gg % kGatePf == 0) {  // uniform; only when gqa > kGatePf
+      if (gg >= kGatePf && gg % kGatePf == 0) {  // uniform; only when nh > kGatePf
         // the next kGatePf heads' gate inputs replace the staged ones (every wave has
         // passed the previous head's last barrier, so sGin is free)
         if (wave < kGatePf) {
           float ga = 0.f, gb = 0.f;
-          if (gg + wave < gqa && l < nvalid) {
+          if (gg + wave < nh && l < nvalid) {
             const long long i0 = t0 * p.Hv + h + wave;
             const unsigned lo = (unsigned)l * (unsigned)p.Hv;
             if constexpr (MODE == MODE_LAYER) {
@@ -464,7 +468,7 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
           sGin[wave * 2 * C + l] = ga;
           sGin[wave * 2 * C + C + l] = gb;
           if constexpr (MODE == MODE_LAYER) {
-            if (l == 0 && gg + wave < gqa) {
+            if (l == 0 && gg + wave < nh) {
               sPar[wave][0] = p.A_log[h + wave];
               sPar[wave][1] = p.dt_bias[h + wave];
             }
@@ -657,7 +661,7 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
       lds_barrier();  // sLf / sTd are rewritten for the next value head
     }
     // (layer) the task of a sequence's first chunk clears the exchange ring of the row
-    // partials of the sequence's value heads under this key head (tag 0); the scan that
+    // partials of the sequence's value heads that it takes (tag 0); the scan that
     // fuses the gated norm writes chunk c's entries with tag c + 1 (stores through a buffer
     // whose range ends at the ring: lanes past it are dropped).  The scan writes and reads
     // the ring at system scope, past the L2s, so the zeros are written through to memory
@@ -665,9 +669,9 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
     // entries there carry the tags this call waits for.
     if constexpr (MODE == MODE_LAYER) {
       if (p.ss_xch && t0 == s0) {
-        const int cnt = gqa * p.ss_xch_slots * kXchRing * C;  // {value, tag} pairs
+        const int cnt = nh * p.ss_xch_slots * kXchRing * C;  // {value, tag} pairs
         const auto xr = buf_rsrc(
-            p.ss_xch + 2 * (((size_t)n * p.Hv + hk * gqa) * p.ss_xch_slots) * kXchRing * C,
+            p.ss_xch + 2 * (((size_t)n * p.Hv + h0) * p.ss_xch_slots) * kXchRing * C,
             8u * (unsigned)cnt);
         for (int k = 0; k < cnt; k += NT)
           __builtin_amdgcn_raw_buffer_store_b64(u32x2{0u, 0u}, xr, 8u * (unsigned)(k + tid), 0, 17);
@@ -678,11 +682,20 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
 
 template <int DK, int MODE, bool BWD = false>
 hipError_t launch_prep_cfg(const ChunkParams& p, hipStream_t stream) {
-  // one workgroup per (chunk slot, key head)
+  // one workgroup, or several, per (chunk slot, key head)
   const long long tasks = (long long)p.n_rec * p.Hk;
   if (tasks == 0) return hipSuccess;
-  const unsigned grid = (unsigned)tasks;
-  hipLaunchKernelGGL((prep_kernel<DK, MODE, BWD>), dim3(grid), dim3(NT), 0, stream, p);
+  // A grid the chip holds at once is one workgroup's latency: the value heads of a key head,
+  // one after the other in one workgroup, then go to workgroups of their own (each forms the
+  // rows and Gram tiles again) as far as all of them are still resident together.
+  // B=1 T=77 Hk=16 Hv=32 d=128: 15.0 -> 12.6 us; T=300 Hk=8 Hv=32: 16.1 -> 10.2 us.
+  const int gqa = p.Hv / p.Hk;
+  const long long room = (long long)prep_blocks_per_cu<DK, MODE>() * device_cus();
+  int parts = 1;
+  for (int d = 2; d <= gqa && tasks * d <= room; ++d)
+    if (gqa % d == 0) parts = d;
+  const unsigned grid = (unsigned)(tasks * parts);
+  hipLaunchKernelGGL((prep_kernel<DK, MODE, BWD>), dim3(grid), dim3(NT), 0, stream, p, parts);
   return hipGetLastError();
 }
 

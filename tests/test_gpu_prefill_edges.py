@@ -1,9 +1,10 @@
 """GPU parity of the forward kernels at the edges of their dispatch, against the fp64 oracle.
 
 The layer scan takes 16-, 32- or 64-column workgroups and either applies the gated norm itself
-or leaves it to the epilogue kernel, by the number of sequences x value heads x columns.
+or leaves it to the epilogue kernel, by the number of sequences x value heads x columns; the
+prep gives a key head's value heads to one workgroup or to several, by the number of chunks.
 The suite's small shapes all take the first of each.  Tolerances as in
-tests/test_gpu_layer.py, whose inputs these reuse.
+tests/test_gpu_layer.py and tests/test_gpu_prefill.py, whose inputs these reuse.
 """
 import numpy as np
 import pytest
@@ -11,6 +12,7 @@ import pytest
 from omegalax_amd import workloads as W
 
 import test_gpu_layer as layer
+import test_gpu_prefill as core
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -87,3 +89,27 @@ def test_layer_of_no_tokens_keeps_the_states():
     S0 = np.random.default_rng(8301).standard_normal((40, 4, 128, 128)).astype(np.float32)
     _, S, _ = layer.gpu_prefill(t, dims, None, S0)
     assert np.array_equal(layer.np_(S), S0)
+
+
+@pytest.mark.parametrize("B,T,Hk,Hv,dtype", [
+    (1, 70, 1, 1, "bf16"), (1, 70, 1, 4, "bf16"),   # one part; one value head to a part
+    (1, 130, 1, 8, "bf16"), (1, 130, 1, 6, "f32"),
+    (80, 300, 1, 6, "bf16"),                        # 400 chunks: two value heads to a part or more
+    (40, 300, 1, 6, "f32"),
+    (80, 300, 2, 4, "bf16"),                        # 800 chunk tasks
+])
+def test_prep_split_over_value_heads(B, T, Hk, Hv, dtype):
+    core.say(f"prep split B={B} T={T} Hk={Hk} Hv={Hv} {dtype}")
+    args = core.make(8400 + T + Hv, B, T, Hk, Hv, 64, 64, dtype)
+    o, S = core.run_gpu(*args, dtype)
+    for n in (0, B - 1):
+        ro, rs = core.run_ref(*(x[n:n + 1] for x in args), dtype)
+        tol = core.BF16_TOL if dtype == "bf16" else core.F32_OUT_TOL
+        assert core.rel(o[n:n + 1], ro) < tol
+        assert core.rel(S[n:n + 1], rs) < core.STATE_TOL
+
+
+@pytest.mark.parametrize("B,T,Hk,Hv", [(1, 70, 1, 1), (1, 70, 2, 8), (1, 130, 1, 6), (70, 300, 1, 6)])
+def test_layer_prep_split_over_value_heads(B, T, Hk, Hv):
+    layer.say(f"layer prep split B={B} T={T} Hk={Hk} Hv={Hv}")
+    check_rows(B, T, dict(Hk=Hk, dk=64, Hv=Hv, dv=64), (0, B - 1), 8500 + T + Hv)
