@@ -89,7 +89,7 @@ def lib() -> ctypes.CDLL:
 
 def call(name: str, *args) -> int:
     """Call entry point `name`; raise GDNError on a negative return."""
-    L = lib()
+    L = _lib or lib()
     rc = getattr(L, name)(*args)
     if rc != OK:
         raise GDNError(name, rc, L.omx_gdn_last_error().decode())

@@ -30,23 +30,24 @@ def _ptr(t):
 
 
 def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle of the current stream, without building a torch.cuda.Stream per call
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _dev(*ts):
-    dev = None
+    first, index = None, -1
     for t in ts:
         if t is None:
             continue
         if not t.is_cuda:
             raise ValueError("omegalax_amd kernels need GPU tensors (got a CPU tensor)")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError(f"tensors on different devices: {dev} vs {t.device}")
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise ValueError(f"tensors on different devices: {first.device} vs {t.device}")
         if not t.is_contiguous():
             raise ValueError("omegalax_amd kernels need contiguous tensors")
-    return dev
+    return None if first is None else first.device
 
 
 def _dtype_code(t):
@@ -58,7 +59,9 @@ def _dtype_code(t):
 
 
 def _f32(t):
-    return None if t is None else t.to(torch.float32).contiguous()
+    if t is None or (t.dtype is torch.float32 and t.is_contiguous()):
+        return t
+    return t.to(torch.float32).contiguous()
 
 
 def _cu_seqlens(cu, B, T, dev):
