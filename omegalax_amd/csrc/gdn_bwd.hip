@@ -406,8 +406,7 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
   // chunk step later.
   constexpr int NKQ = 2 * C * (DK / 4) / NT;
   static_assert(NKQ * NT == 2 * C * (DK / 4), "item split");
-  constexpr int NXP = 2 * kNPairs * 64 / NT;  // (PREC) 16-byte pieces of the record's X
-  static_assert(NXP * NT == 2 * kNPairs * 64, "record pieces");
+  constexpr int NXP = (2 * kNPieces * 64 + NT - 1) / NT;  // (PREC) 16-byte items of the record's X
   struct Pf {
     typename Vec4<KT>::type pkq[NKQ];
     float4 pdo[C * BV / 4 / NT], pxp[PREC ? 1 : 2 * C * 16 / NT];
@@ -446,7 +445,8 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
     const unsigned char* rec = p.rec + ((size_t)sl * p.Hv + h) * rec_stride;
     if constexpr (PREC) {
 #pragma unroll
-      for (int m = 0; m < NXP; ++m) f.px[m] = *(const u32x4*)(rec + kRecT + 16 * (st + m * NT));
+      for (int m = 0; m < NXP; ++m)
+        f.px[m] = *(const u32x4*)(rec + kRecT + 16 * (st + m * NT));  // (past X: P, unused)
       f.pg = xb[kXlpgG + (st & (C - 1))];
     } else {
 #pragma unroll
@@ -476,15 +476,25 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
       put_row4(sDOh, sDOl, (it / (BV / 4)) * LDB + 4 * (it % (BV / 4)), f32x4{f.pdo[m].x, f.pdo[m].y, f.pdo[m].z, f.pdo[m].w});
     }
     if constexpr (PREC) {
-      // piece 2x + part of the record's T part: lane (q, r) of pair x = (ib, jp) holds
-      // X[16 ib + r][32 jp + 4q .. +3] and [32 jp + 16 + 4q .. +3], hi (part 0) or lo
+      // piece 2x + part of the record's T part, hi (part 0) or lo: lane (q, r) of the pieces
+      // x >= 1, pairs (ib, jp) = (1, 0), (2, 0), (3, 0), (3, 1), holds X[16 ib + r][32 jp +
+      // 4q .. +3] and [32 jp + 16 + 4q .. +3]; of piece 0 the diagonal tiles (0, 0) and
+      // (2, 2), whose right neighbours are zero
 #pragma unroll
       for (int m = 0; m < NXP; ++m) {
         const int piece = (st >> 6) + m * (NT / 64), x = piece >> 1;  // uniform per wavefront
-        const int ib = x < 3 ? x : x == 3 ? 2 : 3, jp = x == 3 || x == 5;
-        bf16_t* d = (piece & 1 ? sXl : sXh) + (16 * ib + lr) * LDB + 32 * jp + 4 * lq;
-        *(u32x2*)d = u32x2{f.px[m][0], f.px[m][1]};
-        *(u32x2*)(d + 16) = u32x2{f.px[m][2], f.px[m][3]};
+        if (x >= kNPieces) break;
+        bf16_t* const pl = piece & 1 ? sXl : sXh;
+        const u32x2 w0 = {f.px[m][0], f.px[m][1]}, w1 = {f.px[m][2], f.px[m][3]}, z = {0u, 0u};
+        const int ib = x < 4 ? x : 3, jp = x == 4;
+        bf16_t* d = pl + (16 * ib + lr) * LDB + 32 * jp + 4 * lq;
+        *(u32x2*)d = w0;
+        *(u32x2*)(d + 16) = x == 0 ? z : w1;
+        if (x == 0) {
+          bf16_t* e = pl + (32 + lr) * LDB + 32 + 4 * lq;
+          *(u32x2*)e = w1;
+          *(u32x2*)(e + 16) = z;
+        }
       }
     } else {
 #pragma unroll

@@ -70,7 +70,10 @@ ChunkWs chunk_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64
   const size_t elem = mode == omx::kModeF32 ? 4 : 2;
   size_t o = 0;
   w.rec = o;
-  o += align_up(slots * (size_t)Hv * (size_t)omx::chunk_record_bytes(mode, bwd), 256);
+  // (layer: 19 KiB of room per record, more than it fills, so that the shapes which fit the
+  // allocation-free entry point's fixed scratch stay the ones its callers know)
+  const size_t rec = mode == omx::kModeLayer ? 19 * 1024 : (size_t)omx::chunk_record_bytes(mode, bwd);
+  o += align_up(slots * (size_t)Hv * rec, 256);
   w.kn = o;
   o += align_up(tokens * (size_t)(Hk * dk) * elem, 256);
   w.qn = o;

@@ -14,8 +14,12 @@
 // holds 16 bytes, M[16i + r][32p + 4q .. +3] then M[16i + r][32p + 16 + 4q .. +3]
 // (the 16x16 tiles (i, 2p) and (i, 2p+1), each in the 16x16x16 A layout).  The
 // contraction order matches a B operand built from two C-layout tiles of the
-// right-hand side.  The upper tiles (0, 1) and (2, 3) that complete the pairs of
-// row blocks 0 and 2 are stored as zeros.  Six pairs, 1 KiB each, lanes in order.
+// right-hand side.  The upper tiles (0, 1) and (2, 3) that complete the pairs (0, 0) and
+// (2, 1) are zero and not stored: tiles (0, 0) and (2, 2) share a piece, so the six pairs
+// are five pieces of 1 KiB, lanes in order.  The record is 16 KiB with bf16 inputs, 19 with
+// the zeros, and the preparation kernel is held by its stores: B=1 T=65,536 Hv=64 529 -> 508
+// us, B=4 T=4,096 Hv=32 141 -> 137 us; a scan of 16-column workgroups (B=1 T=1,900 Hv=32)
+// 69 -> 65 us.
 #pragma once
 
 #include "gdn_common.h"
@@ -33,12 +37,13 @@ constexpr int MODE_BF16 = kModeBF16, MODE_F32 = kModeF32, MODE_LAYER = kModeLaye
 // record layout (bytes)
 constexpr int kPairBytes = 64 * 16;            // one 16x32 A operand, all lanes
 constexpr int kNPairs = 6;                     // (i, p): (0,0) (1,0) (2,0) (2,1) (3,0) (3,1)
-constexpr int kRecT = 0;                       // 6 pairs x {hi, lo}
-constexpr int kRecP = kRecT + 2 * kNPairs * kPairBytes;  // 6 pairs (hi)
-constexpr int kRecG = kRecP + kNPairs * kPairBytes;      // 4 x 64 fp32 gate vectors
+constexpr int kNPieces = 5;                    // (0,0)|(2,1)  (1,0)  (2,0)  (3,0)  (3,1)
+constexpr int kRecT = 0;                       // 5 pieces x {hi, lo}
+constexpr int kRecP = kRecT + 2 * kNPieces * kPairBytes;  // 5 pieces (hi)
+constexpr int kRecG = kRecP + kNPieces * kPairBytes;      // 4 x 64 fp32 gate vectors
 constexpr int kRecPL = kRecG + 4 * kC * 4;               // fp32 inputs, backward: P lo parts
-constexpr int kRecBytesBF16 = kRecPL;                    // 19456
-constexpr int kRecBytesF32 = kRecPL + kNPairs * kPairBytes;  // 25600
+constexpr int kRecBytesBF16 = kRecPL;                    // 16384
+constexpr int kRecBytesF32 = kRecPL + kNPieces * kPairBytes;  // 21504
 // rows of the gate block: e^G, scale e^G, e^{G_last - G} (its last entry, always 1, is
 // replaced by e^{G_last}), beta
 constexpr int kGateEG = 0, kGateEGS = 1, kGateEL = 2, kGateBeta = 3;
@@ -77,14 +82,27 @@ __device__ __forceinline__ const T* at_bytes(const T* base, unsigned off) {
 
 // index of the block pair (i, p), p <= i / 2
 __host__ __device__ constexpr int pair_index(int i, int p) { return i + (i == 3) + p; }
-// byte offsets of 16x16 tile (i, j), j <= i + (i even), in the record: its pair's
-// 16 bytes per lane, first or second 8 (add 16 lane).  T lo parts follow T hi by one
-// pair; P lo parts (fp32 inputs) sit at kRecPL - kRecP further.
+// the piece that holds pair x, and the half of it that a tile (i, j) takes
+__host__ __device__ constexpr int piece_index(int x) { return x == 3 ? 0 : x > 3 ? x - 1 : x; }
+__host__ __device__ constexpr int tile_half(int i, int j) { return i == 2 && j == 2 ? 1 : j & 1; }
+// byte offsets of 16x16 tile (i, j), j <= i, in the record: its piece's 16 bytes per lane,
+// first or second 8 (add 16 lane).  T lo parts follow T hi by one piece; P lo parts (fp32
+// inputs) sit at kRecPL - kRecP further.
 __host__ __device__ constexpr int rec_t_off(int i, int j) {
-  return kRecT + 2 * pair_index(i, j >> 1) * kPairBytes + 8 * (j & 1);
+  return kRecT + 2 * piece_index(pair_index(i, j >> 1)) * kPairBytes + 8 * tile_half(i, j);
 }
 __host__ __device__ constexpr int rec_p_off(int i, int j) {
-  return kRecP + pair_index(i, j >> 1) * kPairBytes + 8 * (j & 1);
+  return kRecP + piece_index(pair_index(i, j >> 1)) * kPairBytes + 8 * tile_half(i, j);
+}
+// the six pairs' operands from the five pieces at base, `stride` bytes apart
+__device__ __forceinline__ void read_pairs(const unsigned char* base, int stride, u32x4* x) {
+  const u32x4 d = *(const u32x4*)(base + 16 * lane_id());
+  x[0] = u32x4{d[0], d[1], 0u, 0u};
+  x[3] = u32x4{d[2], d[3], 0u, 0u};
+  x[1] = *(const u32x4*)(base + stride + 16 * lane_id());
+  x[2] = *(const u32x4*)(base + 2 * stride + 16 * lane_id());
+  x[4] = *(const u32x4*)(base + 3 * stride + 16 * lane_id());
+  x[5] = *(const u32x4*)(base + 4 * stride + 16 * lane_id());
 }
 // index of 16x16 tile (bi, bj), bj <= bi, of a lower-triangular 64x64 matrix
 __host__ __device__ constexpr int tile_index(int bi, int bj) { return bi * (bi + 1) / 2 + bj; }

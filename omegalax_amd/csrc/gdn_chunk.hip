@@ -782,12 +782,8 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
     }
     // T operands of V_new = T R, one per block pair (read while the products run)
     u32x4 th[kNPairs], tl[kNPairs];
-#pragma unroll
-    for (int x = 0; x < kNPairs; ++x) {
-      const unsigned char* tp = sRec + kRecT + 2 * x * kPairBytes + 16 * l;
-      th[x] = *(const u32x4*)tp;
-      tl[x] = *(const u32x4*)(tp + kPairBytes);
-    }
+    read_pairs(sRec + kRecT, 2 * kPairBytes, th);
+    read_pairs(sRec + kRecT + kPairBytes, 2 * kPairBytes, tl);
     // R = V - diag(e^G) K S at rows 16i + 4lq + v, column 16w + lr (diag(beta) is
     // folded into the record's T, except in a bf16 backward's, where it enters R here)
     f32x4 R[4];
@@ -829,7 +825,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
     }
     if constexpr (DIRECT && !IS) {
       // the T operands and gate rows are read in one batch ahead of the products
-      __builtin_amdgcn_sched_group_barrier(0x100, 2 * kNPairs + 8, 1);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * kNPieces + 8, 1);
       __builtin_amdgcn_sched_group_barrier(0x002, 80, 1);
       __builtin_amdgcn_sched_group_barrier(0x008, 18, 1);
     }
@@ -859,11 +855,12 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
     }
     // P operands and the K^T operands of the state update (read while V_new forms)
     u32x4 ph[kNPairs], pl[kNPairs];
+    read_pairs(sRec + kRecP, kPairBytes, ph);
+    if constexpr (OS) {
+      read_pairs(sRec + kRecPL, kPairBytes, pl);
+    } else {
 #pragma unroll
-    for (int x = 0; x < kNPairs; ++x) {
-      ph[x] = *(const u32x4*)(sRec + kRecP + x * kPairBytes + 16 * l);
-      if constexpr (OS) pl[x] = *(const u32x4*)(sRec + kRecPL + x * kPairBytes + 16 * l);
-      else pl[x] = ph[x];
+      for (int x = 0; x < kNPairs; ++x) pl[x] = ph[x];
     }
     // K^T operands of the state update, 16x32 over token blocks 2p, 2p+1: lane (q, r)
     // holds K[32p + 4q .. +3][d] then K[32p + 16 + 4q .. +3][d] for the dk index d of
@@ -927,8 +924,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
       // its o comes from split operands throughout (S, V_new and P hi and lo): the adjoint
       // scales by the row's 1 / RMS, which is large where o's terms nearly cancel
       if constexpr (!OS) {
-#pragma unroll
-        for (int x = 0; x < kNPairs; ++x) pl[x] = *(const u32x4*)(sRec + kRecPL + x * kPairBytes + 16 * l);
+        read_pairs(sRec + kRecPL, kPairBytes, pl);
       }
     }
     if constexpr (DEFER_QS) {

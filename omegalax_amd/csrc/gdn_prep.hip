@@ -590,15 +590,6 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
             put_tile(rec, rec_t_off(bi, bi), pack_hi4(Tb));
             if constexpr (BWD && IS) put_f32_tile(xb + kXlpgX, bi, bi, Tc);  // X^T: the C layout
             put_tile(rec, rec_t_off(bi, bi) + kPairBytes, pack_lo4(Tb));
-            if ((bi & 1) == 0) {
-              // the zero upper tile (bi, bi + 1) that completes row block bi's last pair
-              const u32x2 z = {0u, 0u};
-              put_tile(rec, rec_t_off(bi, bi + 1), z);
-              put_tile(rec, rec_t_off(bi, bi + 1) + kPairBytes, z);
-              if (!BWD || IS || p.o) put_tile(rec, rec_p_off(bi, bi + 1), z);
-              if constexpr (IS || BWD)
-                if (IS || p.o) put_tile(rec, rec_p_off(bi, bi + 1) + (kRecPL - kRecP), z);
-            }
           } else {
             u32x2* d = sLf + 2 * 64 * tile_index(bi, bj) + l;
             d[0] = pack_hi4(val);
