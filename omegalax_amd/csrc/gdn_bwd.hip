@@ -363,7 +363,7 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool loader = LDR && wave >= NWC;      // (LDR) the last four: rows and P tiles only
   const int st = loader ? tid - 64 * NWC : tid;  // index among the NT threads that stage rows
-  const ScanItem item = scan_item(p.seq_order, p.N, p.Hk, p.Hv, p.nb);
+  const ScanItem item = scan_item(p.seq_order, p.N, p.Hk, p.Hv, p.nb, blockIdx.x);
   const int blk = item.blk, h = item.h, n = item.n;
   const int gqa = p.Hv / p.Hk, hk = h / gqa;
   const int DV = p.DV, col0 = BV * blk, c = 16 * wave;

@@ -58,7 +58,7 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 // sums of o^2 for the gated norm, and the plan of packed sequences (chunk offsets and
 // the ordered copy of cu_seqlens the kernels read).
 struct ChunkWs {
-  size_t rec, kn, qn, vc, opart, oss, xch, off, cu, ord, total;
+  size_t rec, tickets, kn, qn, vc, opart, oss, xch, off, cu, ord, total;
 };
 
 ChunkWs chunk_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64_t dv, int64_t N,
@@ -71,9 +71,11 @@ ChunkWs chunk_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64
   size_t o = 0;
   w.rec = o;
   // (layer: 19 KiB of room per record, more than it fills, so that the shapes which fit the
-  // allocation-free entry point's fixed scratch stay the ones its callers know)
-  const size_t rec = mode == omx::kModeLayer ? 19 * 1024 : (size_t)omx::chunk_record_bytes(mode, bwd);
-  o += align_up(slots * (size_t)Hv * rec, 256);
+  // allocation-free entry point's fixed scratch stay the ones its callers know; the scan's
+  // tickets take 32 bytes of the rest)
+  const size_t rec = (size_t)omx::chunk_record_bytes(mode, bwd);
+  w.tickets = align_up(slots * (size_t)Hv * rec, 256);
+  o += align_up(slots * (size_t)Hv * (mode == omx::kModeLayer ? 19 * 1024 : rec), 256);
   w.kn = o;
   o += align_up(tokens * (size_t)(Hk * dk) * elem, 256);
   w.qn = o;
@@ -356,6 +358,7 @@ void setup_chunked(omx::ChunkParams& p, const ChunkWs& ws, void* workspace, int 
     p.vs_ld = (long long)p.Hv * p.DV;
     p.ss_xch = (unsigned*)(base + ws.xch);
     p.ss_xch_slots = omx::layer_scan_blocks(p);
+    p.tickets = (int*)(base + ws.tickets);
   } else {
     p.vs = p.v;
     p.vs_ld = p.v_ld;

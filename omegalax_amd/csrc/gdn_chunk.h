@@ -234,9 +234,9 @@ __device__ __forceinline__ void seq_range(const int32_t* cu, int n, int T, long 
 }
 
 // Work item of a workgroup of the scans (forward and reverse): sequence n, value head h
-// and column block blk, from blockIdx.x.  The workgroups of one key head of one sequence
-// (gqa value heads x nb blocks, which read the same q/k rows) form a group that runs on
-// one XCD (the hardware deals workgroup i to XCD i % 8), so they share its L2.  When the
+// and column block blk, from index b (blockIdx.x, or the place a ticket gives).  The
+// workgroups of one key head of one sequence (gqa value heads x nb blocks, which read the
+// same q/k rows) form a group that runs on one XCD (the hardware deals workgroup i to XCD i % 8), so they share its L2.  When the
 // group count is a multiple of 8, group ranks are dealt round-robin over the XCDs in the
 // order of `order` (sequences longest first; null = index order): every XCD gets a share
 // of every sequence and starts its longest chains first.  Otherwise each XCD takes a
@@ -245,9 +245,9 @@ struct ScanItem {
   int n, h, blk;
 };
 __device__ __forceinline__ ScanItem scan_item(const int32_t* order, int N, int Hk, int Hv,
-                                              int nb) {
+                                              int nb, unsigned b) {
   const int gqa = Hv / Hk, G = gqa * nb, NG = N * Hk;
-  const unsigned b = blockIdx.x, xcd = b % 8, slot = b / 8;
+  const unsigned xcd = b % 8, slot = b / 8;
   int grp, member;
   if (NG % 8 == 0) {
     grp = 8 * (int)(slot / G) + (int)xcd;

@@ -477,10 +477,27 @@ __device__ __forceinline__ void put_vr(const ChunkParams& p, const VRRegs<MODE, 
   }
 }
 
+// The place of a workgroup in a grid larger than the chip: the next free one of its XCD's
+// eighth of the grid (places congruent to the XCD's number mod 8, which scan_item gives whole
+// groups in order), or of another's when that is used up.  Tickets follow the order in which
+// workgroups start, whatever the hardware's dispatch order is, and a value head's column
+// blocks are consecutive places of one eighth.  So at any time at most one value head per
+// eighth has started blocks that wait for blocks not yet started; every other started
+// workgroup can finish, and the ones to come take the missing places.
+__device__ __forceinline__ unsigned take_ticket(int* tickets, unsigned per) {
+  const unsigned xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7u;  // HW_REG_XCC_ID
+  for (unsigned k = 0; k < 8; ++k) {
+    const unsigned x = (xcc + k) & 7u;
+    const unsigned t = (unsigned)__hip_atomic_fetch_add(tickets + x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t < per) return 8u * t + x;
+  }
+  return 0;  // not reached: there are as many places as workgroups
+}
+
 // BWD (the backward pass's recompute): stores the state entering every chunk and V_new,
 // and o only when p.o is set.
 //
-// FUSE (layer, direct loads, a grid the chip holds in one round): the gated RMSNorm
+// FUSE (layer, direct loads): the gated RMSNorm
 // (deltanet.py:282-293) is applied here and the scan writes the layer's output.  A row of
 // o spans the nb workgroups of a value head (its column blocks), so its statistic needs
 // their partial sums: each workgroup's loader publishes its rows' partial (the fp32 o's
@@ -490,9 +507,10 @@ __device__ __forceinline__ void put_vr(const ChunkParams& p, const VRRegs<MODE, 
 // epilogue kernel uses and leaves 1/RMS per row in LDS.  Meanwhile the compute
 // wavefronts keep their bf16 o rows in a four-chunk LDS ring and, three steps after the
 // chunk, normalise and gate them: w (o rsqrt(mean + eps)) silu(z), the epilogue kernel's
-// arithmetic, so the output is bit-identical to the unfused path's.  Every workgroup of
-// the grid is resident at once, so a wait for another block's flag ends; it is bounded
-// all the same.
+// arithmetic, so the output is bit-identical to the unfused path's.  A wait for another
+// block's flag ends because every block it waits for runs: in a grid the chip holds at once
+// all of them are resident; in a larger one each workgroup takes its place from a ticket as
+// it starts (take_ticket).  The wait is bounded all the same.
 template <int DK, int MODE, bool BWD = false, int NWC_ = 4, bool FUSE = false>
 // One workgroup per CU is the design point (the state fills the register file): the
 // compiler may use the whole file (half of it with a loader wavefront, which shares a
@@ -553,7 +571,16 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
   const bool compute = wave < NWC;             // owns 16 state columns
   // XCD-aware work item (scan_item): a key head's workgroups share one XCD's L2, and
   // packed sequences start longest first
-  const ScanItem item = scan_item(p.seq_order, p.N, p.Hk, p.Hv, p.nb);
+  unsigned place = blockIdx.x;
+  if constexpr (FUSE) {
+    __shared__ unsigned sPlace;
+    if (p.tickets) {  // uniform
+      if (tid == 0) sPlace = take_ticket(p.tickets, gridDim.x / 8);
+      __syncthreads();
+      place = __builtin_amdgcn_readfirstlane(sPlace);
+    }
+  }
+  const ScanItem item = scan_item(p.seq_order, p.N, p.Hk, p.Hv, p.nb, place);
   const int blk = item.blk, h = item.h, n = item.n;
   const int gqa = p.Hv / p.Hk;
   const int hk = h / gqa;
@@ -1381,6 +1408,7 @@ hipError_t launch_scan_cfg(const ChunkParams& p, hipStream_t stream) {
   // loads, else one per wavefront
   q.ss_slots = Q_::DIRECT ? q.nb : p.DV / 16;
   const unsigned grid = (unsigned)(q.N * q.Hv * q.nb);
+  if (grid <= (unsigned)device_cus()) q.tickets = nullptr;  // all resident: place = blockIdx.x
   hipLaunchKernelGGL((scan_kernel<DK, MODE, BWD, NWC, FUSE>), dim3(grid), dim3(Q_::NTH), 0, stream, q);
   return hipGetLastError();
 }
@@ -1433,14 +1461,22 @@ int layer_scan_blocks(const ChunkParams& p) {
   return p.DV / (16 * scan_tiles_per_wg(p));
 }
 
-// The layer scan applies the gated norm itself (FUSE) when it loads directly (dk = 128),
-// the exchange array is there and its grid is one round of the chip: at one workgroup per
-// CU (the scan's LDS), every workgroup is then resident together, so the waits for the
-// other column blocks' partials end.
+// The layer scan applies the gated norm itself (FUSE) when it loads directly (dk = 128), the
+// exchange array is there, and the waits for the other column blocks' partials end: its grid
+// is one round of the chip (one workgroup per CU: the scan's LDS), or tickets can order a
+// larger one: the groups divide over the eight XCDs, and a value head has few enough blocks
+// that those waiting for partners not yet started, at most blocks - 1 of each of eight
+// eighths, cannot fill an XCD's 32 CUs.  The larger grid's workgroups each end with the
+// exchange's drain, the smaller one's once for all: from eight chunks a sequence the saved
+// pass over o outweighs it (and the prep, which clears the tickets, has work).  Scan and
+// epilogue -> fused scan, Hk=16 Hv=32 d=128: 8 documents of 32,768 tokens 543 -> 502 us;
+// B=16 T=500 153 -> 140 us; 6 documents of 4,096 tokens (Hv=64) 146 -> 147 us; one chunk a
+// sequence (B=64 T=64) 154 -> 182 us, which stays with the epilogue kernel.
 bool layer_scan_fuses_norm(const ChunkParams& p) {
   if (!p.ss_xch || !layer_v_in_scan(p.dk)) return false;
   const long long grid = (long long)p.N * p.Hv * layer_scan_blocks(p);
-  return grid <= device_cus();
+  if (grid <= device_cus()) return true;
+  return (long long)p.N * p.Hk % 8 == 0 && layer_scan_blocks(p) <= 4 && p.n_rec >= 8LL * p.N;
 }
 
 int layer_ss_slots(const ChunkParams& p) {

@@ -63,6 +63,7 @@ struct ChunkParams {
   void* o_part;                // unnormalised o [tokens, Hv, DV] bf16 (workspace)
   float* o_ss;                 // [ceil(tokens / 64), Hv, ss_slots, 64] fp32 (workspace):
                                // partial sums of squares of the fp32 o over a row
+  int* tickets;                // (layer) 8 counters, cleared by the prep (see take_ticket)
   int ss_slots;                // partials per (token, head) row (set by the scan's launcher)
   // (layer, scan with the gated norm fused) the workgroups' row partials of recent chunks,
   // [N][Hv][ss_xch_slots][kXchRing][64] pairs {fp32 bits, tag}: chunk c of a sequence uses

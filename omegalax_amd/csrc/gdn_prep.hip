@@ -281,6 +281,8 @@ __global__ __launch_bounds__(NT, (prep_blocks_per_cu<DK, MODE>())) void prep_ker
   const int n_ci = p.chunk_off ? uniform_ld(p.chunk_off, p.N) : p.n_rec;
   const int total = n_ci * p.Hk;
   const int task = (int)blockIdx.x / parts, part = (int)blockIdx.x % parts;
+  if constexpr (MODE == MODE_LAYER)
+    if (blockIdx.x == 0 && tid < 8) p.tickets[tid] = 0;
   if (task >= total) return;  // uniform
 
   PrepIn<DK, MODE> pf;
