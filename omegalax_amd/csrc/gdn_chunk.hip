@@ -109,9 +109,9 @@ struct Cfg {
   static constexpr bool LSTAGE = !DIRECT && 2 * BUF <= 160 * 1024;
   static constexpr int NL = DIRECT ? ((MODE == MODE_BF16 && BWD_) || NWC_ < 4 ? 2 : 1) : (LSTAGE ? NST / 64 : 0);
   // (layer, 16 and 32 columns) one more wavefront stores or (FUSE) exchanges the rows'
-  // partial sums, so that the loaders wait for nothing but their rows, and (FUSE) one
-  // normalises the finished chunks
-  static constexpr bool XWAVE = VCONV && NWC_ < 4, FWAVE = XWAVE && FUSE_;
+  // partial sums, so that the loaders wait for nothing but their rows; (FUSE) one
+  // normalises finished chunks, in 64-column workgroups half of their rows
+  static constexpr bool XWAVE = VCONV && NWC_ < 4, FWAVE = VCONV && FUSE_;
   static constexpr int NTH = NT + 64 * (NL + NH + XWAVE + FWAVE);
   static constexpr int WPE = (NTH / 64 + 3) / 4;
   static constexpr int NBUF = DIRECT || LSTAGE ? 2 : 1;
@@ -542,8 +542,8 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
   constexpr bool XW = Q_::XWAVE, FW = Q_::FWAVE;
   // (FUSE) chunks of bf16 o kept per compute wavefront: with a finalizing wavefront a chunk
   // is read while a later one is written
-  constexpr int kRing = FW ? 8 : 4;
-  constexpr int kFin = FW ? 4 : 3;  // (FUSE) steps from a chunk to its normalisation
+  constexpr int kRing = FW && XW ? 8 : 4;
+  constexpr int kFin = FW && XW ? 4 : 3;  // (FUSE) steps from a chunk to its normalisation
   static_assert(kFin < kRing, "a chunk is normalised before its ring entry is rewritten");
   // (FUSE) lane l's 4 x 4 bf16 o values of row block i of chunk c, wave w: sO[c % 4][w][i][l]
   __shared__ __align__(16) u32x2 sO[FUSE ? kRing : 1][FUSE ? NWC : 1][FUSE ? 4 : 1][64];
@@ -566,6 +566,8 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
     hw = NWC == 1 ? (wave == 3 ? 0 : wave == 5 ? 1 : -1) : (wave == 2 || wave == 3 ? wave - 2 : -1);
     xwave = wave == 4;
     fwave = FW && wave == 5 + NWC;
+  } else if constexpr (FW) {
+    fwave = wave == NWC + Q_::NL + Q_::NH;
   }
   const bool loader = lw >= 0, helper = hw >= 0;
   const bool compute = wave < NWC;             // owns 16 state columns
@@ -640,57 +642,68 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
   // the step; out = w (o rn) silu(z), stored through a buffer whose range ends at the
   // chunk's last valid row.  The row offsets are in the lane offsets, which the range
   // check covers (a scalar offset is not relied on to be checked).  c < 0 does nothing.
-  // (FW: on the finalizing wavefront, for the NWC compute wavefronts' columns)
+  // FW: the compute wavefronts normalise row tiles 0 .. FH - 1 of their own columns, the
+  // finalizing wavefront the others, of all NWC column slices.  Narrow workgroups leave it
+  // all tiles; with four slices those would outlast the step (B=4 T=4,096 Hv=32 d=128: 257
+  // us with all four row tiles, 234 with three, 233 with two, 239 with one, 242 without the
+  // wavefront; 8 documents of 32,768 tokens 490 with two, 498 without).
+  constexpr int FH = !FUSE ? 0 : !FW ? 4 : XW ? 0 : 2;
   constexpr int NF = FW ? NWC : 1;
   u32x2 zf[NF][4];
   float4 nw4[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f)
-    nw4[f] = FUSE && (!FW || fwave) ? *(const float4*)(p.norm_w + col0 + 16 * (FW ? f : wave) + 4 * lq)
-                                    : make_float4(0.f, 0.f, 0.f, 0.f);
-  // element offset of row lr, columns 4 lq .. +3 of compute wavefront f's slice
-  auto f_elem = [&](int f) { return (unsigned)lr * o_rs + 16u * (FW ? f : wave) + 4u * lq; };
+    nw4[f] = FUSE && (fwave || (FH > 0 && f == 0 && compute))
+                 ? *(const float4*)(p.norm_w + col0 + 16 * (fwave ? f : wave) + 4 * lq)
+                 : make_float4(0.f, 0.f, 0.f, 0.f);
   auto chunk_rows = [&](int c, long long& tc) {
     tc = s0 + (long long)c * C;
     return (int)((s1 - tc) < C ? (s1 - tc) : C);
   };
-  auto z_load = [&](int c) {
-    if constexpr (FUSE) {
+  // slice f (the finalizing wavefront's: fin) or the compute wavefront's own, row tiles i0 ..
+  // i1 - 1; lane: row lr, columns 4 lq .. +3 of the slice
+  auto z_load = [&](int c, auto fin) {
+    constexpr int i0 = fin.value ? FH : 0, i1 = fin.value ? 4 : FH, nf = fin.value ? NF : 1;
+    if constexpr (FUSE && i0 < i1) {
       if (c < 0) return;  // uniform
       long long tc;
       const int nvc = chunk_rows(c, tc);
       const auto zr = buf_rsrc((const bf16_t*)p.z + (tc * p.Hv + h) * (long long)DV + col0,
                                2u * nvc * o_rs);
 #pragma unroll
-      for (int f = 0; f < NF; ++f)
+      for (int f = 0; f < nf; ++f)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          zf[f][i] = __builtin_amdgcn_raw_buffer_load_b64(zr, 2u * (f_elem(f) + 16u * i * o_rs), 0, 0);
+        for (int i = i0; i < i1; ++i)
+          zf[f][i] = __builtin_amdgcn_raw_buffer_load_b64(
+              zr, 2u * ((unsigned)lr * o_rs + 16u * (fin.value ? f : wave) + 4u * lq + 16u * i * o_rs), 0, 0);
     }
   };
-  auto finalize = [&](int c) {
-    if constexpr (FUSE) {
+  auto finalize = [&](int c, auto fin) {
+    constexpr int i0 = fin.value ? FH : 0, i1 = fin.value ? 4 : FH, nf = fin.value ? NF : 1;
+    if constexpr (FUSE && i0 < i1) {
       if (c < 0) return;  // uniform
       long long tc;
       const int nvc = chunk_rows(c, tc);
       const auto orr = buf_rsrc((bf16_t*)p.out + (tc * p.Hv + h) * (long long)DV + col0,
                                 2u * nvc * o_rs);
 #pragma unroll
-      for (int f = 0; f < NF; ++f)
+      for (int f = 0; f < nf; ++f)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float w[4] = {nw4[f].x, nw4[f].y, nw4[f].z, nw4[f].w};
-        const u32x2 ow = sO[c % kRing][FW ? f : wave][i][l];
-        const float rn = sRN[c & 1][16 * i + lr];
-        uint32_t r[2];
+        for (int i = i0; i < i1; ++i) {
+          const int sl = fin.value ? f : wave;
+          const float w[4] = {nw4[f].x, nw4[f].y, nw4[f].z, nw4[f].w};
+          const u32x2 ow = sO[c % kRing][sl][i][l];
+          const float rn = sRN[c & 1][16 * i + lr];
+          uint32_t r[2];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const float o0 = __uint_as_float(ow[e] << 16), o1 = __uint_as_float(ow[e] & 0xffff0000u);
-          const float z0 = __uint_as_float(zf[f][i][e] << 16), z1 = __uint_as_float(zf[f][i][e] & 0xffff0000u);
-          r[e] = pack_bf16(w[2 * e] * (o0 * rn) * silu_fast(z0), w[2 * e + 1] * (o1 * rn) * silu_fast(z1));
+          for (int e = 0; e < 2; ++e) {
+            const float o0 = __uint_as_float(ow[e] << 16), o1 = __uint_as_float(ow[e] & 0xffff0000u);
+            const float z0 = __uint_as_float(zf[f][i][e] << 16), z1 = __uint_as_float(zf[f][i][e] & 0xffff0000u);
+            r[e] = pack_bf16(w[2 * e] * (o0 * rn) * silu_fast(z0), w[2 * e + 1] * (o1 * rn) * silu_fast(z1));
+          }
+          __builtin_amdgcn_raw_buffer_store_b64(
+              u32x2{r[0], r[1]}, orr, 2u * ((unsigned)lr * o_rs + 16u * sl + 4u * lq + 16u * i * o_rs), 0, 0);
         }
-        __builtin_amdgcn_raw_buffer_store_b64(u32x2{r[0], r[1]}, orr, 2u * (f_elem(f) + 16u * i * o_rs), 0, 0);
-      }
     }
   };
 
@@ -710,7 +723,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
         if (j >= 1) sSS[(j - 1) & 1][wave][16 * lq + lr] = ss_prev;
       }
       // (FUSE) z of the chunk normalised at the end of this step, in flight meanwhile
-      if constexpr (FUSE && !FW) z_load(j - kFin);
+      z_load(j - kFin, std::false_type{});
     } else if constexpr (LSTAGE) {
       // the loaders have stored chunk j, and chunk j-1, the last reader of the other set,
       // is finished everywhere
@@ -1013,7 +1026,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
       for (int i = 0; i < 4; ++i)
         sO[j % kRing][wave][i][l] = u32x2{pack_bf16(o[i][0], o[i][1]), pack_bf16(o[i][2], o[i][3])};
       sSS[j & 1][wave][16 * lq + lr] = row_sq_scatter(o);
-      if constexpr (!FW) finalize(j - kFin);
+      finalize(j - kFin, std::false_type{});
     } else {
       // unnormalised o in bf16; the epilogue kernel applies the norm, from the fp32 sums
       // of squares stored below
@@ -1247,8 +1260,8 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
       if constexpr (FW) {
         for (int j = 0; nchunks > 0 && j < nchunks + kFin; ++j) {
           lds_barrier();
-          finalize(j - kFin);
-          if (j + 1 < nchunks + kFin) z_load(j + 1 - kFin);
+          finalize(j - kFin, std::true_type{});
+          if (j + 1 < nchunks + kFin) z_load(j + 1 - kFin, std::true_type{});
         }
       }
     } else if (helper) {
@@ -1310,10 +1323,8 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
         if (nchunks > 0)
           for (int j = nchunks; j < nchunks + kFin; ++j) {
             lds_barrier();
-            if constexpr (!FW) {
-              z_load(j - kFin);
-              finalize(j - kFin);
-            }
+            z_load(j - kFin, std::false_type{});
+            finalize(j - kFin, std::false_type{});
           }
       } else if constexpr (WG_SS) {  // the loader's two barriers after its loop
         if (nchunks > 0) {
