@@ -327,7 +327,12 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
   static_assert(!F32 || NWC == 4, "fp32 inputs: the four compute wavefronts stage the rows");
   constexpr int BV = 16 * NWC;  // columns of dv per workgroup
   using KT = typename std::conditional<F32, float, bf16_t>::type;
-  constexpr int LDK = DK + (F32 ? 4 : 8);
+  // bf16 rows of 128 lie in the scans' swizzled layout, others padded by 16 bytes.  Padded,
+  // half of the LDS's busy cycles were conflicts (the transposed reads four ways, each
+  // 16-byte pass one; now 14M of 54M cycles for 40M of 81M): C1 317 -> 307 us, layer rows at
+  // B=1 T=3,001 Hv=32 110.5 -> 107.
+  constexpr bool SWZ = !F32 && DK == 128;
+  constexpr int LDK = SWZ ? DK : DK + (F32 ? 4 : 8);
   constexpr int LDB = C + 8;  // stride (bf16) of a split plane
   constexpr bool LDR = !F32;
   // bf16 inputs form the P operands in registers (PREC) from the staged K and Q rows and G
@@ -468,7 +473,7 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
       const int it = st + m * NT;
       const int which = it / (C * DK / 4), rem = it % (C * DK / 4);
       const int row = rem / (DK / 4), c4 = 4 * (rem % (DK / 4));
-      store4((which ? bf.Q : bf.K) + row * LDK + c4, f.pkq[m]);
+      store4((which ? bf.Q : bf.K) + (SWZ ? swz_off<128>(row, c4) : row * LDK + c4), f.pkq[m]);
     }
 #pragma unroll
     for (int m = 0; m < C * BV / 4 / NT; ++m) {
@@ -510,6 +515,25 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
       if (st < C) bf.Gl[st] = f.pg;
     bf.Gate[st] = f.pgate;
   };
+  // kq_row and kq_st on the staged K and Q rows
+  auto k_row = [&](const auto* m, int r0, int k0) {
+    if constexpr (SWZ) {
+      Op o;
+      o.h = o.l = swz_frag(m, r0, k0);
+      return o;
+    } else {
+      return kq_row<false>(m, LDK, r0, k0);
+    }
+  };
+  auto k_st = [&](const auto* m, int t, int k0) {
+    if constexpr (SWZ) {
+      Op o;
+      o.h = o.l = join(kt_rows4_swz(m, k0, t), kt_rows4_swz(m, k0 + 16, t));
+      return o;
+    } else {
+      return kq_st(m, LDK, t, k0);
+    }
+  };
   // (LDR) tile (mb, nb) of P = lower(scale Q K^T * Gamma) in the C layout, from the rows
   // staged in bf, with the preparation kernel's arithmetic:
   // scale * acc * 2^{min(G_m log2 e - G_n log2 e, 0)} * mask
@@ -517,8 +541,7 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
     f32x4 acc = zero4();
 #pragma unroll
     for (int s2 = 0; s2 < DK / 32; ++s2)
-      acc = mma16(frag_bf16((const bf16_t*)bf.Q, LDK, 16 * mb, 32 * s2),
-                  frag_bf16((const bf16_t*)bf.K, LDK, 16 * nb, 32 * s2), acc);
+      acc = mma16(k_row((const bf16_t*)bf.Q, 16 * mb, 32 * s2).h, k_row((const bf16_t*)bf.K, 16 * nb, 32 * s2).h, acc);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int m = 16 * mb + 4 * lq + v, n = 16 * nb + lr;
@@ -587,7 +610,7 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
 #pragma unroll
     for (int s = 0; s < DK / 32; ++s)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) kds[i] = mm3<F32, true>(kds[i], kq_row<false>(sK, LDK, 16 * i, 32 * s), dsb[s]);
+      for (int i = 0; i < 4; ++i) kds[i] = mm3<F32, true>(kds[i], k_row(sK, 16 * i, 32 * s), dsb[s]);
 #pragma unroll
     for (int p2 = 0; p2 < 2; ++p2) {
       float x[8];
@@ -647,7 +670,7 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
 #pragma unroll
       for (int v = 0; v < 4; ++v) dS[t][v] *= egl;
 #pragma unroll
-      for (int p2 = 0; p2 < 2; ++p2) dS[t] = mm3<F32, true>(dS[t], kq_st(sQ, LDK, t, 32 * p2), b1[p2]);
+      for (int p2 = 0; p2 < 2; ++p2) dS[t] = mm3<F32, true>(dS[t], k_st(sQ, t, 32 * p2), b1[p2]);
     }
     __builtin_amdgcn_sched_barrier(0);
     // ---------------------------------------------------------------- dR = X^T dV_new, Y = diag(beta) dR
@@ -677,7 +700,7 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
 #pragma unroll
     for (int t = 0; t < DK / 16; ++t)
 #pragma unroll
-      for (int p2 = 0; p2 < 2; ++p2) dS[t] = mm3<F32, true>(dS[t], kq_st(sK, LDK, t, 32 * p2), b2[p2]);
+      for (int p2 = 0; p2 < 2; ++p2) dS[t] = mm3<F32, true>(dS[t], k_st(sK, t, 32 * p2), b2[p2]);
 #pragma unroll
     for (int s = 0; s < DK / 32; ++s) dsb[s] = join_op(dS[2 * s], dS[2 * s + 1]);
   };

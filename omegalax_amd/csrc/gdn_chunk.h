@@ -266,4 +266,54 @@ __device__ __forceinline__ ScanItem scan_item(const int32_t* order, int N, int H
   return it;
 }
 
+__device__ __forceinline__ u32x4 join(u32x2 a, u32x2 b) { return u32x4{a[0], a[1], b[0], b[1]}; }
+
+// Swizzled layouts of rows staged in LDS without padding.  A K or Q row (dk = 128) is 16
+// segments of 8 bf16; logical segment g of row r sits at physical segment
+// g ^ swz_k(r).  swz_k is a bijection on 0..15, so the 16 rows of a 16-byte MFMA
+// fragment read hit 16 different segments (all 64 banks).  A pass of that read takes lanes
+// 0-3, 12-15 and 20-27 (and so on), that is, rows 0-3 and 12-15 of one segment with rows
+// 4-11 of its neighbour g ^ 1: the first eight rows' images are closed under ^ 1, so the
+// two halves do not meet.  A pass of the transposed 8-byte read covers four segments of
+// eight rows, one half of each: the images of rows 0..7 (and 8..15) hold each value of the
+// upper two bits twice, the least a read of halves allows.  With images 2 (r & 7) + r / 8,
+// which met in every 16-byte pass, 192 conflict cycles per wavefront and chunk, now 64
+// (counters), and the scans: B=4 T=4,096 Hv=32 236 -> 224 us, 8 documents of 32,768 tokens
+// 479 -> 465, the rule alone at B=1 T=65,536 Hv=64 1,942 -> 1,881.
+// A V row of a 64-column block is 8 segments; swz_v(r) = r & 6
+// makes the 8 rows x 32 bytes of a transposed read pass conflict-free the same way.  Rows
+// of narrower blocks (SV = 4 or 2 segments) keep the bits of r & 6 that index a segment.
+__device__ __forceinline__ int swz_k(int r) {
+  return ((r & 3) << 2) | (((r >> 1) & 2) ^ (((r >> 3) & 1) * 3));
+}
+template <int SV>
+__device__ __forceinline__ int swz_v(int r) { return r & 6 & (SV - 1); }
+
+// element offset of (row, col) in a swizzled buffer with 8-element segments: K / Q rows
+// (128 elements) or V rows (ROWLEN = the block's columns)
+template <int ROWLEN>
+__device__ __forceinline__ int swz_off(int row, int col) {
+  const int g = col >> 3;
+  const int sw = ROWLEN == 128 ? swz_k(row & 15) : swz_v<ROWLEN / 8>(row);
+  return row * ROWLEN + ((g ^ sw) << 3) + (col & 7);
+}
+
+// 16x32 MFMA fragment (rows row0 + lane%16, elements k0 + 8 (lane/16) .. +7)
+__device__ __forceinline__ u32x4 swz_frag(const bf16_t* base, int row0, int k0) {
+  const int l = lane_id();
+  return *(const u32x4*)(base + swz_off<128>(row0 + (l & 15), k0 + 8 * (l >> 4)));
+}
+// The state's row order: row r of state tile t is dk index
+//   32 (t / 2) + 8 (r / 4) + 4 (t % 2) + r % 4,
+// so that tiles 2 s2 and 2 s2 + 1 side by side are the 16x16x32 B operand over dk
+// 32 s2 .. 32 s2 + 31 in natural order.  kt_rows4* read, for the state update, the
+// A operand rows of tile t transposed out of a [token][dk] buffer: lane (q, r) gets
+// tokens row0 + 4q .. +3 of dk column (row r of tile t); source lane s of each
+// 16-lane group points at token row0 + 4q + s/4 and the 4 columns of row group s%4.
+__device__ __forceinline__ int kt_col(int t, int s) { return 32 * (t >> 1) + 4 * (t & 1) + 8 * (s & 3); }
+__device__ __forceinline__ u32x2 kt_rows4_swz(const bf16_t* base, int row0, int t) {
+  const int l = lane_id(), q = l >> 4, s = l & 15;
+  return ds_read_tr(base + swz_off<128>(row0 + 4 * q + (s >> 2), kt_col(t, s)));
+}
+
 }  // namespace omx
