@@ -70,12 +70,12 @@ ChunkWs chunk_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64
   const size_t elem = mode == omx::kModeF32 ? 4 : 2;
   size_t o = 0;
   w.rec = o;
-  // (layer: 19 KiB of room per record, more than it fills, so that the shapes which fit the
-  // allocation-free entry point's fixed scratch stay the ones its callers know; the scan's
-  // tickets take 32 bytes of the rest)
-  const size_t rec = (size_t)omx::chunk_record_bytes(mode, bwd);
-  w.tickets = align_up(slots * (size_t)Hv * rec, 256);
-  o += align_up(slots * (size_t)Hv * (mode == omx::kModeLayer ? 19 * 1024 : rec), 256);
+  // 19 KiB of room per record, 25 with P's lo parts: more than it fills, so that workspace
+  // sizes, and the shapes which fit the allocation-free entry point's fixed scratch, stay the
+  // ones callers know.  The layer scan's tickets take 32 bytes of the rest.
+  const size_t room = (mode == omx::kModeF32 || bwd ? 25 : 19) * 1024;
+  w.tickets = align_up(slots * (size_t)Hv * (size_t)omx::chunk_record_bytes(mode, bwd), 256);
+  o += align_up(slots * (size_t)Hv * room, 256);
   w.kn = o;
   o += align_up(tokens * (size_t)(Hk * dk) * elem, 256);
   w.qn = o;
@@ -119,8 +119,8 @@ BwdWs bwd_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64_t d
   const size_t tokens = (size_t)(B * T);
   const size_t slots = (tokens + 63) / 64 + (size_t)N;
   size_t o = w.f.total;
-  w.xlpg = o;
-  o += align_up(slots * (size_t)Hv * omx::xlpg_floats_host(mode == omx::kModeF32) * 4, 256);
+  w.xlpg = o;  // (room for the matrices with either input precision: sizes callers know)
+  o += align_up(slots * (size_t)Hv * omx::xlpg_floats_host(true) * 4, 256);
   w.states = o;
   o += align_up(slots * (size_t)(Hv * dk * dv) * 4, 256);
   w.dstates = o;
