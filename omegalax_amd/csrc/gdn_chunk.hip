@@ -12,8 +12,8 @@
 //     S    <- e^{G_last} S + K^T diag(e^{G_last - G}) V_new    (:139-142)
 //
 // Work mapping.  One workgroup per (sequence, value head, block of dv columns) walks
-// that sequence's chunks in order; a block is 64 columns (4 compute wavefronts), or on
-// the direct-load path 32 or 16 when 64-column blocks would leave CUs idle.  Wavefront w
+// that sequence's chunks in order; a block is 64 columns (4 compute wavefronts), or,
+// where loader wavefronts stage the rows, 32 or 16 when 64-column blocks would leave CUs idle.  Wavefront w
 // owns state columns [16w, 16w+16) of the block: its fp32 slice S[dk][16] stays in MFMA
 // accumulator registers for the whole sequence, and every product that touches it runs
 // on that wavefront alone.  All products are 16x16x32 MFMAs: the
@@ -23,7 +23,8 @@
 // two C-layout tiles of R or V_new side by side.  With bf16 inputs and dk = 128
 // the next chunk's K, Q, V rows and record are loaded straight into the other of
 // two LDS buffers while the current chunk computes (one workgroup barrier per
-// chunk); otherwise they are staged through registers.  On the layer path with
+// chunk); otherwise they are staged through registers, by loader wavefronts where two sets of
+// buffers fit.  On the layer path with
 // dk = 128 two helper wavefronts form the next chunk's V rows instead (conv + SiLU of
 // mixed_qkv's value channels, deltanet.py:243), so the preparation kernel neither
 // reads the value channels nor writes conv(v) to the workspace.
@@ -36,8 +37,8 @@
 // backward's recompute (BWD with p.o set), which forms o from hi+lo S, V_new and P.
 //
 // Modes: MODE_BF16 / MODE_F32 (core function) store o in fp32.  MODE_LAYER stores
-// o in bf16; the epilogue kernel (gdn_epilogue.hip) applies the gated RMSNorm
-// (deltanet.py:282-293).
+// o in bf16 for the epilogue kernel (gdn_epilogue.hip), which applies the gated RMSNorm
+// (deltanet.py:282-293), or applies it itself (FUSE).
 #include <type_traits>
 
 #include "gdn_chunk.h"
@@ -460,9 +461,11 @@ __device__ __forceinline__ unsigned take_ticket(int* tickets, unsigned per) {
 // to memory (system scope) with a flag raised behind it, and one step later reads every
 // block's partial (L2 bypassed), sums them in slot order with the pairwise tree the
 // epilogue kernel uses and leaves 1/RMS per row in LDS.  Meanwhile the compute
-// wavefronts keep their bf16 o rows in a four-chunk LDS ring and, three steps after the
-// chunk, normalise and gate them: w (o rsqrt(mean + eps)) silu(z), the epilogue kernel's
-// arithmetic, so the output is bit-identical to the unfused path's.  A wait for another
+// wavefronts keep their bf16 o rows in an LDS ring; three steps after the chunk they and a
+// finalizing wavefront normalise and gate them: w (o rsqrt(mean + eps)) silu(z), the epilogue
+// kernel's arithmetic, so the output is bit-identical to the unfused path's.  (Narrow
+// workgroups: an exchange wavefront in the loader's place, a step deeper, and all rows on the
+// finalizing one.)  A wait for another
 // block's flag ends because every block it waits for runs: in a grid the chip holds at once
 // all of them are resident; in a larger one each workgroup takes its place from a ticket as
 // it starts (take_ticket).  The wait is bounded all the same.
@@ -495,12 +498,12 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
   float ss_prev = 0.f;  // this lane's row sum of the previous chunk, not yet in sSS
   static_assert(!FUSE || WG_SS, "the fused norm runs on the layer's direct-load scan");
   constexpr bool XW = Q_::XWAVE, FW = Q_::FWAVE;
-  // (FUSE) chunks of bf16 o kept per compute wavefront: with a finalizing wavefront a chunk
-  // is read while a later one is written
+  // (FUSE) chunks of bf16 o kept per compute wavefront: a chunk is read while a later one is
+  // written
   constexpr int kRing = FW && XW ? 8 : 4;
   constexpr int kFin = FW && XW ? 4 : 3;  // (FUSE) steps from a chunk to its normalisation
   static_assert(kFin < kRing, "a chunk is normalised before its ring entry is rewritten");
-  // (FUSE) lane l's 4 x 4 bf16 o values of row block i of chunk c, wave w: sO[c % 4][w][i][l]
+  // (FUSE) lane l's 4 x 4 bf16 o values of row block i of chunk c, wave w: sO[c % kRing][w][i][l]
   __shared__ __align__(16) u32x2 sO[FUSE ? kRing : 1][FUSE ? NWC : 1][FUSE ? 4 : 1][64];
   __shared__ float sRN[FUSE ? 2 : 1][C];  // (FUSE) 1/RMS of each row of a chunk
   constexpr int K_LO = C * LDK, V_LO = C * LDT;
