@@ -210,14 +210,14 @@ def cpu_decode_baseline(batches=(1, 8, 64), budget_s=4.0):
 # scaled by a plain copy kernel's counters), for the shapes they were taken on, with the
 # profiles/ summary that gives the commands and per-kernel figures.
 MEASURED_TRAFFIC = {
-    ("core", 4, 4096, 16, 32, 128): (1_153_999_872, "profiles/prefill_c1.md (core call)"),
-    ("core", 1, 65536, 16, 64, 128): (7_707_787_264, "profiles/prefill_c3_c4.md (C4 core call)"),
+    ("core", 4, 4096, 16, 32, 128): (1_099_222_221, "profiles/prefill_c1.md (core call)"),
+    ("core", 1, 65536, 16, 64, 128): (9_761_823_130, "profiles/prefill_c3_c4.md (C4 core call)"),
     ("decode", 64, 16, 32, 128): (277_346_304, "profiles/decode_step_c2.md (B=64)"),
     ("decode", 256, 16, 32, 128): (1_108_210_688, "profiles/decode_step_c2.md (B=256)"),
-    # layer step: prep 155.3 + 283.3 MiB, scan (with the gated norm) 546.6 + 136.0
-    ("prefill", 4, 4096, 16, 32, 128): (1_175_575_552, "profiles/prefill_c1.md (layer kernels)"),
-    ("c3", 32768, 8): (2_954_456_781, "profiles/prefill_c3_c4.md (C3 layer call)"),
-    ("bwd", 4, 4096, 16, 32, 128): (6_873_572_192, "profiles/bwd_c1.md (backward call)"),
+    # layer step: prep 154.0 + 258.3 MiB, scan (with the gated norm) 531.0 + 136.0
+    ("prefill", 4, 4096, 16, 32, 128): (1_131_728_077, "profiles/prefill_c1.md (layer kernels)"),
+    ("c3", 32768, 8): (2_335_912_755, "profiles/prefill_c3_c4.md (C3 layer call)"),
+    ("bwd", 4, 4096, 16, 32, 128): (6_415_712_256, "profiles/bwd_c1.md (backward call)"),
 }
 
 
