@@ -1382,20 +1382,31 @@ hipError_t launch_scan_cfg(const ChunkParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Column tiles per workgroup: 4 (64 columns) when that gives a workgroup per CU, else 2 or
-// 1, the widest that still does.  The workgroups walk their sequences' chunks in order, so a
+// Column tiles per workgroup (4: 64 columns).  Sequences of one length: the narrowest whose
+// workgroups the chip holds at once, one per CU, else 4: a second round would walk every
+// chunk again, for a chunk step that is at most 1.6 times shorter (d=128, two rounds of the
+// next narrower width -> one: layer scan of B=3 T=1,000 Hv=32 82 -> 52 us, of B=1 T=2,000
+// Hv=48, with its norm, 138 -> 72; training of B=5 T=600 Hv=8, recompute 40 -> 26, reverse
+// 68 -> 39; d=64, B=6 T=600 Hv=32, 42 -> 31 and 57 -> 38).
+// Packed sequences, whose lengths the host does not know: the widest that gives a workgroup
+// per CU, since the longest chain, started first, then runs at the shortest step while the
+// others share what is left (narrow -> one round of the wider: three documents of 3,000
+// tokens, Hv=32, layer scan 88 -> 87 us, recompute 114 -> 130, reverse 116 -> 129; six of
+// 6,000, Hv=16, 97 -> 106).
+// The workgroups walk their sequences' chunks in order, so a
 // grid smaller than the chip leaves CUs idle for the whole call; narrower workgroups also
 // leave each CU's LDS to fewer wavefronts.  Against 64 columns: backward of B=1 T=2,548 Hv=32
 // d=128, recompute scan 112 -> 79 us and reverse scan 166 -> 135 us (256 workgroups of 16
 // columns for 64); fp32 inputs, B=2 T=512 H=4 d=64, 23.7 -> 19.3 us (32 for 8); layer rows,
 // B=8 T=1,000 Hv=16 d=64, 30.7 -> 27.7 us (256 of 32 columns for 128).
-int tiles_per_wg(long long tiles) {
+int tiles_per_wg(long long tiles, bool packed) {
   const long long cus = device_cus();
-  if (tiles >= 4 * cus) return 4;
-  if (tiles >= 2 * cus) return 2;
-  return 1;
+  if (packed) return tiles >= 4 * cus ? 4 : tiles >= 2 * cus ? 2 : 1;
+  return tiles > 2 * cus ? 4 : tiles > cus ? 2 : 1;
 }
-int scan_tiles_per_wg(const ChunkParams& p) { return tiles_per_wg((long long)p.N * p.Hv * (p.DV / 16)); }
+int scan_tiles_per_wg(const ChunkParams& p) {
+  return tiles_per_wg((long long)p.N * p.Hv * (p.DV / 16), p.cu_seqlens != nullptr);
+}
 
 template <int DK, int MODE, bool BWD = false, bool FUSE = false>
 hipError_t launch_scan_tiles(const ChunkParams& p, hipStream_t stream) {
@@ -1424,7 +1435,9 @@ int device_cus() {
 
 int chunk_block_cols() { return kBlockCols; }
 
-int scan_column_tiles(int N, int Hv, int DV) { return tiles_per_wg((long long)N * Hv * (DV / 16)); }
+int scan_column_tiles(int N, int Hv, int DV, bool packed) {
+  return tiles_per_wg((long long)N * Hv * (DV / 16), packed);
+}
 
 int layer_scan_blocks(const ChunkParams& p) {
   return p.DV / (16 * scan_tiles_per_wg(p));

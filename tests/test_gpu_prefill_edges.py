@@ -47,10 +47,9 @@ def test_layer_scan_pipeline_depth(B, Hk, Hv, dv, T):
 
 
 @pytest.mark.parametrize("B,Hk,Hv,dk,dv", [
-    (8, 1, 4, 128, 256),    # 32-column workgroups, eight to a value head, one round
-    (9, 1, 4, 128, 256),    # the same, past one round: the epilogue kernel
-    (24, 1, 4, 128, 128),   # 32-column, past one round
-    (25, 1, 4, 128, 128),   # the same, groups not a multiple of eight
+    (8, 1, 4, 128, 256),    # 32-column workgroups, eight to a value head
+    (9, 1, 4, 128, 256),    # 64-column, less than one round
+    (10, 1, 4, 128, 128),   # 32-column, less than one round
     (33, 1, 4, 128, 128),   # 64-column, past one round, groups not a multiple of eight
     (40, 1, 4, 128, 128),   # 64-column, past one round
     (24, 1, 3, 128, 256),   # 64-column, four to a value head, past one round
@@ -62,17 +61,22 @@ def test_layer_scan_at_every_workgroup_width(B, Hk, Hv, dk, dv):
     check_rows(B, 460, dict(Hk=Hk, dk=dk, Hv=Hv, dv=dv), (0, B // 2, B - 1), 8100 + B + dv)
 
 
-def test_layer_scan_of_many_packed_sequences():
-    """40 packed sequences, some of them empty, from their own states: past one round of the
-    chip, longest first."""
-    layer.say("layer scan: 40 packed sequences")
+@pytest.mark.parametrize("N", [
+    10,   # 16-column workgroups past one round of the chip: the epilogue kernel
+    24,   # 32-column, past one round
+    25,   # the same, groups not a multiple of eight: the epilogue kernel
+    40,   # 64-column, past one round
+])
+def test_layer_scan_of_packed_sequences_past_one_round(N):
+    """Packed sequences, some of them empty, from their own states, longest first."""
+    layer.say(f"layer scan: {N} packed sequences")
     dims = dict(Hk=1, dk=128, Hv=4, dv=128)
-    rng = np.random.default_rng(8200)
-    lens = rng.integers(0, 1100, size=40)
-    lens[[0, 7, 39]] = 0
+    rng = np.random.default_rng(8200 + N)
+    lens = rng.integers(0, 1200, size=N)
+    lens[[0, 7, N - 1]] = 0
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
-    d = W.layer_inputs(1, int(cu[-1]), **dims, seed=8201)
-    S0 = (0.02 * rng.standard_normal((40, 4, 128, 128))).astype(np.float32)
+    d = W.layer_inputs(1, int(cu[-1]), **dims, seed=8201 + N)
+    S0 = (0.02 * rng.standard_normal((N, 4, 128, 128))).astype(np.float32)
     out, S, conv = layer.gpu_prefill(W.to_device(d), dims, cu, S0)
     ref, S_ref, conv_ref = layer.ref_prefill(d, dims, cu, S0)
     assert layer.rel(layer.np_(out), ref) < layer.BF16_TOL
