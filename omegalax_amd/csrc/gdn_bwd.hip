@@ -1117,15 +1117,16 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // ---------------------------------------------------------------- dP and dL tiles
   // P = lower(scale Q K^T * Gamma) and Lg = strict_lower(K K^T * Gamma) at this wavefront's
   // tiles: fp32 inputs read them from the preparation kernel's matrices, bf16 inputs form
-  // them with its arithmetic (the same products summed by the same MFMA over the same dk
-  // blocks in the same order)
+  // them (the same products summed by the same MFMA over the same dk blocks in the same
+  // order).  Gamma comes from the difference of the gates: scaled to base 2 one by one, each
+  // would leave its own rounding there, 4e-5 at G = -1,000, and on the diagonal too.
   {
     f32x4 rowp = zero4(), rowl = zero4(), rowb = zero4();
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       f32x4 cg = zero4();
       const int col = 16 * j + lr;
-      const float gc = sG[col] * 1.4426950408889634f;
+      const float gc = sG[col];
       if (j <= rp) {  // uniform
         const f32x4 d4 = j < 2 ? tp[j] : tx[j - 2];
         f32x4 pp = zero4(), dpg;
@@ -1138,7 +1139,7 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int row = 16 * rp + 4 * lq + v;
-          const float e = __builtin_amdgcn_exp2f(fminf(sG[row] * 1.4426950408889634f - gc, 0.f));
+          const float e = __expf(fminf(sG[row] - gc, 0.f));
           const float d = row >= col ? d4[v] : 0.f;
           const float x = d * (F32 ? xb[kXlpgP + row * C + col] : scale * pp[v] * e);
           rowp[v] += x;
@@ -1159,7 +1160,7 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int row = 16 * rl + 4 * lq + v;
-          const float e = __builtin_amdgcn_exp2f(fminf(sG[row] * 1.4426950408889634f - gc, 0.f));
+          const float e = __expf(fminf(sG[row] - gc, 0.f));
           const float d = row > col ? -d4[v] : 0.f;      // dL
           const float x = d * (F32 ? xb[kXlpgLg + row * C + col] : kk[v] * e);
           const float y = sBt[row] * x;                  // dL * L

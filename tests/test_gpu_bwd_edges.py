@@ -40,6 +40,20 @@ def test_core_backward_with_zero_and_one_beta(dtype):
     core.check(got, core.run_ref(*args, dtype), dtype)
 
 
+@pytest.mark.parametrize("dk", [64, 32])
+def test_core_backward_of_fast_decay_keeps_the_diagonal(dk):
+    """Gates summing to -3,800 in a chunk leave Gamma its unit diagonal alone, so dq is one
+    product chain of four split operands (dO, V_new, dP, K) of relative error 2^-17 each: 2^-16
+    together, in quadrature.  A diagonal off by the rounding of G gives 4e-5 and more."""
+    core.say(f"bwd fast decay dk={dk}")
+    args = list(core.make(7150 + dk, 2, 192, 1, 2, dk, 64, "f32"))
+    args[3] = (-60 - np.random.default_rng(7150).uniform(0, 1, args[3].shape)).astype(np.float32)
+    got, ref = core.run_gpu(*args, "f32"), core.run_ref(*args, "f32")
+    core.check(got, ref, "f32", skip=("dg",))  # dg is a difference of sums that are all but equal
+    err = np.linalg.norm(got[0] - ref[0]) / np.linalg.norm(ref[0])
+    assert err < 2.0 ** -16, err
+
+
 @pytest.mark.parametrize("lens,Hk,Hv,dk,dv", [
     ([1], 1, 1, 64, 64),                              # one token; 192 channels (not a multiple of 256)
     ([2, 1, 1, 3], 1, 2, 64, 64),                     # sequences shorter than the conv window
