@@ -1109,7 +1109,7 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
           for (int w = 0; w < NWC; ++w) v[w] = sSS[c & 1][w][l];
           // rows past the chunk's end are given an offset past the range: dropped
           __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(ss_tree<NWC>(v)), (unsigned)c + 1u}, xr,
-                                                l < nvc ? 8u * l : 0x80000000u, xch_off(c, blk), 17);
+                                                l < nvc ? 8u * l : kDropOffset, xch_off(c, blk), 17);
         }
       };
       // every block's partial of chunk c's row l, read past the caches (system scope)

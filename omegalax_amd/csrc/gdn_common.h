@@ -33,6 +33,11 @@ __device__ __forceinline__ float round_bf(float f) { return bf2f(f2bf(f)); }
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
+// The lane offset of an access that is to be dropped: past every range it is used with,
+// aligned to the widest access, and far enough below 2^32 that neither the scalar offset nor
+// an access's later dwords take it past the end of 32 bits and back to the range's start.
+constexpr unsigned kDropOffset = 0x80000000u;
+static_assert(kDropOffset % 16 == 0 && kDropOffset <= 0xffffffffu - (1u << 30), "drop offset");
 
 // Workgroup barrier that orders LDS accesses only: it does not wait for the wave's
 // outstanding global loads and stores (__syncthreads does), so prefetches and result

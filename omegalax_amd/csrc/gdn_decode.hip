@@ -390,7 +390,6 @@ void decode_stream_kernel(DecodeParams p) {
   static_assert(DV == 64 || DV == 128, "stream decode dv");
   static_assert(DK % RGW == 0 && R >= 1, "stream decode rows");
   static_assert(NPC <= kPreChannels && (GQA == 1 || GQA == 2), "stream decode item shape");
-  constexpr unsigned kDrop = 0x80000000u;              // a lane offset past every range
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -504,7 +503,7 @@ void decode_stream_kernel(DecodeParams p) {
       acc += round_bf(w3) * bf2f(px[m]);
       const float y = round_bf(siluf_(round_bf(acc)));
       // shift the cache: drop the oldest input, append this token's raw input
-      const unsigned co = real ? 2u * 3u * c : kDrop;
+      const unsigned co = real ? 2u * 3u * c : kDropOffset;
       __builtin_amdgcn_raw_buffer_store_b16(ph[m][1], cw, co, 0, 0);
       __builtin_amdgcn_raw_buffer_store_b16(ph[m][2], cw, co, 2, 0);
       __builtin_amdgcn_raw_buffer_store_b16(px[m], cw, co, 4, 0);
@@ -608,7 +607,7 @@ void decode_stream_kernel(DecodeParams p) {
     const u32x2w ov{pack_bf16(nw.x * (o[0] * rn) * sz.x, nw.y * (o[1] * rn) * sz.y),
                     pack_bf16(nw.z * (o[2] * rn) * sz.z, nw.w * (o[3] * rn) * sz.w)};
     // one lane per column group stores (the row groups hold the same values)
-    __builtin_amdgcn_raw_buffer_store_b64(ov, orr, rg == 0 ? 2u * (unsigned)col : kDrop, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(ov, orr, rg == 0 ? 2u * (unsigned)col : kDropOffset, 0, 0);
   };
 
   if (my_items <= 0) return;

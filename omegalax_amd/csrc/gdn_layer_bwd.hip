@@ -359,7 +359,6 @@ __device__ __forceinline__ void conv_bwd(const LayerBwdParams& p, long long bid,
     // outside the range: dropped, no branch)
     const long long rows = p.tokens - tb < kConvSB ? p.tokens - tb : kConvSB;
     const auto dxr = buf_rsrc(p.dx + tb * p.conv_dim, 2u * (unsigned)(rows * p.conv_dim));
-    const unsigned drop = 0xffffffffu;
     float xf[4][4];  // [d][channel]: x[t - d]
 #pragma unroll
     for (int d = 1; d < 4; ++d)
@@ -401,7 +400,7 @@ __device__ __forceinline__ void conv_bwd(const LayerBwdParams& p, long long bid,
       }
       if (k >= 3)
         __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16(dx[3][0], dx[3][1]), pack_bf16(dx[3][2], dx[3][3])}, dxr,
-                                              in ? 2u * (unsigned)((k - 3) * p.conv_dim + c0) : drop, 0, 0);
+                                              in ? 2u * (unsigned)((k - 3) * p.conv_dim + c0) : kDropOffset, 0, 0);
 #pragma unroll
       for (int d = 3; d > 0; --d)
 #pragma unroll

@@ -332,3 +332,18 @@ def test_qkv_conv_proj_rejects_bad_shapes_on_the_host():
     assert f(16, 16, None, 16, 8, 128, 256, 8, 4, 1, None) == _lib.EINVAL  # conv needs conv_w
     assert f(24, 16, 16, 16, 8, 128, 256, 8, 4, 1, None) == _lib.EINVAL
     assert "aligned" in L.omx_gdn_last_error().decode()
+
+
+def test_no_buffer_access_is_dropped_by_an_offset_that_can_wrap():
+    """A dropped lane's offset comes from kDropOffset, whose alignment and distance from 2^32
+    a static_assert pins: at 0xffffffff the second dword of an 8-byte store lies past the end
+    of 32 bits, where a wrapped address is the first row of the range."""
+    csrc = os.path.join(ROOT, "omegalax_amd", "csrc")
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".hip", ".h")):
+            continue
+        src = open(os.path.join(csrc, name)).read()
+        for const in re.findall(r"unsigned \w*[dD]rop\w* = (0x[0-9a-f]+)u", src):
+            assert int(const, 16) % 16 == 0 and int(const, 16) <= 0xffffffff - (1 << 30), (name, const)
+        for stmt in re.findall(r"raw_buffer_(?:load|store)_b\d+\([^;]*;", src):
+            assert "0xffffffff" not in stmt, (name, stmt)

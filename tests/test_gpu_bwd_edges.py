@@ -56,6 +56,7 @@ def test_core_backward_of_fast_decay_keeps_the_diagonal(dk):
 
 @pytest.mark.parametrize("lens,Hk,Hv,dk,dv", [
     ([1], 1, 1, 64, 64),                              # one token; 192 channels (not a multiple of 256)
+    ([40], 1, 1, 64, 64),                             # the same over three wavefronts' rows, each with a first one
     ([2, 1, 1, 3], 1, 2, 64, 64),                     # sequences shorter than the conv window
     ([15, 1, 2, 14, 17, 15], 1, 1, 64, 128),          # starts on both sides of 16-token edges
     ([62, 1, 1, 3, 64, 0, 5], 2, 4, 128, 128),        # starts around a 64-token edge, one empty
