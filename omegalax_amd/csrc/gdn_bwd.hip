@@ -535,8 +535,9 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
     }
   };
   // (LDR) tile (mb, nb) of P = lower(scale Q K^T * Gamma) in the C layout, from the rows
-  // staged in bf, with the preparation kernel's arithmetic:
-  // scale * acc * 2^{min(G_m log2 e - G_n log2 e, 0)} * mask
+  // staged in bf.  Gamma comes from the difference of the gates, as in the gradient kernel:
+  // scaled to base 2 one by one, a product contracted into the subtraction would leave the
+  // other's rounding, 2e-4 at G = -3,800, on the diagonal too.
   auto form_ptile = [&](int mb, int nb, const Buf& bf) {
     f32x4 acc = zero4();
 #pragma unroll
@@ -545,9 +546,7 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int m = 16 * mb + 4 * lq + v, n = 16 * nb + lr;
-      acc[v] = p.scale * acc[v] *
-               __builtin_amdgcn_exp2f(fminf(bf.Gl[m] * 1.4426950408889634f - bf.Gl[n] * 1.4426950408889634f, 0.f)) *
-               (float)(m >= n);
+      acc[v] = p.scale * acc[v] * __expf(fminf(bf.Gl[m] - bf.Gl[n], 0.f)) * (float)(m >= n);
     }
     return acc;
   };

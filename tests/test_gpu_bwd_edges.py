@@ -54,6 +54,25 @@ def test_core_backward_of_fast_decay_keeps_the_diagonal(dk):
     assert err < 2.0 ** -16, err
 
 
+@pytest.mark.parametrize("dk", [128, 64])
+def test_bf16_backward_of_fast_decay_keeps_the_diagonal(dk):
+    """The same for the reverse scan's P, which bf16 inputs form there: with Gamma's unit
+    diagonal alone dbeta_i is scale (q_i . k_i) (dO_i . v_i), P and dO split to 2^-17 each and
+    v exact.  q and k rows hold 64 entries of +-1, so that their normalised rows are exact."""
+    core.say(f"bwd fast decay bf16 dk={dk}")
+    args = list(core.make(7160 + dk, 2, 192, 1, 2, dk, 64, "bf16"))
+    for n in (0, 1):
+        args[n] = np.sign(args[n])
+        args[n][..., 64:] = 0
+    args[3] = (-60 - np.random.default_rng(7160).uniform(0, 1, args[3].shape)).astype(np.float32)
+    got, ref = core.run_gpu(*args, "bf16"), core.run_ref(*args, "bf16")
+    assert all(np.isfinite(x).all() for x in got)
+    core.check(got, ref, "bf16", skip=("dg",))  # dg is a difference of sums that are all but equal
+    err = np.linalg.norm(got[4] - ref[4]) / np.linalg.norm(ref[4])
+    core.say(f"  dbeta {err:.2e}")
+    assert err < 2.0 ** -16, err
+
+
 @pytest.mark.parametrize("lens,Hk,Hv,dk,dv", [
     ([1], 1, 1, 64, 64),                              # one token; 192 channels (not a multiple of 256)
     ([40], 1, 1, 64, 64),                             # the same over three wavefronts' rows, each with a first one
