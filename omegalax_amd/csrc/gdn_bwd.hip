@@ -973,7 +973,7 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   f32x4 tp[2], tl[2], tx[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) tp[j] = tl[j] = tx[j] = zero4();
-  float sds = 0.f;                     // sum of dS * S (each element is loaded once here)
+  float sds = 0.f;                     // sum of dS * S in fp32 (each element is loaded once here)
   float rv[NRI];                       // dR . v of the thread's rows, its columns
 #pragma unroll
   for (int m = 0; m < NRI; ++m) rv[m] = 0.f;
@@ -1032,10 +1032,8 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     Op bd[NKB];
 #pragma unroll
     for (int t = 0; t < NKB; ++t) {
-      float x[8];
-      op_values(bs[t], x);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sds += x[e] * dfr[t][e];
+      for (int e = 0; e < 8; ++e) sds += sfr[t][e] * dfr[t][e];
       bd[t] = split8(dfr[t]);
     }
     __builtin_amdgcn_sched_barrier(0);

@@ -73,6 +73,25 @@ def test_bf16_backward_of_fast_decay_keeps_the_diagonal(dk):
     assert err < 2.0 ** -16, err
 
 
+@pytest.mark.parametrize("T,dk,dv,dtype", [(64, 64, 64, "f32"), (40, 32, 128, "f32"),
+                                           (64, 128, 128, "bf16"), (40, 64, 64, "bf16")])
+def test_gate_gradient_takes_the_state_in_fp32(T, dk, dv, dtype):
+    """Without decay, writes (beta = 0) or a cotangent of o, dg is the sum of dS * S.  Every
+    entry of S is 1 + 2^-9 + 2^-17, whose last bit two bf16 parts do not hold: 2^-17 of the
+    sum.  In fp32 a lane's products and sums are exact, and the ten additions over lanes and
+    wavefronts leave at most 10 * 2^-24."""
+    core.say(f"bwd dg from the state T={T} dk={dk} dv={dv} {dtype}")
+    q, k, v, g, beta, S0, do, dht = core.make(7170 + T + dk, 1, T, 1, 2, dk, dv, dtype)
+    S0[:] = 1 + 2.0 ** -9 + 2.0 ** -17
+    dht[:] = 0.5
+    args = (q, k, v, 0 * g, 0 * beta, S0, 0 * do, dht)
+    got, ref = core.run_gpu(*args, dtype), core.run_ref(*args, dtype)
+    core.check(got, ref, dtype, skip=("dq",))  # zero
+    err = core.rel(got[3], ref[3])
+    core.say(f"  dg {err:.2e}")
+    assert err < 10 * 2.0 ** -24, err
+
+
 @pytest.mark.parametrize("lens,Hk,Hv,dk,dv", [
     ([1], 1, 1, 64, 64),                              # one token; 192 channels (not a multiple of 256)
     ([40], 1, 1, 64, 64),                             # the same over three wavefronts' rows, each with a first one
