@@ -213,14 +213,20 @@ __global__ __launch_bounds__(64 * kSmallWaves) void ab_proj_small_kernel(const b
 #pragma unroll
     for (int j = 0; j < 2 * kSmallSteps; ++j) {
       const int k = k0 + 64 * kSmallWaves * (j >> 1) + 16 * lq + 8 * (j & 1);
-      const int kc = k < D ? k : 0;  // past D: element 0, and zeros in x
+      const int kc = k < D ? k : 0;  // past D: element 0, replaced by zeros below
       xv[j] = *(const u32x4*)(xr + kc);
       wv[j] = *(const u32x4*)(wr + kc);
     }
+    if (k0 + 64 * kSmallWaves * (kSmallSteps - 1) + 64 <= D) {  // uniform
 #pragma unroll
-    for (int j = 0; j < 2 * kSmallSteps; ++j) {
-      const int k = k0 + 64 * kSmallWaves * (j >> 1) + 16 * lq + 8 * (j & 1);
-      acc = mma16(wv[j], k < D ? xv[j] : z4, acc);
+      for (int j = 0; j < 2 * kSmallSteps; ++j) acc = mma16(wv[j], xv[j], acc);
+    } else {
+      // zeros in both operands past D: an infinite weight must not meet a zero of x
+#pragma unroll
+      for (int j = 0; j < 2 * kSmallSteps; ++j) {
+        const int k = k0 + 64 * kSmallWaves * (j >> 1) + 16 * lq + 8 * (j & 1);
+        acc = mma16(k < D ? wv[j] : z4, k < D ? xv[j] : z4, acc);
+      }
     }
   }
   sum[wave][l] = acc;

@@ -139,3 +139,20 @@ def test_ab_projections_of_few_rows(M, D, Hv):
     """The few-row kernel's edges: rows and columns past a tile, a contraction shorter than its
     eight wavefronts' first step and one ending inside a step, and its largest row count."""
     test_ab_projections_match_fp64_and_library_gemms(M, D, Hv)
+
+
+@pytest.mark.parametrize("M,D,Hv", [(17, 1024, 32), (3, 64, 6), (33, 520, 16)])
+def test_ab_projections_of_few_rows_keep_infinities(M, D, Hv):
+    """The contraction's steps past D are no products: an infinite weight or activation gives
+    the infinities and NaN of its own row or column, as the library product does."""
+    from omegalax_amd import gdn_ab_projections
+    print(f"ab projections with infinities M={M} D={D} Hv={Hv}", flush=True)
+    x, wa, wb = inputs(M, D, Hv, 3 * M + D)
+    x[x == 0] = 1
+    wa[0, 0], wb[Hv - 1, 7], x[M - 1, 5] = float("inf"), float("-inf"), float("inf")
+    for got, w in zip(gdn_ab_projections(x, wa, wb), (wa, wb)):
+        want = torch.nn.functional.linear(x.float().cpu(), w.float().cpu())
+        got = got.float().cpu()
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(torch.isinf(got), torch.isinf(want))
+        assert torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])
