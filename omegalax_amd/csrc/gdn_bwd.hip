@@ -1345,7 +1345,7 @@ hipError_t launch_bwd_dk(const BwdParams& p, hipStream_t stream) {
   if constexpr (F32) {
     e = launch_rscan<DK, F32, 4>(p, stream);
   } else {
-    const int tiles = scan_column_tiles(p.N, p.Hv, p.DV, p.cu_seqlens != nullptr);
+    const int tiles = scan_column_tiles(p.N, p.Hv, p.DV, p.dk, p.cu_seqlens != nullptr, true);
     e = tiles == 1   ? launch_rscan<DK, F32, 1>(p, stream)
         : tiles == 2 ? launch_rscan<DK, F32, 2>(p, stream)
                      : launch_rscan<DK, F32, 4>(p, stream);

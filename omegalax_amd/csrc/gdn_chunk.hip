@@ -1382,35 +1382,13 @@ hipError_t launch_scan_cfg(const ChunkParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Column tiles per workgroup (4: 64 columns).  Sequences of one length: the narrowest whose
-// workgroups the chip holds at once, one per CU, else 4: a second round would walk every
-// chunk again, for a chunk step that is at most 1.6 times shorter (d=128, two rounds of the
-// next narrower width -> one: layer scan of B=3 T=1,000 Hv=32 82 -> 52 us, of B=1 T=2,000
-// Hv=48, with its norm, 138 -> 72; training of B=5 T=600 Hv=8, recompute 40 -> 26, reverse
-// 68 -> 39; d=64, B=6 T=600 Hv=32, 42 -> 31 and 57 -> 38).
-// Packed sequences, whose lengths the host does not know: the widest that gives a workgroup
-// per CU, since the longest chain, started first, then runs at the shortest step while the
-// others share what is left (narrow -> one round of the wider: three documents of 3,000
-// tokens, Hv=32, layer scan 88 -> 87 us, recompute 114 -> 130, reverse 116 -> 129; six of
-// 6,000, Hv=16, 97 -> 106).
-// The workgroups walk their sequences' chunks in order, so a
-// grid smaller than the chip leaves CUs idle for the whole call; narrower workgroups also
-// leave each CU's LDS to fewer wavefronts.  Against 64 columns: backward of B=1 T=2,548 Hv=32
-// d=128, recompute scan 112 -> 79 us and reverse scan 166 -> 135 us (256 workgroups of 16
-// columns for 64); fp32 inputs, B=2 T=512 H=4 d=64, 23.7 -> 19.3 us (32 for 8); layer rows,
-// B=8 T=1,000 Hv=16 d=64, 30.7 -> 27.7 us (256 of 32 columns for 128).
-int tiles_per_wg(long long tiles, bool packed) {
-  const long long cus = device_cus();
-  if (packed) return tiles >= 4 * cus ? 4 : tiles >= 2 * cus ? 2 : 1;
-  return tiles > 2 * cus ? 4 : tiles > cus ? 2 : 1;
-}
-int scan_tiles_per_wg(const ChunkParams& p) {
-  return tiles_per_wg((long long)p.N * p.Hv * (p.DV / 16), p.cu_seqlens != nullptr);
+int scan_tiles_per_wg(const ChunkParams& p, bool bwd) {
+  return scan_column_tiles(p.N, p.Hv, p.DV, p.dk, p.cu_seqlens != nullptr, bwd);
 }
 
 template <int DK, int MODE, bool BWD = false, bool FUSE = false>
 hipError_t launch_scan_tiles(const ChunkParams& p, hipStream_t stream) {
-  switch (scan_tiles_per_wg(p)) {
+  switch (scan_tiles_per_wg(p, BWD)) {
     case 1: return launch_scan_cfg<DK, MODE, BWD, 1, FUSE>(p, stream);
     case 2: return launch_scan_cfg<DK, MODE, BWD, 2, FUSE>(p, stream);
     default: return launch_scan_cfg<DK, MODE, BWD, 4, FUSE>(p, stream);
@@ -1435,12 +1413,30 @@ int device_cus() {
 
 int chunk_block_cols() { return kBlockCols; }
 
-int scan_column_tiles(int N, int Hv, int DV, bool packed) {
-  return tiles_per_wg((long long)N * Hv * (DV / 16), packed);
+// Column tiles per workgroup (4: 64 columns).  The workgroups walk their sequences' chunks in
+// order, so a grid smaller than the chip leaves CUs idle for the whole call; narrower
+// workgroups also leave each CU's LDS to fewer wavefronts.  So: the narrowest whose
+// workgroups the chip holds at once, one per CU, else 4.  A second round would walk every
+// chunk again, for a chunk step that is at most 1.6 times shorter (d=128, two rounds of the
+// next narrower width -> one: layer scan of B=3 T=1,000 Hv=32 82 -> 52 us, of B=1 T=2,000
+// Hv=48, with its norm, 138 -> 72; training of B=5 T=600 Hv=8, recompute 40 -> 26, reverse
+// 68 -> 39; d=64, B=6 T=600 Hv=32, 42 -> 31 and 57 -> 38).  Against 64 columns: backward of
+// B=1 T=2,548 Hv=32 d=128, recompute scan 112 -> 79 us and reverse scan 166 -> 135 us (256
+// workgroups of 16 columns for 64); fp32 inputs, B=2 T=512 H=4 d=64, 23.7 -> 19.3 us (32 for
+// 8); layer rows, B=8 T=1,000 Hv=16 d=64, 30.7 -> 27.7 us (256 of 32 columns for 128).
+// The forward scan of several packed sequences at dk = 128 takes the widest that gives a
+// workgroup per CU: their lengths, which the host does not know, mostly differ, and then the
+// longest chain, started first, runs at the shortest step while the others share what is left
+// (six documents of 6,000 tokens on average, Hv=16, 97 us against 106 in one round of the
+// wider; three of 3,000, Hv=32, 88 against 87).
+int scan_column_tiles(int N, int Hv, int DV, int dk, bool packed, bool bwd) {
+  const long long tiles = (long long)N * Hv * (DV / 16), cus = device_cus();
+  if (packed && N > 1 && dk == 128 && !bwd) return tiles >= 4 * cus ? 4 : tiles >= 2 * cus ? 2 : 1;
+  return tiles > 2 * cus ? 4 : tiles > cus ? 2 : 1;
 }
 
 int layer_scan_blocks(const ChunkParams& p) {
-  return p.DV / (16 * scan_tiles_per_wg(p));
+  return p.DV / (16 * scan_tiles_per_wg(p, false));
 }
 
 // The layer scan applies the gated norm itself (FUSE) when it loads directly (dk = 128), the
@@ -1462,7 +1458,7 @@ bool layer_scan_fuses_norm(const ChunkParams& p) {
 }
 
 int layer_ss_slots(const ChunkParams& p) {
-  return p.dk == 128 ? p.DV / (16 * scan_tiles_per_wg(p)) : p.DV / 16;
+  return p.dk == 128 ? p.DV / (16 * scan_tiles_per_wg(p, false)) : p.DV / 16;
 }
 
 int chunk_record_bytes(int mode, bool bwd) { return rec_bytes(mode, bwd); }

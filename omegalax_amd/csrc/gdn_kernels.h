@@ -147,7 +147,7 @@ bool chunk_dims_supported(int dk, int dv, bool f32_inputs);
 int chunk_block_cols();
 int device_cus();  // compute units of the current device
 // 16-column tiles per workgroup (4, 2 or 1) of the forward and reverse scans
-int scan_column_tiles(int N, int Hv, int DV, bool packed);
+int scan_column_tiles(int N, int Hv, int DV, int dk, bool packed, bool bwd);
 bool layer_dims_supported(int dk, int dv);
 // (layer) whether the scan forms the v rows itself (conv + SiLU), so the workspace holds
 // no conv(v) rows

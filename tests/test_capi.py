@@ -347,3 +347,26 @@ def test_no_buffer_access_is_dropped_by_an_offset_that_can_wrap():
             assert int(const, 16) % 16 == 0 and int(const, 16) <= 0xffffffff - (1 << 30), (name, const)
         for stmt in re.findall(r"raw_buffer_(?:load|store)_b\d+\([^;]*;", src):
             assert "0xffffffff" not in stmt, (name, stmt)
+
+
+@pytest.mark.parametrize("dk,bwd", [(64, False), (64, True), (128, True)])
+@pytest.mark.parametrize("N", [1, 3, 9, 40])
+@pytest.mark.parametrize("Hv,DV", [(1, 64), (16, 128), (32, 64), (48, 128)])
+def test_packed_scans_that_took_64_columns_never_take_two_rounds_of_narrower_ones(N, Hv, DV, dk, bwd):
+    """Documents of one length, packed, walk every chunk again in a second round: the widths of
+    the scans of packed rows are those of a batch, except in the dk = 128 forward scan of
+    several (omx::scan_column_tiles; a host without a GPU counts 256 CUs)."""
+    f = getattr(_lib.lib(), "_ZN3omx17scan_column_tilesEiiiibb")
+    f.argtypes, f.restype = [ctypes.c_int] * 4 + [ctypes.c_bool] * 2, ctypes.c_int
+    tiles = N * Hv * DV // 16
+    got = f(N, Hv, DV, dk, True, bwd)
+    assert got == f(N, Hv, DV, dk, False, bwd)
+    assert got == 4 or tiles // got <= 256
+
+
+def test_one_packed_sequence_takes_the_widths_of_a_batch_of_one():
+    f = getattr(_lib.lib(), "_ZN3omx17scan_column_tilesEiiiibb")
+    f.argtypes, f.restype = [ctypes.c_int] * 4 + [ctypes.c_bool] * 2, ctypes.c_int
+    for Hv in (16, 32, 48, 64, 96):
+        assert f(1, Hv, 128, 128, True, False) == f(1, Hv, 128, 128, False, False)
+    assert f(3, 16, 128, 128, True, False) == 1 and f(3, 16, 128, 128, False, False) == 2

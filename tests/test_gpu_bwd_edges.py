@@ -73,6 +73,20 @@ def test_bf16_backward_of_fast_decay_keeps_the_diagonal(dk):
     assert err < 2.0 ** -16, err
 
 
+@pytest.mark.parametrize("dk,dtype", [(128, "bf16"), (64, "bf16"), (64, "f32")])
+def test_packed_documents_of_one_length_agree_with_the_batch(dk, dtype):
+    """Three documents of one length, packed, take the widths of the batch of three and give
+    its gradients bit for bit (24 heads: more 16-column workgroups than the chip has CUs)."""
+    core.say(f"bwd packed widths dk={dk} {dtype}")
+    N, T, Hk, Hv = 3, 150, 8, 24
+    args = core.make(7180 + dk, N, T, Hk, Hv, dk, 64 if dk == 64 else 128, dtype)
+    batch = core.run_gpu(*args, dtype)
+    row = [x.reshape(1, N * T, *x.shape[2:]) for x in args[:5]] + [args[5], args[6].reshape(1, N * T, *args[6].shape[2:]), args[7]]
+    packed = core.run_gpu(*row, dtype, np.arange(N + 1, dtype=np.int32) * T)
+    for a, b in zip(batch, packed):
+        assert np.array_equal(a.reshape(b.shape), b)
+
+
 @pytest.mark.parametrize("T,dk,dv,dtype", [(64, 64, 64, "f32"), (40, 32, 128, "f32"),
                                            (64, 128, 128, "bf16"), (40, 64, 64, "bf16")])
 def test_gate_gradient_takes_the_state_in_fp32(T, dk, dv, dtype):
