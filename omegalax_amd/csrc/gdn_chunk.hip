@@ -56,7 +56,8 @@ constexpr int kBlockCols = 64;  // dv columns per block of the other kernels (nb
 // NWC_: 16-column state tiles (compute wavefronts) per workgroup: four, or two or one, so
 // that sequences x heads x dv / 16 tiles fill the chip when 64-column workgroups would leave
 // CUs idle (where loader wavefronts stage the rows; see scan_column_tiles).
-template <int DK, int MODE, int NWC_ = 4, bool BWD_ = false, bool FUSE_ = false>
+// OWN_: without loader wavefronts where there is a choice (see staging_wavefronts).
+template <int DK, int MODE, int NWC_ = 4, bool BWD_ = false, bool FUSE_ = false, bool OWN_ = false>
 struct Cfg {
   static constexpr int NWC = NWC_;
   static constexpr int BV = 16 * NWC;  // state columns per workgroup
@@ -104,10 +105,10 @@ struct Cfg {
   // the chunk after next in registers and store the next chunk into the free set, while the
   // compute wavefronts work on the other: one barrier per chunk, and neither the rows' waits
   // nor their conversion (fp32 rows are split on staging) sit on the state's chain.  Otherwise
-  // (fp32 inputs at dk = 128) the compute wavefronts stage the rows themselves, between two
-  // barriers.  fp32 inputs at d = 64 (B=2, T=512, H=4):
+  // (fp32 inputs at dk = 128, OWN_) the compute wavefronts stage the rows themselves, between
+  // two barriers.  fp32 inputs at d = 64 (B=2, T=512, H=4):
   // the scan 30.1 -> 23.6 us; layer rows at d = 64 (B=4, T=500, Hv=16): 22.1 -> 18.0 us.
-  static constexpr bool LSTAGE = !DIRECT && 2 * BUF <= 160 * 1024;
+  static constexpr bool LSTAGE = !DIRECT && !OWN_ && 2 * BUF <= 160 * 1024;
   static constexpr int NL = DIRECT ? ((MODE == MODE_BF16 && BWD_) || NWC_ < 4 ? 2 : 1) : (LSTAGE ? NST / 64 : 0);
   // (layer, 16 and 32 columns) one more wavefront stores or (FUSE) exchanges the rows'
   // partial sums, so that the loaders wait for nothing but their rows; (FUSE) one
@@ -469,12 +470,12 @@ __device__ __forceinline__ unsigned take_ticket(int* tickets, unsigned per) {
 // block's flag ends because every block it waits for runs: in a grid the chip holds at once
 // all of them are resident; in a larger one each workgroup takes its place from a ticket as
 // it starts (take_ticket).  The wait is bounded all the same.
-template <int DK, int MODE, bool BWD = false, int NWC_ = 4, bool FUSE = false>
+template <int DK, int MODE, bool BWD = false, int NWC_ = 4, bool FUSE = false, bool OWN = false>
 // One workgroup per CU is the design point (the state fills the register file): the
 // compiler may use the whole file (half of it with a loader wavefront, which shares a
 // SIMD) instead of holding back for a second workgroup.
-__global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute__((amdgpu_waves_per_eu(Cfg<DK, MODE, NWC_, BWD, FUSE>::WPE, Cfg<DK, MODE, NWC_, BWD, FUSE>::WPE))) void scan_kernel(ChunkParams p) {
-  using Q_ = Cfg<DK, MODE, NWC_, BWD, FUSE>;
+__global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE, OWN>::NTH)) __attribute__((amdgpu_waves_per_eu(Cfg<DK, MODE, NWC_, BWD, FUSE, OWN>::WPE, Cfg<DK, MODE, NWC_, BWD, FUSE, OWN>::WPE))) void scan_kernel(ChunkParams p) {
+  using Q_ = Cfg<DK, MODE, NWC_, BWD, FUSE, OWN>;
   constexpr int NWC = Q_::NWC, BV = Q_::BV, NT = Q_::NT;
   constexpr int LDK = Q_::LDK;
   constexpr bool IS = Q_::IS, OS = Q_::OS;
@@ -1368,9 +1369,9 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE>::NTH)) __attribute_
 
 // The scan's workgroups cover Cfg::BV columns each; p.nb (the other kernels' 64-column
 // blocks) is replaced by the scan's own count in a copy of the parameters.
-template <int DK, int MODE, bool BWD = false, int NWC = 4, bool FUSE = false>
+template <int DK, int MODE, bool BWD = false, int NWC = 4, bool FUSE = false, bool OWN = false>
 hipError_t launch_scan_cfg(const ChunkParams& p, hipStream_t stream) {
-  using Q_ = Cfg<DK, MODE, NWC, BWD, FUSE>;
+  using Q_ = Cfg<DK, MODE, NWC, BWD, FUSE, OWN>;
   ChunkParams q = p;
   q.nb = p.DV / Q_::BV;
   // (layer) row-sum partials per (token, value head): one per workgroup with direct
@@ -1378,7 +1379,7 @@ hipError_t launch_scan_cfg(const ChunkParams& p, hipStream_t stream) {
   q.ss_slots = Q_::DIRECT ? q.nb : p.DV / 16;
   const unsigned grid = (unsigned)(q.N * q.Hv * q.nb);
   if (grid <= (unsigned)device_cus()) q.tickets = nullptr;  // all resident: place = blockIdx.x
-  hipLaunchKernelGGL((scan_kernel<DK, MODE, BWD, NWC, FUSE>), dim3(grid), dim3(Q_::NTH), 0, stream, q);
+  hipLaunchKernelGGL((scan_kernel<DK, MODE, BWD, NWC, FUSE, OWN>), dim3(grid), dim3(Q_::NTH), 0, stream, q);
   return hipGetLastError();
 }
 
@@ -1386,13 +1387,31 @@ int scan_tiles_per_wg(const ChunkParams& p, bool bwd) {
   return scan_column_tiles(p.N, p.Hv, p.DV, p.dk, p.cu_seqlens != nullptr, bwd);
 }
 
+// (bf16 rows of dk = 64, forward, 64 columns) whether loader wavefronts stage the rows.  They
+// have nothing to run ahead of when sequences have one chunk (B=600 T=64 Hv=16 264 us, without
+// them 247).  And ahead of the products they let the workgroups of one key head drift apart:
+// while the call's records and rows stay in the 256 MiB cache behind the L2s that costs
+// nothing (records of 72 MiB, B=12 T=1,500 Hk=4 Hv=16, 76 us, without them 91; layer rows,
+// B=6 T=1,500 Hv=32 dv=128, 221 and 235), past it the shared K and Q rows come from memory
+// again (96 MiB: B=16 T=1,500 Hk=4 Hv=16 111 and 103; B=8 T=1,500 Hv=32 120 and 112; layer
+// rows 187 and 180; 188 MiB, B=12 T=3,000 Hk=4 Hv=16 183 and 169).  A key head of one value
+// head shares none (B=40 T=3,000 Hv=16, 470 MiB, 682 and 692).
+bool staging_wavefronts(const ChunkParams& p) {
+  constexpr long long kCached = 84LL << 20;
+  if (p.n_rec < 2LL * p.N) return false;
+  return p.Hv == p.Hk || (long long)p.n_rec * p.Hv * kRecBytesBF16 <= kCached;
+}
+
 template <int DK, int MODE, bool BWD = false, bool FUSE = false>
 hipError_t launch_scan_tiles(const ChunkParams& p, hipStream_t stream) {
   switch (scan_tiles_per_wg(p, BWD)) {
     case 1: return launch_scan_cfg<DK, MODE, BWD, 1, FUSE>(p, stream);
     case 2: return launch_scan_cfg<DK, MODE, BWD, 2, FUSE>(p, stream);
-    default: return launch_scan_cfg<DK, MODE, BWD, 4, FUSE>(p, stream);
+    default: break;
   }
+  if constexpr (DK == 64 && MODE != MODE_F32 && !BWD)
+    if (!staging_wavefronts(p)) return launch_scan_cfg<DK, MODE, BWD, 4, FUSE, true>(p, stream);
+  return launch_scan_cfg<DK, MODE, BWD, 4, FUSE>(p, stream);
 }
 
 }  // namespace

@@ -117,3 +117,40 @@ def test_prep_split_over_value_heads(B, T, Hk, Hv, dtype):
 def test_layer_prep_split_over_value_heads(B, T, Hk, Hv):
     layer.say(f"layer prep split B={B} T={T} Hk={Hk} Hv={Hv}")
     check_rows(B, T, dict(Hk=Hk, dk=64, Hv=Hv, dv=64), (0, B - 1), 8500 + T + Hv)
+
+
+@pytest.mark.parametrize("B,T,Hk,Hv", [
+    (40, 1, 8, 16), (40, 63, 8, 16), (40, 64, 8, 16),   # one chunk a sequence
+    (30, 150, 16, 64),                                  # records past 84 MiB, shared K and Q rows
+    (9, 65, 16, 16),                                    # with loader wavefronts, for comparison
+])
+@pytest.mark.parametrize("path", ["core", "layer", "layer packed"])
+def test_scan_of_64_columns_with_and_without_loader_wavefronts(B, T, Hk, Hv, path):
+    """dk = 64, bf16: a sequence of the batch against the oracle, and bit for bit against the
+    call of that sequence alone, whose 16-column workgroups have loader wavefronts."""
+    layer.say(f"staging {path} B={B} T={T} Hk={Hk} Hv={Hv}")
+    dims = dict(Hk=Hk, dk=64, Hv=Hv, dv=64)
+    if path == "core":
+        args = core.make(8600 + T + Hv, B, T, Hk, Hv, 64, 64, "bf16")
+        o, S = core.run_gpu(*args, "bf16")
+        one = [x[B - 1:] for x in args]
+        o1, S1 = core.run_gpu(*one, "bf16")
+        assert np.array_equal(o[B - 1:], o1) and np.array_equal(S[B - 1:], S1)
+        ro, rs = core.run_ref(*one, "bf16")
+        assert core.rel(o1, ro) < core.BF16_TOL and core.rel(S1, rs) < core.STATE_TOL
+        return
+    d = W.layer_inputs(B, T, **dims, seed=8600 + T + Hv)
+    S0 = (0.02 * np.random.default_rng(T).standard_normal((B, Hv, 64, 64))).astype(np.float32)
+    one = {k: (v[B - 1:] if k in ROWS else v) for k, v in d.items()}
+    cu = None
+    if path == "layer packed":
+        d = {k: (v.reshape(1, B * T, *v.shape[2:]) if k in ROWS else v) for k, v in d.items()}
+        cu = np.arange(B + 1, dtype=np.int32) * T
+    got = [layer.np_(x) for x in layer.gpu_prefill(W.to_device(d), dims, cu, S0)]
+    got[0] = got[0].reshape(B, T, -1)
+    alone = [layer.np_(x) for x in layer.gpu_prefill(W.to_device(one), dims, None, S0[B - 1:])]
+    for a, b in zip(got, alone):
+        assert np.array_equal(a[B - 1:].reshape(b.shape), b)
+    ref, S_ref, conv_ref = layer.ref_prefill(one, dims, None, S0[B - 1:])
+    assert layer.rel(alone[0], ref) < layer.BF16_TOL and layer.rel(alone[1], S_ref) < layer.STATE_TOL
+    assert np.array_equal(alone[2], conv_ref)
