@@ -1135,7 +1135,10 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE, OWN>::NTH)) __attri
             return l >= nvc || r;
           };
           for (int tries = 0; !gave_up && __ballot(!ready()) != 0ull; ++tries) {
-            if (tries == (1 << 20)) {  // about a second: give up rather than hang
+            // About half a minute: give up rather than hang.  Only other work that keeps
+            // every CU busy between two partners' starts makes a wait long (see take_ticket),
+            // and such a call must still come out right.
+            if (tries == (1 << 24)) {
               gave_up = 1;
               break;
             }
@@ -1150,9 +1153,8 @@ __global__ __launch_bounds__((Cfg<DK, MODE, NWC_, BWD, FUSE, OWN>::NTH)) __attri
           for (int w = 1; w < NBX; w <<= 1)
 #pragma unroll
             for (int s = 0; s + w < NBX; s += 2 * w) t[s] += t[s + w];
-          // as the epilogue kernel; a wait that gave up (a partner block never ran, which a
-          // grid the chip holds at once rules out unless other work kept CUs for a second)
-          // leaves NaN rows rather than rows normalised by partial sums
+          // as the epilogue kernel; a wait that gave up (a partner block never ran) leaves NaN
+          // rows rather than rows normalised by partial sums
           sRN[c & 1][l] = gave_up ? __builtin_nanf("") : rsqrtf(__builtin_fmaf(t[0], p.inv_dv, p.eps));
         }
       };

@@ -154,3 +154,74 @@ def test_scan_of_64_columns_with_and_without_loader_wavefronts(B, T, Hk, Hv, pat
     ref, S_ref, conv_ref = layer.ref_prefill(one, dims, None, S0[B - 1:])
     assert layer.rel(alone[0], ref) < layer.BF16_TOL and layer.rel(alone[1], S_ref) < layer.STATE_TOL
     assert np.array_equal(alone[2], conv_ref)
+
+
+# more 64-column workgroups than the chip has CUs, eight chunks a sequence or more: the fused
+# scan's workgroups take their places by ticket and wait for the other blocks of their head
+TICKETED = dict(Hk=2, dk=128, Hv=8, dv=128)
+
+
+def ticketed(B, T, seed):
+    d = W.layer_inputs(B, T, **TICKETED, seed=seed)
+    rng = np.random.default_rng(seed)
+    S0 = (0.02 * rng.standard_normal((B, 8, 128, 128))).astype(np.float32)
+    return d, W.to_device(d), S0
+
+
+def test_ticketed_layer_scan_replays_under_graph_capture():
+    """The tickets start from zero in every replay: fresh inputs copied into the captured
+    buffers, with eager calls and synchronisations in between, equal the eager call and, on two
+    sequences, the scan of one round, which takes no tickets."""
+    B, T = 24, 520
+    layer.say(f"ticketed layer scan under capture B={B} T={T}")
+    _, t, S0 = ticketed(B, T, 8700)
+    layer.gpu_prefill(t, TICKETED, None, S0)
+    from omegalax_amd import gdn_prefill
+    names = ("mixed_qkv", "z", "a", "b", "conv_w", "A_log", "dt_bias", "norm_w")
+    state = torch.from_numpy(S0).cuda()
+    kw = dict(num_k_heads=2, head_k_dim=128, num_v_heads=8, head_v_dim=128, output_final_state=True)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = gdn_prefill(*(t[n] for n in names), initial_state=state, **kw)
+    for rep in range(4):
+        d2, t2, S2 = ticketed(B, T, 8710 + rep)
+        for n in names:
+            t[n].copy_(t2[n])
+        state.copy_(torch.from_numpy(S2))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        want = layer.gpu_prefill(t2, TICKETED, None, S2)
+        for a, b in zip(out, want):
+            assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+        few = {n: (t2[n][:2].contiguous() if n in ROWS else t2[n]) for n in names}
+        for a, b in zip(out, layer.gpu_prefill(few, TICKETED, None, S2[:2])):
+            assert torch.equal(a[:2], b)
+
+
+def test_ticketed_layer_scans_beside_each_other_and_other_work():
+    """Two streams of ticketed scans and a third of matrix products share the CUs: waiting
+    workgroups, at most three of each eighth of a grid, leave room for the ones they wait for."""
+    B, T = 40, 520
+    layer.say(f"ticketed layer scans on two streams B={B} T={T}")
+    from omegalax_amd import gdn_prefill
+    names = ("mixed_qkv", "z", "a", "b", "conv_w", "A_log", "dt_bias", "norm_w")
+    kw = dict(num_k_heads=2, head_k_dim=128, num_v_heads=8, head_v_dim=128, output_final_state=True)
+    ins = [ticketed(B, T, 8720 + i)[1] for i in range(2)]
+    want = [gdn_prefill(*(t[n] for n in names), **kw) for t in ins]
+    x = torch.randn(4096, 4096, device="cuda").bfloat16()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(6):
+        for i in range(2):
+            with torch.cuda.stream(streams[i]):
+                got[i].append(gdn_prefill(*(ins[i][n] for n in names), **kw))
+        with torch.cuda.stream(streams[2]):
+            for _ in range(4):
+                y = x @ x
+    torch.cuda.synchronize()
+    for i in range(2):
+        for res in got[i]:
+            for a, b in zip(res, want[i]):
+                assert torch.equal(a, b)
