@@ -72,7 +72,7 @@ ChunkWs chunk_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64
   w.rec = o;
   // 19 KiB of room per record, 25 with P's lo parts: more than it fills, so that workspace
   // sizes, and the shapes which fit the allocation-free entry point's fixed scratch, stay the
-  // ones callers know.  The layer scan's tickets take 32 bytes of the rest.
+  // ones the tests of this interface pin.  The layer scan's tickets take 32 bytes of the rest.
   const size_t room = (mode == omx::kModeF32 || bwd ? 25 : 19) * 1024;
   w.tickets = align_up(slots * (size_t)Hv * (size_t)omx::chunk_record_bytes(mode, bwd), 256);
   o += align_up(slots * (size_t)Hv * room, 256);
@@ -119,7 +119,7 @@ BwdWs bwd_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk, int64_t d
   const size_t tokens = (size_t)(B * T);
   const size_t slots = (tokens + 63) / 64 + (size_t)N;
   size_t o = w.f.total;
-  w.xlpg = o;  // (room for the matrices with either input precision: sizes callers know)
+  w.xlpg = o;  // (room for the matrices with either input precision, as for the records)
   o += align_up(slots * (size_t)Hv * omx::xlpg_floats_host(true) * 4, 256);
   w.states = o;
   o += align_up(slots * (size_t)(Hv * dk * dv) * 4, 256);
@@ -987,7 +987,9 @@ namespace {
 
 // Workspace of the layer backward: the rule's backward workspace, then the recomputed
 // conv + SiLU output (q, k, v rows), g and beta, the rule's fp32 o and its cotangent, the
-// rule's gradients of q, k, v, g and beta, and the partial sums of the parameter gradients.
+// rule's gradients of q, k, v, g and beta, and the partial sums of the parameter gradients
+// (the gates' in the room that the rule's workspace keeps for the matrices, which bf16 inputs
+// leave empty behind G: a workspace that was ever large enough stays so).
 struct LayerBwdWs {
   BwdWs c;
   size_t q, k, v, g, beta, o, dO, gq, gk, gv, dg, dbeta, pn, pg, pc, total;
@@ -1019,7 +1021,11 @@ LayerBwdWs layer_bwd_ws(int64_t B, int64_t T, int64_t Hk, int64_t Hv, int64_t dk
   w.dg = take(tokens * (size_t)Hv * 4);
   w.dbeta = take(tokens * (size_t)Hv * 4);
   w.pn = take((size_t)omx::layer_bwd_norm_blocks() * (size_t)dv * 4);
-  w.pg = take((size_t)omx::layer_bwd_gate_blocks((long long)tokens) * 2 * (size_t)Hv * 4);
+  const size_t slots = (tokens + 63) / 64 + (size_t)N;
+  w.pg = w.c.xlpg + align_up(slots * (size_t)Hv * omx::xlpg_floats_host(false) * 4, 256);
+  // two sums per 32 tokens (or fewer) and value head, that is four floats per slot
+  static_assert(omx::xlpg_floats_host(false) + 4 + 256 / 4 <= omx::xlpg_floats_host(true),
+                "the gates' partial sums fit the matrices' room");
   w.pc = take((size_t)omx::layer_bwd_conv_blocks((long long)tokens) * conv_dim * 4 * 4);
   w.total = o;
   return w;

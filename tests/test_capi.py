@@ -370,3 +370,19 @@ def test_one_packed_sequence_takes_the_widths_of_a_batch_of_one():
     for Hv in (16, 32, 48, 64, 96):
         assert f(1, Hv, 128, 128, True, False) == f(1, Hv, 128, 128, False, False)
     assert f(3, 16, 128, 128, True, False) == 1 and f(3, 16, 128, 128, False, False) == 2
+
+
+@pytest.mark.parametrize("B,T,Hk,Hv,d,N", [(4, 4096, 16, 32, 128, 4), (1, 1, 1, 1, 64, 1), (1, 0, 1, 1, 64, 1),
+                                           (1, 3001, 16, 32, 128, 5), (1, 70000, 2, 256, 64, 3)])
+def test_layer_backward_takes_every_workspace_that_was_large_enough(B, T, Hk, Hv, d, N):
+    """The rule's workspace, the recomputed rows and the partial sums with one row of the gates'
+    per 256 tokens: the size of the first kernels, whatever the present ones split more finely."""
+    L = _lib.lib()
+    tok, kd, vd = B * T, Hk * d, Hv * d
+    rows = (tok * kd * 2, tok * kd * 2, tok * vd * 2, tok * Hv * 4, tok * Hv * 4, tok * vd * 4, tok * vd * 4,
+            tok * kd * 2, tok * kd * 2, tok * vd * 2, tok * Hv * 4, tok * Hv * 4)
+    gates = max(1, min(1024, (tok + 255) // 256))
+    parts = (4096 * d * 4, gates * 2 * Hv * 4, (tok + 63) // 64 * (2 * kd + vd) * 16)
+    most = L.omx_gdn_chunk_bwd_workspace_size(B, T, Hk, Hv, d, d, N, _lib.BF16) \
+        + sum((x + 255) // 256 * 256 for x in rows + parts)
+    assert L.omx_gdn_prefill_bwd_workspace_size(B, T, Hk, Hv, d, d, N) <= most
