@@ -29,9 +29,15 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+# the raw handle of the current stream, without building a torch.cuda.Stream per call, where
+# this torch has the private function for it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(device):
-    # the raw handle of the current stream, without building a torch.cuda.Stream per call
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def _dev(*ts):

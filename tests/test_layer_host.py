@@ -106,3 +106,16 @@ def test_ab_projection_limits_are_checked_up_front():
     w = torch.zeros(4, 20, dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="multiple of 8"):
         _ab_proj_fwd(x, w, w)
+
+
+def test_stream_handle_without_the_private_torch_function(monkeypatch):
+    """A torch that lacks the private function is asked for the stream by the public one."""
+    from types import SimpleNamespace
+
+    from omegalax_amd import deltanet
+    asked = []
+    monkeypatch.setattr(deltanet, "_raw_stream", None, raising=False)
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: asked.append(d) or SimpleNamespace(cuda_stream=1234))
+    device = torch.device("cuda", 3)
+    assert deltanet._stream(device) == 1234 and asked == [device]
