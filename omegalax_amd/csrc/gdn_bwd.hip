@@ -9,11 +9,11 @@
 //     O     = scale diag(e^G) Q S + P V_new                   (:136-137)
 //     S'    = e^{G_last} S + K^T diag(e^{G_last - G}) V_new   (:139-142)
 // Three kernels, after the forward's preparation and scan have been rerun in their
-// backward variants (which leave X, Lg, P, G per chunk and the state entering every
-// chunk plus V_new):
+// backward variants (which leave per chunk X and G, for fp32 inputs Lg and P too, and the
+// state entering every chunk plus V_new):
 //  1. rscan_kernel walks each sequence's chunks backwards carrying dS, the gradient of
 //     the state leaving the chunk, in registers (one workgroup per (sequence, value head,
-//     64 columns of dv), 16 columns per wavefront):
+//     64 columns of dv, or 32 or 16 with bf16 inputs; 16 columns per wavefront):
 //         dV_new = P^T dO + diag(e^{G_last - G}) K dS
 //         dR     = X^T dV_new
 //         dS    <- e^{G_last} dS + scale Q^T diag(e^G) dO - K^T diag(e^G) diag(beta) dR
@@ -76,48 +76,35 @@ __device__ __forceinline__ Op join_op(f32x4 a, f32x4 b) {
 __device__ __forceinline__ float ldx(const float* p) { return *p; }
 __device__ __forceinline__ float ldx(const bf16_t* p) { return bf2f(*p); }
 
-// Contraction index of operand slot e in lane group q: the natural order 8q + e, or the
-// block-pair order (4q + e%4, then 16 + 4q + e%4) of two C-layout tiles side by side.
-template <bool PAIR>
-__device__ __forceinline__ int kslot(int q, int e) {
-  return PAIR ? 4 * q + (e & 3) + 16 * (e >> 2) : 8 * q + e;
-}
-
-// operand row `row` of a row-major M[row][k], slots over k from k0
-template <bool PAIR, class T>
+// operand row `row` of a row-major M[row][k], slots over k from k0 (slot e of lane group q:
+// 8q + e)
+template <class T>
 __device__ __forceinline__ void frag_row(const T* m, int ld, int row, int k0, float* x) {
   const int q = lane_id() >> 4;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = ldx(m + row * ld + k0 + kslot<PAIR>(q, e));
+  for (int e = 0; e < 8; ++e) x[e] = ldx(m + row * ld + k0 + 8 * q + e);
 }
-// operand column `col` of a row-major M[k][col], slots over the rows from k0
-template <bool PAIR, class T>
+// operand column `col` of a row-major M[k][col], slots over the rows from k0 in the
+// block-pair order of two C-layout tiles side by side (4q + e%4, then 16 + 4q + e%4)
+template <class T>
 __device__ __forceinline__ void frag_col(const T* m, int ld, int col, int k0, float* x) {
   const int q = lane_id() >> 4;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = ldx(m + (k0 + kslot<PAIR>(q, e)) * ld + col);
+  for (int e = 0; e < 8; ++e) x[e] = ldx(m + (k0 + 4 * q + (e & 3) + 16 * (e >> 2)) * ld + col);
 }
 
 // K / Q operand fragments from the staged rows: bf16 rows are exact bf16 (one vector or
 // two transposed LDS reads, no lo part); fp32 rows are read element-wise and split.
 // kq_row: row row0 + lane%16, slots over columns from k0.
-template <bool PAIR>
 __device__ __forceinline__ Op kq_row(const float* m, int ld, int row0, int k0) {
   float x[8];
-  frag_row<PAIR>(m, ld, row0 + (lane_id() & 15), k0, x);
+  frag_row(m, ld, row0 + (lane_id() & 15), k0, x);
   return split8(x);
 }
-template <bool PAIR>
 __device__ __forceinline__ Op kq_row(const bf16_t* m, int ld, int row0, int k0) {
   const int l = lane_id(), q = l >> 4;
-  const bf16_t* pr = m + (row0 + (l & 15)) * ld + k0;
   Op o;
-  if constexpr (PAIR) {
-    const u32x2 a = *(const u32x2*)(pr + 4 * q), b = *(const u32x2*)(pr + 16 + 4 * q);
-    o.h = u32x4{a[0], a[1], b[0], b[1]};
-  } else {
-    o.h = *(const u32x4*)(pr + 8 * q);
-  }
+  o.h = *(const u32x4*)(m + (row0 + (l & 15)) * ld + k0 + 8 * q);
   o.l = o.h;
   return o;
 }
@@ -126,7 +113,7 @@ __device__ __forceinline__ Op kq_row(const bf16_t* m, int ld, int row0, int k0) 
 __device__ __forceinline__ Op kq_st(const float* m, int ld, int t, int k0) {
   const int r = lane_id() & 15;
   float x[8];
-  frag_col<true>(m, ld, 32 * (t >> 1) + 4 * (t & 1) + 8 * (r >> 2) + (r & 3), k0, x);
+  frag_col(m, ld, 32 * (t >> 1) + 4 * (t & 1) + 8 * (r >> 2) + (r & 3), k0, x);
   return split8(x);
 }
 __device__ __forceinline__ Op kq_st(const bf16_t* m, int ld, int t, int k0) {
@@ -159,11 +146,6 @@ template <> struct Vec4<float> { typedef float4 type; };
 template <> struct Vec4<bf16_t> { typedef u32x2 type; };
 __device__ __forceinline__ float4 load4(const float* src) { return *(const float4*)src; }
 __device__ __forceinline__ void store4(float* dst, float4 x) { *(float4*)dst = x; }
-// a float at the precision T (bf16 rounded to nearest even)
-template <class T> __device__ __forceinline__ T from_f32(float x);
-template <> __device__ __forceinline__ float from_f32<float>(float x) { return x; }
-template <> __device__ __forceinline__ bf16_t from_f32<bf16_t>(float x) { return f2bf(x); }
-
 __device__ __forceinline__ float4 to_f4(float4 x) { return x; }
 __device__ __forceinline__ float4 to_f4(u32x2 x) {
   return float4{__uint_as_float(x[0] << 16), __uint_as_float(x[0] & 0xffff0000u),
@@ -274,7 +256,7 @@ __device__ __forceinline__ void put_row4(bf16_t* h, bf16_t* lo, int off, f32x4 c
   *(u32x2*)(lo + off) = pack_lo4(c);
 }
 
-// op_vec in the block-pair contraction order (kslot<true>): entries k0 + 4q .. +3 and
+// op_vec in the block-pair contraction order (as frag_col): entries k0 + 4q .. +3 and
 // k0 + 16 + 4q .. +3 of storage row r0 + r.
 __device__ __forceinline__ Op op_pair(const bf16_t* h, const bf16_t* lo, int ld, int r0, int k0) {
   const int l = lane_id();
@@ -286,7 +268,7 @@ __device__ __forceinline__ Op op_pair(const bf16_t* h, const bf16_t* lo, int ld,
   o.l = u32x4{c[0], c[1], d[0], d[1]};
   return o;
 }
-// op_tr in the block-pair contraction order (kslot<true>): entries k0 + 4q .. +3 and
+// op_tr in the block-pair contraction order (as frag_col): entries k0 + 4q .. +3 and
 // k0 + 16 + 4q .. +3 down storage column c0 + r
 __device__ __forceinline__ Op op_tr_pair(const bf16_t* h, const bf16_t* lo, int ld, int c0, int k0) {
   const int l = lane_id(), q = l >> 4, s = l & 15;
@@ -522,7 +504,7 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
       o.h = o.l = swz_frag(m, r0, k0);
       return o;
     } else {
-      return kq_row<false>(m, LDK, r0, k0);
+      return kq_row(m, LDK, r0, k0);
     }
   };
   auto k_st = [&](const auto* m, int t, int k0) {
@@ -1015,7 +997,8 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     load_state(rDS, u, dfr);  // this step's, used after the products with S
     lds_barrier();
     // the products with S, then those with dS, then the tiles: few operands live at a time
-    // (all of them at once spilled accumulators, whose reloads waited for every load)
+    // (all of them at once spilled accumulators, whose reloads waited for every load; so, two
+    // registers are left spilled at dk = dv = 128, one at dv = 64, none at dk <= 64)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const Op ao = op_vec(sDOh, sDOl, LDR, 16 * i, 0);

@@ -31,7 +31,6 @@ namespace omx {
 constexpr int kC = 64;      // chunk length (deltanet.py:59)
 constexpr int kNT = 256;    // threads per workgroup in both kernels
 constexpr int kLDT = kC + 8;   // row stride (elements) of 64-wide bf16 LDS arrays
-constexpr int kLDD = 16 + 4;   // row stride of 16-wide LDS arrays
 constexpr int MODE_BF16 = kModeBF16, MODE_F32 = kModeF32, MODE_LAYER = kModeLayer;
 
 // record layout (bytes)
@@ -236,11 +235,11 @@ __device__ __forceinline__ void seq_range(const int32_t* cu, int n, int T, long 
 // Work item of a workgroup of the scans (forward and reverse): sequence n, value head h
 // and column block blk, from index b (blockIdx.x, or the place a ticket gives).  The
 // workgroups of one key head of one sequence (gqa value heads x nb blocks, which read the
-// same q/k rows) form a group that runs on one XCD (the hardware deals workgroup i to XCD i % 8), so they share its L2.  When the
-// group count is a multiple of 8, group ranks are dealt round-robin over the XCDs in the
-// order of `order` (sequences longest first; null = index order): every XCD gets a share
-// of every sequence and starts its longest chains first.  Otherwise each XCD takes a
-// contiguous range of groups in index order.
+// same q/k rows) form a group that runs on one XCD (the hardware deals workgroup i to XCD
+// i % 8), so they share its L2.  When the group count is a multiple of 8, group ranks are
+// dealt round-robin over the XCDs in the order of `order` (sequences longest first; null =
+// index order): every XCD gets a share of every sequence and starts its longest chains
+// first.  Otherwise each XCD takes a contiguous range of groups in index order.
 struct ScanItem {
   int n, h, blk;
 };

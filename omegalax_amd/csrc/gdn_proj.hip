@@ -6,9 +6,9 @@
 // HBM (64 MiB at C1) for a few MFLOP of work, twice.  This kernel reads each hidden row
 // once and forms both outputs from it: a memory-bound skinny product.
 //
-// Work mapping (many rows; few rows: ab_proj_small_kernel): one workgroup per 64 token rows, wavefront w owning rows 16 (w % 4) ..
-// +15 of contraction part w / 4 (one or two parts, the partial sums added at the end);
-// each part runs its chunks of KC.  A chunk's weight rows (both matrices, 2 x 16 NT rows,
+// Work mapping (many rows; few rows: ab_proj_small_kernel): one workgroup per 64 token
+// rows, wavefront w owning rows 16 (w % 4) .. +15 of contraction part w / 4 (one or two
+// parts, the partial sums added at the end); each part runs its chunks of KC.  A chunk's weight rows (both matrices, 2 x 16 NT rows,
 // rows past Hv zero) are staged once per part in LDS (rows padded by 16 bytes, so the 16
 // rows of a fragment read fall in different banks) and shared by its four wavefronts;
 // each lane loads its own token row's part straight into registers.  Both
@@ -281,7 +281,7 @@ hipError_t launch_nt(const void* x, const void* wa, const void* wb, void* a, voi
 // 11.7 us; Hv=32, 1,024 rows, 5.9 against 15.4 us; Hv=64, 512 rows, 5.9 against 21.5 us);
 // with twice the rows it ties (D=1024, Hv=32: 9.4 against 9.0 us), since each column tile
 // rereads the rows.
-constexpr long long kSmallBlocks = 256;
+bool few_rows(long long M, int Hv) { return small_blocks(M, Hv) <= device_cus(); }
 
 int ab_proj_max_heads() { return 128; }
 
@@ -289,7 +289,7 @@ hipError_t launch_ab_proj(const void* x, const void* wa, const void* wb, void* a
                           long long M, int D, int Hv, hipStream_t stream) {
   if (M == 0) return hipSuccess;
   if (D <= 0 || D % 8 != 0 || Hv < 1 || Hv > 128) return hipErrorInvalidValue;
-  if (small_blocks(M, Hv) <= kSmallBlocks) return launch_small(x, wa, wb, a, b, M, D, Hv, stream);
+  if (few_rows(M, Hv)) return launch_small(x, wa, wb, a, b, M, D, Hv, stream);
   if (Hv <= 16) return launch_nt<1>(x, wa, wb, a, b, M, D, Hv, stream);
   if (Hv <= 32) return launch_nt<2>(x, wa, wb, a, b, M, D, Hv, stream);
   if (Hv <= 64) return launch_nt<4>(x, wa, wb, a, b, M, D, Hv, stream);
