@@ -8,8 +8,8 @@
 //
 // Work mapping (many rows; few rows: ab_proj_small_kernel): one workgroup per 64 token
 // rows, wavefront w owning rows 16 (w % 4) .. +15 of contraction part w / 4 (one or two
-// parts, the partial sums added at the end); each part runs its chunks of KC.  A chunk's weight rows (both matrices, 2 x 16 NT rows,
-// rows past Hv zero) are staged once per part in LDS (rows padded by 16 bytes, so the 16
+// parts, the partial sums added at the end); each part runs its chunks of KC.  A chunk's
+// weight rows (both matrices, 2 x 16 NT rows, rows past Hv zero) are staged once per part in LDS (rows padded by 16 bytes, so the 16
 // rows of a fragment read fall in different banks) and shared by its four wavefronts;
 // each lane loads its own token row's part straight into registers.  Both
 // are read in the "row r, contraction slots 8q .. 8q+7" layout of a 16x16x32 MFMA
