@@ -339,7 +339,10 @@ __device__ __forceinline__ void conv_bwd(const LayerBwdParams& p, long long bid,
         for (int m = 0; m < d; ++m)
           if (k + m >= 0) back[d] &= ~(1u << (k + m));
     };
-    const long long t2 = tb > 2 ? tb - 2 : 0, tend = tb + kConvSB + 3;
+    // (starts at or past the last token cut nothing: rows of offsets are often filled up to a
+    // fixed count with empty sequences there)
+    const long long t2 = tb > 2 ? tb - 2 : 0;
+    const long long tend = tb + kConvSB + 3 < p.tokens ? tb + kConvSB + 3 : p.tokens;
     if (p.cu_seqlens) {
       int lo = 0, hi = p.N;  // the last sequence with cu[n] <= t2
       while (hi - lo > 1) {

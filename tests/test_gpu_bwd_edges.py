@@ -112,6 +112,7 @@ def test_gate_gradient_takes_the_state_in_fp32(T, dk, dv, dtype):
     ([2, 1, 1, 3], 1, 2, 64, 64),                     # sequences shorter than the conv window
     ([15, 1, 2, 14, 17, 15], 1, 1, 64, 128),          # starts on both sides of 16-token edges
     ([62, 1, 1, 3, 64, 0, 5], 2, 4, 128, 128),        # starts around a 64-token edge, one empty
+    ([0, 0, 17, 0, 0, 0, 30] + [0] * 40, 1, 2, 64, 64),  # empty ones everywhere, the row filled up with them
 ])
 def test_layer_backward_at_conv_edges(lens, Hk, Hv, dk, dv):
     layer.say(f"layer bwd edges lens={lens}")
