@@ -1389,19 +1389,26 @@ int scan_tiles_per_wg(const ChunkParams& p, bool bwd) {
   return scan_column_tiles(p.N, p.Hv, p.DV, p.dk, p.cu_seqlens != nullptr, bwd);
 }
 
-// (bf16 rows of dk = 64, forward, 64 columns) whether loader wavefronts stage the rows.  They
-// have nothing to run ahead of when sequences have one chunk (B=600 T=64 Hv=16 264 us, without
-// them 247).  And ahead of the products they let the workgroups of one key head drift apart:
-// while the call's records and rows stay in the 256 MiB cache behind the L2s that costs
-// nothing (records of 72 MiB, B=12 T=1,500 Hk=4 Hv=16, 76 us, without them 91; layer rows,
-// B=6 T=1,500 Hv=32 dv=128, 221 and 235), past it the shared K and Q rows come from memory
-// again (96 MiB: B=16 T=1,500 Hk=4 Hv=16 111 and 103; B=8 T=1,500 Hv=32 120 and 112; layer
-// rows 187 and 180; 188 MiB, B=12 T=3,000 Hk=4 Hv=16 183 and 169).  A key head of one value
-// head shares none (B=40 T=3,000 Hv=16, 470 MiB, 682 and 692).
+// (bf16 rows of dk = 64, forward, 64 columns) whether loader wavefronts stage the rows.  Ahead
+// of the products they let the workgroups of one key head drift apart.  While the call's
+// records and rows stay in the 256 MiB cache behind the L2s that costs nothing (records of 72
+// MiB, B=12 T=1,500 Hk=4 Hv=16, 76 us, without loaders 91), past it the shared K and Q rows
+// come from memory again (96 MiB: B=16 T=1,500 Hk=4 Hv=16 111 and 103; B=8 T=1,500 Hv=32 120
+// and 112; layer rows 187 and 180; 188 MiB, B=12 T=3,000 Hk=4 Hv=16 183 and 169).  A key head
+// of one value head shares none (B=40 T=3,000 Hv=16, 470 MiB, 682 and 692), in sequences of
+// few chunks nothing drifts far (B=600 T=128 Hv=16 398 and 398, 600 packed documents of 100
+// tokens 413 and 427, layer rows, B=400 T=256 Hk=4 Hv=16, 686 and 694), and two column blocks
+// a head measured even.  With one chunk a sequence the core's loaders have nothing to run
+// ahead of (B=600 T=64 Hv=16 264 and 247; layer rows 404 and 407).
+template <int MODE>
 bool staging_wavefronts(const ChunkParams& p) {
-  constexpr long long kCached = 84LL << 20;
-  if (p.n_rec < 2LL * p.N) return false;
-  return p.Hv == p.Hk || (long long)p.n_rec * p.Hv * kRecBytesBF16 <= kCached;
+  constexpr long long kCached = 84LL << 20, kLong = MODE == MODE_LAYER ? 8 : 4;
+  if (p.DV != 64) return true;
+  if (MODE != MODE_LAYER && !p.cu_seqlens && p.nch == 1) return false;
+  // packed: the tokens' whole chunks (n_rec has a slot for every sequence beside them, and rows
+  // of offsets are often filled up with empty ones)
+  const long long chunks = p.cu_seqlens ? p.nch : p.n_rec;
+  return p.Hv == p.Hk || chunks < kLong * p.N || chunks * p.Hv * kRecBytesBF16 <= kCached;
 }
 
 template <int DK, int MODE, bool BWD = false, bool FUSE = false>
@@ -1412,7 +1419,7 @@ hipError_t launch_scan_tiles(const ChunkParams& p, hipStream_t stream) {
     default: break;
   }
   if constexpr (DK == 64 && MODE != MODE_F32 && !BWD)
-    if (!staging_wavefronts(p)) return launch_scan_cfg<DK, MODE, BWD, 4, FUSE, true>(p, stream);
+    if (!staging_wavefronts<MODE>(p)) return launch_scan_cfg<DK, MODE, BWD, 4, FUSE, true>(p, stream);
   return launch_scan_cfg<DK, MODE, BWD, 4, FUSE>(p, stream);
 }
 

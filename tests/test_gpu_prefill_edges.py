@@ -121,7 +121,8 @@ def test_layer_prep_split_over_value_heads(B, T, Hk, Hv):
 
 @pytest.mark.parametrize("B,T,Hk,Hv", [
     (40, 1, 8, 16), (40, 63, 8, 16), (40, 64, 8, 16),   # one chunk a sequence
-    (30, 150, 16, 64),                                  # records past 84 MiB, shared K and Q rows
+    (30, 150, 16, 64),                                  # three chunks: with them
+    (12, 460, 16, 64),                                  # eight, records past 84 MiB, shared K and Q rows
     (9, 65, 16, 16),                                    # with loader wavefronts, for comparison
 ])
 @pytest.mark.parametrize("path", ["core", "layer", "layer packed"])
