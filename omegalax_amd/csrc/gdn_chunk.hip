@@ -1477,11 +1477,17 @@ int layer_scan_blocks(const ChunkParams& p) {
 // pass over o outweighs it (and the prep, which clears the tickets, has work).  Scan and
 // epilogue -> fused scan, Hk=16 Hv=32 d=128: 8 documents of 32,768 tokens 543 -> 502 us;
 // B=16 T=500 153 -> 140 us; 6 documents of 4,096 tokens (Hv=64) 146 -> 147 us; one chunk a
-// sequence (B=64 T=64) 154 -> 182 us, which stays with the epilogue kernel.
+// sequence (B=64 T=64) 154 -> 182 us, which stays with the epilogue kernel.  So do packed rows
+// of at most 16 heads of one block: few workgroups then walk a long document while the chip
+// idles, and the fused norm lengthens their step (Hv=16 dv=64, layer call, fused and not: one
+// document of 10,000 tokens and 23 of 435 536 and 473 us, unevenly drawn lengths 252 and 247,
+// 300 and 287, even ones 230 and 233; with 24 heads 483 and 456, 221 and 233, 267 and 274,
+// 237 and 246).
 bool layer_scan_fuses_norm(const ChunkParams& p) {
   if (!p.ss_xch || !layer_v_in_scan(p.dk)) return false;
   const long long grid = (long long)p.N * p.Hv * layer_scan_blocks(p);
   if (grid <= device_cus()) return true;
+  if (p.cu_seqlens && layer_scan_blocks(p) == 1 && p.Hv <= 16) return false;
   return (long long)p.N * p.Hk % 8 == 0 && layer_scan_blocks(p) <= 4 && p.n_rec >= 8LL * p.N;
 }
 

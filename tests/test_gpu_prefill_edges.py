@@ -84,6 +84,22 @@ def test_layer_scan_of_packed_sequences_past_one_round(N):
     assert np.array_equal(layer.np_(conv), conv_ref)
 
 
+@pytest.mark.parametrize("Hv", [16, 24])
+def test_packed_layer_rows_of_one_block_a_head_equal_the_batch(Hv):
+    """dv = 64, more workgroups than CUs, eight chunks a sequence or more: the batch takes the
+    fused scan, packed rows of 16 heads the epilogue kernel, of 24 the fused scan; bit for bit."""
+    B, T = 24, 520
+    layer.say(f"layer scan: one block a head, Hv={Hv}")
+    dims = dict(Hk=8, dk=128, Hv=Hv, dv=64)
+    d = W.layer_inputs(B, T, **dims, seed=8250 + Hv)
+    S0 = (0.02 * np.random.default_rng(8250).standard_normal((B, Hv, 128, 64))).astype(np.float32)
+    batch = layer.gpu_prefill(W.to_device(d), dims, None, S0)
+    row = {k: (v.reshape(1, B * T, *v.shape[2:]) if k in ROWS else v) for k, v in d.items()}
+    packed = layer.gpu_prefill(W.to_device(row), dims, np.arange(B + 1, dtype=np.int32) * T, S0)
+    for a, b in zip(batch, packed):
+        assert torch.equal(a.reshape(b.shape), b)
+
+
 def test_layer_of_no_tokens_keeps_the_states():
     """T = 0 over more workgroups than the chip holds: no chunk to prepare, states copied."""
     layer.say("layer T=0")
