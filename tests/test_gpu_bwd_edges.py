@@ -49,6 +49,7 @@ def test_core_backward_of_fast_decay_keeps_the_diagonal(dk):
     args = list(core.make(7150 + dk, 2, 192, 1, 2, dk, 64, "f32"))
     args[3] = (-60 - np.random.default_rng(7150).uniform(0, 1, args[3].shape)).astype(np.float32)
     got, ref = core.run_gpu(*args, "f32"), core.run_ref(*args, "f32")
+    assert all(np.isfinite(x).all() for x in got)
     core.check(got, ref, "f32", skip=("dg",))  # dg is a difference of sums that are all but equal
     err = np.linalg.norm(got[0] - ref[0]) / np.linalg.norm(ref[0])
     assert err < 2.0 ** -16, err
