@@ -208,6 +208,13 @@ __device__ __forceinline__ void set_cols(float* arr, int bj, f32x4 x) {
   if ((l >> 4) == 0) arr[16 * bj + (l & 15)] = s;
 }
 
+// Gamma = e^{a - b}, at most 1, from the hardware exp2 (below 2^-126: zero).  The difference
+// comes first: scaled to base 2 one by one, each gate would leave its own rounding in Gamma,
+// on its unit diagonal too where a product is contracted into the subtraction.
+__device__ __forceinline__ float gate_ratio(float a, float b) {
+  return __builtin_amdgcn_exp2f(fminf(a - b, 0.f) * 1.4426950408889634f);
+}
+
 // Sum over the 64 lanes, left in every lane (DPP within each row, then the row swaps).
 __device__ __forceinline__ float wave_sum(float s) {
   s = group_sum_dpp<16>(s);
@@ -517,20 +524,27 @@ __global__ __launch_bounds__(F32 ? NT : 64 * NWC + NT) void rscan_kernel(BwdPara
     }
   };
   // (LDR) tile (mb, nb) of P = lower(scale Q K^T * Gamma) in the C layout, from the rows
-  // staged in bf.  Gamma comes from the difference of the gates, as in the gradient kernel:
-  // scaled to base 2 one by one, a product contracted into the subtraction would leave the
-  // other's rounding, 2e-4 at G = -3,800, on the diagonal too.
+  // staged in bf (Gamma's diagonal was 2e-4 off at G = -3,800 before gate_ratio)
   auto form_ptile = [&](int mb, int nb, const Buf& bf) {
-    f32x4 acc = zero4();
+    u32x4 qf[DK / 32], kf[DK / 32];
+    f32x4 acc = zero4(), w;
+    float gm[4];
+    const float gn = bf.Gl[16 * nb + lr];
 #pragma unroll
-    for (int s2 = 0; s2 < DK / 32; ++s2)
-      acc = mma16(k_row((const bf16_t*)bf.Q, 16 * mb, 32 * s2).h, k_row((const bf16_t*)bf.K, 16 * nb, 32 * s2).h, acc);
+    for (int v = 0; v < 4; ++v) gm[v] = bf.Gl[16 * mb + 4 * lq + v];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int m = 16 * mb + 4 * lq + v, n = 16 * nb + lr;
-      acc[v] = p.scale * acc[v] * __expf(fminf(bf.Gl[m] - bf.Gl[n], 0.f)) * (float)(m >= n);
+    for (int s2 = 0; s2 < DK / 32; ++s2) {
+      qf[s2] = k_row((const bf16_t*)bf.Q, 16 * mb, 32 * s2).h;
+      kf[s2] = k_row((const bf16_t*)bf.K, 16 * nb, 32 * s2).h;
     }
-    return acc;
+    // the factors while the fragments arrive: the compute wavefronts wait for the tiles, so
+    // only one product per value follows the MFMAs
+#pragma unroll
+    for (int v = 0; v < 4; ++v) w[v] = p.scale * gate_ratio(gm[v], gn) * (float)(16 * mb + 4 * lq + v >= 16 * nb + lr);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s2 = 0; s2 < DK / 32; ++s2) acc = mma16(qf[s2], kf[s2], acc);
+    return acc * w;
   };
   // (LDR) the ten tiles, dealt over the four loaders (t = lw, lw + 4, lw + 8), into sPT
   auto form_ptiles = [&](const Buf& bf) {
@@ -1098,8 +1112,7 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // P = lower(scale Q K^T * Gamma) and Lg = strict_lower(K K^T * Gamma) at this wavefront's
   // tiles: fp32 inputs read them from the preparation kernel's matrices, bf16 inputs form
   // them (the same products summed by the same MFMA over the same dk blocks in the same
-  // order).  Gamma comes from the difference of the gates: scaled to base 2 one by one, each
-  // would leave its own rounding there, 4e-5 at G = -1,000, and on the diagonal too.
+  // order).
   {
     f32x4 rowp = zero4(), rowl = zero4(), rowb = zero4();
 #pragma unroll
@@ -1119,7 +1132,7 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int row = 16 * rp + 4 * lq + v;
-          const float e = __expf(fminf(sG[row] - gc, 0.f));
+          const float e = gate_ratio(sG[row], gc);
           const float d = row >= col ? d4[v] : 0.f;
           const float x = d * (F32 ? xb[kXlpgP + row * C + col] : scale * pp[v] * e);
           rowp[v] += x;
@@ -1140,7 +1153,7 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int row = 16 * rl + 4 * lq + v;
-          const float e = __expf(fminf(sG[row] - gc, 0.f));
+          const float e = gate_ratio(sG[row], gc);
           const float d = row > col ? -d4[v] : 0.f;      // dL
           const float x = d * (F32 ? xb[kXlpgLg + row * C + col] : kk[v] * e);
           const float y = sBt[row] * x;                  // dL * L
